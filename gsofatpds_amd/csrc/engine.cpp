@@ -58,9 +58,11 @@ int prepare(const gsofa_csr* a, Prepared& out) {
 bool mirrored(const Prepared& P, const Options& opt) { return opt.symmetric != -1 && P.symmetric; }
 
 // Elimination tree of A + A^T by Liu's algorithm with path compression: every pair {k, i}, k < i,
-// of A's off-diagonal entries is taken at step i. Then subtree sizes.
-static void subtree_sizes(const Prepared& P, std::vector<int32_t>& size) {
+// of A's off-diagonal entries is taken at step i. Then subtree sizes. Kept in P.
+static void elimination_tree(const Prepared& P) {
   const int32_t n = P.n;
+  std::vector<int32_t>& size = P.subtree;
+  std::vector<int32_t>& parent = P.parent;
   std::vector<int32_t> cnt((size_t)n + 1, 0);
   for (int32_t r = 0; r < n; ++r)
     for (int32_t k = P.rowptr[r]; k < P.rowptr[r + 1]; ++k) {
@@ -77,7 +79,8 @@ static void subtree_sizes(const Prepared& P, std::vector<int32_t>& size) {
         if (c != r) lower[(size_t)cur[std::max(c, r)]++] = std::min(c, r);
       }
   }
-  std::vector<int32_t> parent((size_t)n, -1), anc((size_t)n, -1);
+  parent.assign((size_t)n, -1);
+  std::vector<int32_t> anc((size_t)n, -1);
   for (int32_t i = 0; i < n; ++i)
     for (int32_t p = cnt[i]; p < cnt[(size_t)i + 1]; ++p) {
       int32_t r = lower[p];
@@ -102,7 +105,7 @@ int64_t block_cuts(const Prepared& P, int32_t chain_block, int32_t divisor, std:
   cut.assign((size_t)nb, -1);
   const int64_t min_size = std::max<int64_t>(16 * (int64_t)chain_block, n / std::max(divisor, 1));
   if (chain_block < 2 || n < 2 * min_size) return 0;
-  if (P.subtree.empty()) subtree_sizes(P, P.subtree);
+  if (P.subtree.empty()) elimination_tree(P);
   const std::vector<int32_t>& size = P.subtree;
   int64_t count = 0;
   for (int64_t b = 0; b < nb; ++b) {
@@ -130,6 +133,60 @@ static double symmetric_share(const Prepared& P) {
       matched += std::binary_search(P.adj.begin() + P.rowptr[c], P.adj.begin() + P.rowptr[c + 1], v) ? 1 : 0;
     }
   return seen ? (double)matched / (double)seen : 1.0;
+}
+
+int32_t condensation_roots(const Prepared& P, int32_t limit, std::vector<int32_t>& vroot, std::vector<uint8_t>& is_root) {
+  const int32_t n = P.n;
+  const std::vector<int32_t>&size = P.subtree, &parent = P.parent;
+  // Sampled vertices: their root under each share of the limit, and how much of a contracted vertex
+  // is left in the graph (its root's node and list nodes). In nested-dissection order a subtree is
+  // the rows before its root; elsewhere the list lengths below are estimates only (a root that does
+  // not fit escalates, and its subtree then stays uncontracted).
+  constexpr int kSamples = 64;
+  double best = 0.0;
+  int32_t best_t = 0;
+  std::vector<int32_t> up;
+  for (const double share : {0.9, 0.75, 0.6, 0.45, 0.35, 0.25}) {
+    const int32_t t = (int32_t)(share * limit);
+    if (t < kCondMinRoot) break;
+    double gone = 0.0, kept = 0.0;
+    int32_t last = -1;
+    for (int k = 0; k < kSamples; ++k) {
+      int32_t c = (int32_t)((int64_t)n * (2 * k + 1) / (2 * kSamples));
+      if (size[c] > t) continue;
+      while (parent[c] >= 0 && size[parent[c]] <= t) c = parent[c];
+      if (size[c] < kCondMinRoot) continue;
+      if (c != last) {
+        last = c;
+        up.clear();
+        for (int32_t v = std::max(0, c - size[c] + 1); v <= c; ++v)
+          for (int32_t p = P.rowptr[v + 1]; p > P.rowptr[v] && P.adj[p - 1] > c; --p) up.push_back(P.adj[p - 1]);
+        std::sort(up.begin(), up.end());
+        const double u = (double)(std::unique(up.begin(), up.end()) - up.begin());
+        // the directed lists of an unsymmetric pattern miss some of the surface
+        kept = size[c] + 1.1 * u <= limit ? 1.0 - (1.0 + u / kEll) / size[c] : 0.0;
+      }
+      gone += kept;
+    }
+    if (gone > best) {
+      best = gone;
+      best_t = t;
+    }
+  }
+  if (best < (1.0 - kCondMaxShare) * kSamples) return 0;
+  vroot.assign((size_t)n, -1);
+  is_root.assign((size_t)n, 0);
+  int32_t roots = 0;
+  for (int32_t v = n - 1; v >= 0; --v) {
+    if (size[v] > best_t) continue;
+    if (parent[v] >= 0 && size[parent[v]] <= best_t) {
+      vroot[v] = vroot[parent[v]];
+    } else if (size[v] >= kCondMinRoot) {
+      vroot[v] = roots++;
+      is_root[v] = 1;
+    }
+  }
+  return roots;
 }
 
 int32_t light_limit_for(int32_t n, int light_bits) {
@@ -314,6 +371,51 @@ int configure_launch(int32_t n_max, int64_t nrows, bool paired_any, const Option
   return GSOFA_OK;
 }
 
+int configure_condensed(int32_t cn_max, int64_t nodes, const Options& opt, const DeviceInfo& info, LaunchConfig& out) {
+  out = LaunchConfig();
+  out.bw_max = (cn_max + 31) / 32;
+  const size_t reserve = kHeavyCondLdsReserve + heavy_stash_bytes(false);
+  const size_t bitmap_bytes = (size_t)out.bw_max * 4;
+  auto lds_fits = [&](int wgs) { return (size_t)wgs * (bitmap_bytes + reserve + 512 * 8) <= info.lds_per_cu; };
+  // Four workgroups of 256 threads per compute unit while their bitmaps fit: measured (best block
+  // sizes) 128 / 256 / 512 threads: 57 k nodes 1466 / 865 / 919 us, 131 k 3237 / 1851 / 1922, 47 k (3-D)
+  // 2393 / 1266 / 1204, 5.6 k 233 / 181 / 162.
+  int threads = opt.heavy_threads;
+  if (!threads) threads = lds_fits(4) ? 256 : lds_fits(2) ? 512 : 1024;
+  if (threads != 256 && threads != 512 && threads != 1024)
+    return fail(GSOFA_ERR_INVALID_ARG, "heavy_threads must be 256, 512 or 1024");
+  out.heavy_threads = threads;
+  const int target_wgs = opt.heavy_wgs_per_cu ? opt.heavy_wgs_per_cu : 1024 / threads;
+  const size_t budget = std::min(info.lds_per_block, info.lds_per_cu / (size_t)std::max(target_wgs, 1));
+  const int64_t rem = budget > bitmap_bytes + reserve ? (int64_t)(budget - bitmap_bytes - reserve) : 0;
+  if (opt.structure) {
+    const int64_t qmin = opt.qcap ? opt.qcap : 1024;
+    for (int32_t c : {4096, 2048, 1024})
+      if (!out.ucap && rem >= 8 * qmin + 4 * c) out.ucap = c;
+  }
+  int64_t q = opt.qcap;
+  if (!q) {
+    q = rem > 4 * out.ucap ? (rem - 4 * out.ucap) / 8 : 256;
+    q = std::max<int64_t>(256, std::min<int64_t>(16384, q)) & ~int64_t(63);
+  }
+  out.qcap = (int32_t)q;
+  out.heavy_lds = heavy_lds_bytes(out.bw_max, out.qcap, false, out.ucap, false);
+  if (out.heavy_lds + kHeavyCondLdsReserve > info.lds_per_block)
+    return fail(GSOFA_ERR_CAPACITY, "condensed graph: LDS request exceeds the device limit");
+  const int occ = heavy_cond_occupancy(threads, out.heavy_lds);
+  if (occ <= 0) return fail(GSOFA_ERR_CAPACITY, "k_heavy cannot be resident with this LDS size");
+  const int cus = opt.cu_share > 0 ? std::min(opt.cu_share, info.cus) : info.cus;
+  out.heavy_grid = cus * occ;
+  out.heavy_wgs_per_cu = occ;
+  // Nodes per item. A node's traversal starts from its block's earlier ones, so the first of a block
+  // pays for the block; with little left below it that costs less than an idle compute unit. Measured
+  // (256 threads, us of k_heavy at 8 / 16 / 32 / 64 nodes): 2.3 k nodes 164 / 168 / 218 / -, 5.6 k 187 /
+  // 181 / 225 / 318, 47 k (3-D) 1619 / 1266 / 1681 / 2176, 57 k - / 906 / 874 / 944, 131 k - / 2158 /
+  // 1851 / 1854 (24 and 48 nodes lie between their neighbours or above them).
+  out.chain_block = opt.chain_block ? opt.chain_block : nodes < 4096 ? 8 : nodes < 50000 ? 16 : 32;
+  return GSOFA_OK;
+}
+
 int enqueue_preparation(const Sequence& q, hipStream_t s) {
   auto hf = [](hipError_t e, const char* what) {
     return fail(e == hipErrorOutOfMemory ? GSOFA_ERR_OUT_OF_MEMORY : GSOFA_ERR_HIP,
@@ -342,9 +444,10 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
     if (e_ != hipSuccess) return hf(e_, what);  \
   } while (0)
   if (ev) GSOFA_SEQ(hipEventRecord(ev[0], s), "hipEventRecord");
-  GSOFA_SEQ(launch_clear_run(q.acc, (int64_t)q.nmats * kAccSlots, reinterpret_cast<unsigned long long*>(q.ws), 4,
-                             reinterpret_cast<int32_t*>(q.esc), q.esc_words, reinterpret_cast<int32_t*>(q.blk_flag),
-                             2 * q.nblk_total, q.bucket, q.nb_max, s),
+  GSOFA_SEQ(launch_clear_run(q.acc, (int64_t)q.nmats * kAccSlots, reinterpret_cast<unsigned long long*>(q.ws),
+                             q.ncond > 0 ? 8 : 4, reinterpret_cast<int32_t*>(q.esc), q.esc_words,
+                             reinterpret_cast<int32_t*>(q.blk_flag), 2 * q.nblk_total, q.bucket, q.nb_max,
+                             q.cond_zero, q.cond_words, s),
             "clear the run's state");
   if (q.prepare) GSOFA_TRY(enqueue_preparation(q, s));
   if (ev) GSOFA_SEQ(hipEventRecord(ev[1], s), "hipEventRecord");
@@ -360,15 +463,26 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
     if (q.top_ev) GSOFA_SEQ(hipEventRecord(q.top_ev[1], q.side), "hipEventRecord");
     GSOFA_SEQ(hipEventRecord(q.join, q.side), "hipEventRecord(join)");
   }
-  GSOFA_SEQ(launch_light(q.mats, q.nmats, q.item_base, q.nitems, q.ws, q.cfg.light_grid, q.cfg.light_bits, s), "k_light");
+  GSOFA_SEQ(launch_light(q.mats, q.nmats, q.item_base, q.nitems, q.ws, q.cfg.light_grid, q.cfg.light_bits, q.ncond > 0, s),
+            "k_light");
   // cursor, block_sums and total are free again once the transpose is built
-  GSOFA_SEQ(launch_heavy_order(q.mats, q.nblk_total, q.nmats, q.blkq_base, q.blk_flag, q.nb_max, q.bucket, q.cursor,
+  if (q.ncond > 0)
+    GSOFA_SEQ(launch_condense(q.mats, q.cmats, q.nmats, q.row_base, q.nrows, q.cbase, q.cnodes, q.cblk_base, q.cblk_mat,
+                              q.ncond, q.cnblk, q.cut_divisor, q.block_sums, q.total, q.ws_cond, q.citems, s),
+              "condensed graphs");
+  if (q.nplain > 0)
+    GSOFA_SEQ(launch_heavy_order(q.mats, q.nblk_total, q.nmats, q.blkq_base, q.blk_flag, q.nb_max, q.bucket, q.cursor,
                                q.block_sums, q.total, q.ws, q.heavy_items, s),
             "workgroup-path queue");
   if (ev) GSOFA_SEQ(hipEventRecord(ev[2], s), "hipEventRecord");
-  GSOFA_SEQ(launch_heavy(q.cfg.heavy_threads, q.cfg.heavy_grid, q.mats, q.ws, q.heavy_items, q.cfg.bw_max, q.cfg.qcap,
-                         q.n_max, q.paired_any, q.spill, q.hbm_bm, q.cfg.ucap, kAccHeavyExecEdges, s),
-            "k_heavy");
+  if (q.nplain > 0)
+    GSOFA_SEQ(launch_heavy(q.cfg.heavy_threads, q.cfg.heavy_grid, q.mats, q.ws, q.heavy_items, q.cfg.bw_max, q.cfg.qcap,
+                           q.n_max, q.paired_any, q.spill, q.hbm_bm, q.cfg.ucap, kAccHeavyExecEdges, s),
+              "k_heavy");
+  if (q.ncond > 0)
+    GSOFA_SEQ(launch_heavy_cond(q.ccfg.heavy_threads, q.ccfg.heavy_grid, q.cmats, q.ws_cond, q.citems, q.ccfg.bw_max,
+                                q.ccfg.qcap, q.cn_max, q.cspill, q.ccfg.ucap, s),
+              "k_heavy (condensed graphs)");
   if (ev) GSOFA_SEQ(hipEventRecord(ev[3], s), "hipEventRecord");
   if (q.n_top > 0) GSOFA_SEQ(hipStreamWaitEvent(s, q.join, 0), "hipStreamWaitEvent(join)");
   if (q.mirror_any) GSOFA_SEQ(launch_mirror(q.mats, q.nmats, q.blk_base, q.nblocks_sup, s), "k_mirror");
@@ -379,7 +493,7 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
 }
 
 int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream) {
-  opt_ = opt;
+  opt_ = opt_in_ = opt;
   alloc_stream_ = alloc_stream;
   nmats_ = (int)mats.size();
   if (nmats_ <= 0) return fail(GSOFA_ERR_INVALID_ARG, "empty matrix set");
@@ -521,18 +635,12 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   GSOFA_TRY(alloc(item_base_d_, nmats_ + 1, "item base"));
   GSOFA_TRY(alloc(row_base_d_, nmats_ + 1, "row base"));
   GSOFA_TRY(alloc(blk_base_d_, nmats_ + 1, "block base"));
-  GSOFA_TRY(alloc(ws_, n_top_ > 0 ? 2 : 1, "work state"));  // the second: the early launch's
+  GSOFA_TRY(alloc(ws_, 2, "work state"));  // the second: the early launch's, or the condensed graphs'
   GSOFA_TRY(alloc(heavy_items_, 2 * (nblk_total_ + ncut), "escalation list"));
   if (ncut > 0) {
     GSOFA_TRY(alloc(cut_, (size_t)nblk_total_, "block cuts"));
     GSOFA_TRY(upload(cut_, cut_all.data(), cut_all.size() * 4, "upload block cuts"));
   }
-  // per resident workgroup: two frontier spill queues, the U list (beyond its LDS part) and the
-  // saved bitmap of the last row (with paired items: a U list per direction and a ring of the
-  // last saved rows' bitmaps per direction)
-  // (the early launch's workgroups have regions of their own after the main launch's)
-  GSOFA_TRY(alloc(spill_, (size_t)(heavy_grid_ + top_grid_) * (size_t)heavy_region_ints(n_max_, paired_any_ != 0),
-                  "heavy spill regions"));
   if (n_top_ > 0) {
     GSOFA_TRY(alloc(top_items_, (size_t)n_top_, "early items"));
     GSOFA_TRY(upload(top_items_, top_items.data(), top_items.size() * 8, "upload early items"));
@@ -542,7 +650,6 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     GSOFA_HIP(hipEventCreate(&top_ev_[0]), "hipEventCreate");
     GSOFA_HIP(hipEventCreate(&top_ev_[1]), "hipEventCreate");
   }
-  if (hbm_bitmap_) GSOFA_TRY(alloc(hbm_bm_, (size_t)heavy_grid_ * (size_t)bw_max_, "heavy bitmaps"));
   esc_words_ = (2 * nrows_ + 3) / 4;
   GSOFA_TRY(alloc(esc_, (size_t)esc_words_ * 4, "escalation flags"));
   GSOFA_TRY(alloc(blk_flag_, (size_t)(2 * nblk_total_), "block flags"));
@@ -557,7 +664,8 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   // reaches almost nothing below its rows, whatever the subtree) and paired matrices
   // (unstructured: reaches far smaller than their subtrees) keep every attempt. Only matrices
   // with more rows than the limit carry the subtree sizes.
-  std::vector<int32_t> pre_size((size_t)nmats_, INT32_MAX);
+  std::vector<int32_t> pre_size((size_t)nmats_, INT32_MAX), nroots((size_t)nmats_, 0);
+  int32_t list_cap = 0;
   bool any_pre = false;
   if (opt.pre_escalate != -1) {
     for (int b = 0; b < nmats_; ++b) {
@@ -571,15 +679,50 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   }
   if (any_pre) {
     GSOFA_TRY(alloc(subtree_d_, (size_t)nrows_, "subtree sizes"));
-    std::vector<int32_t> sub((size_t)nrows_, 0);
+    std::vector<int32_t> sub((size_t)nrows_, 0), vroot_all, vroot;
+    std::vector<uint8_t> is_root;
     for (int b = 0; b < nmats_; ++b) {
       if (pre_size[b] == INT32_MAX) continue;
       const Prepared& P = *mats[b];
-      if (P.subtree.empty()) subtree_sizes(P, P.subtree);
+      if (P.subtree.empty()) elimination_tree(P);
       std::copy(P.subtree.begin(), P.subtree.end(), sub.begin() + row_base_h_[b]);
+      // the workgroup path on the condensed graph, except where the early launch's fixed items or
+      // HBM bitmaps were asked for
+      if (opt.early_top > 0 || opt.bitmap_in_hbm == 1) continue;
+      nroots[b] = condensation_roots(P, pre_size[b], vroot, is_root);
+      if (nroots[b] == 0) continue;
+      if (vroot_all.empty()) vroot_all.assign((size_t)nrows_, -1);
+      std::copy(vroot.begin(), vroot.end(), vroot_all.begin() + row_base_h_[b]);
+      for (int32_t v = 0; v < P.n; ++v)
+        if (is_root[v]) sub[row_base_h_[b] + v] |= INT32_MIN;
+      list_cap = std::max(list_cap, pre_size[b]);
     }
     GSOFA_TRY(upload(subtree_d_, sub.data(), sub.size() * 4, "upload subtree sizes"));
+    if (!vroot_all.empty()) {
+      GSOFA_TRY(alloc(vroot_, (size_t)nrows_, "condensation roots"));
+      GSOFA_TRY(upload(vroot_, vroot_all.data(), vroot_all.size() * 4, "upload condensation roots"));
+    }
     if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(subtree sizes)");
+  }
+  int64_t roots_all = 0;
+  std::vector<int64_t> root_base((size_t)nmats_ + 1, 0);
+  for (int b = 0; b < nmats_; ++b) root_base[b + 1] = root_base[b] + nroots[b];
+  roots_all = root_base[nmats_];
+  cond_.assign((size_t)nmats_, 0);
+  uint8_t* marks = nullptr;
+  int32_t *root_cnt = nullptr, *root_bad = nullptr;
+  if (roots_all > 0) {
+    // cleared by every run: the marks of both directions (bytes), then per root its two counts and
+    // whether its subtree holds an escalated row
+    const int64_t mark_words = (2 * nrows_ + 3) / 4;
+    cond_words_ = mark_words + 3 * roots_all;
+    GSOFA_TRY(alloc(cond_zero_, (size_t)cond_words_, "condensation marks"));
+    marks = reinterpret_cast<uint8_t*>(cond_zero_);
+    root_cnt = cond_zero_ + mark_words;
+    root_bad = root_cnt + 2 * roots_all;
+    GSOFA_TRY(alloc(root_list_, (size_t)(2 * roots_all * list_cap), "condensation lists"));
+    GSOFA_TRY(alloc(root_wri_, (size_t)(3 * roots_all), "condensation root weights"));
+    GSOFA_TRY(alloc(nid_, (size_t)nrows_, "condensation nodes"));
   }
   if (any_dup) {
     GSOFA_TRY(alloc(dup_u_, nrows_, "duplicate surplus (upper)"));
@@ -654,12 +797,160 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     M.light_limit = light_limit_for(ns_[b], cfg_.light_bits);
     M.subtree = pre_size[b] != INT32_MAX ? subtree_d_ + rb : nullptr;
     M.pre_size = pre_size[b];
+    M.rows = ns_[b];
+    if (nroots[b] > 0) {
+      cond_[b] = 1;
+      const int64_t r0 = root_base[b];
+      M.vroot = vroot_ + rb;
+      M.nid = nid_ + rb;
+      for (int d = 0; d < 2; ++d) {
+        M.mark[d] = marks + d * nrows_ + rb;
+        M.root_cnt[d] = root_cnt + d * roots_all + r0;
+        M.root_list[d] = root_list_ + (d * roots_all + r0) * list_cap;
+      }
+      M.root_bad = root_bad + r0;
+      M.root_w = root_wri_ + r0;
+      M.root_r = root_wri_ + roots_all + r0;
+      M.root_id = root_wri_ + 2 * roots_all + r0;
+      M.list_cap = list_cap;
+    }
   }
   GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
   // The pattern is fixed for the set's lifetime, and so are its device forms (ELL rows, A^T): built
   // here once, like the upload, not on every run.
   GSOFA_TRY(enqueue_preparation(sequence(), alloc_stream_));
+  if (roots_all > 0) GSOFA_TRY(create_condensed(info));
   GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(preparation)");
+  nplain_ = nmats_ - ncond_;
+  if (nplain_ > 0) {
+    // per resident workgroup: two frontier spill queues, the U list (beyond its LDS part) and the
+    // saved bitmap of the last row (with paired items: a U list per direction and a ring of the
+    // last saved rows' bitmaps per direction)
+    // (the early launch's workgroups have regions of their own after the main launch's)
+    GSOFA_TRY(alloc(spill_, (size_t)(heavy_grid_ + top_grid_) * (size_t)heavy_region_ints(n_max_, paired_any_ != 0),
+                    "heavy spill regions"));
+    if (hbm_bitmap_) GSOFA_TRY(alloc(hbm_bm_, (size_t)heavy_grid_ * (size_t)bw_max_, "heavy bitmaps"));
+  } else {
+    heavy_threads_ = ccfg_.heavy_threads;
+    heavy_grid_ = ccfg_.heavy_grid;
+    heavy_wgs_per_cu_ = ccfg_.heavy_wgs_per_cu;
+    qcap_ = ccfg_.qcap;
+    opt_.chain_block = ccfg_.chain_block;
+  }
+  return GSOFA_OK;
+}
+
+// The condensed graphs' buffers. Their sizes are counted by one wave path over the set (nothing
+// else of that run is kept; every run builds its graphs anew, and reports an error should it count
+// other sizes).
+int DeviceSet::create_condensed(const DeviceInfo& info) {
+  hipStream_t s = alloc_stream_;
+  unsigned long long* sizes_d = nullptr;
+  GSOFA_TRY(alloc(sizes_d, (size_t)nmats_, "condensed sizes"));
+  Sequence q = sequence();
+  GSOFA_HIP(launch_clear_run(q.acc, (int64_t)nmats_ * kAccSlots, reinterpret_cast<unsigned long long*>(ws_), 8,
+                             reinterpret_cast<int32_t*>(esc_), esc_words_, reinterpret_cast<int32_t*>(blk_flag_),
+                             2 * nblk_total_, bucket_, nb_max_, cond_zero_, cond_words_, s),
+            "clear the run's state");
+  GSOFA_HIP(launch_fill_u64(sizes_d, nmats_, 0, s), "clear condensed sizes");
+  GSOFA_HIP(launch_light(q.mats, nmats_, q.item_base, nitems_, ws_, cfg_.light_grid, cfg_.light_bits, true, s),
+            "k_light");
+  GSOFA_HIP(launch_cond_sizes(q.mats, nmats_, q.row_base, nrows_, sizes_d, s), "condensed sizes");
+  std::vector<unsigned long long> sizes((size_t)nmats_, 0);
+  GSOFA_TRY(download(sizes.data(), sizes_d, sizes.size() * 8, "read condensed sizes"));
+  // a matrix whose graph keeps too many vertices (roots that did not fit the wave path) runs as it is
+  auto drop = [&](int b) -> int {
+    cond_[b] = 0;
+    std::vector<int32_t> sub((size_t)ns_[b]);
+    MatDev& M = mats_h_[b];
+    GSOFA_TRY(download(sub.data(), M.subtree, sub.size() * 4, "read subtree sizes"));
+    for (int32_t& x : sub) x &= INT32_MAX;
+    GSOFA_TRY(upload(const_cast<int32_t*>(M.subtree), sub.data(), sub.size() * 4, "upload subtree sizes"));
+    if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(subtree sizes)");
+    M.vroot = nullptr;
+    return GSOFA_OK;
+  };
+  for (int b = 0; b < nmats_; ++b)
+    if (cond_[b] && (double)sizes[b] > (kCondMaxShare + 0.1) * ns_[b]) GSOFA_TRY(drop(b));
+  auto total = [&] {
+    cn_max_ = 0;
+    cnodes_ = 0;
+    ncond_ = 0;
+    for (int b = 0; b < nmats_; ++b)
+      if (cond_[b]) {
+        cn_max_ = std::max(cn_max_, (int32_t)sizes[b]);
+        cnodes_ += (int64_t)sizes[b];
+        ++ncond_;
+      }
+  };
+  total();
+  if (ncond_ > 0) {
+    const int rc = configure_condensed(cn_max_, cnodes_, opt_in_, info, ccfg_);
+    if (rc == GSOFA_ERR_CAPACITY) {
+      for (int b = 0; b < nmats_; ++b)
+        if (cond_[b]) GSOFA_TRY(drop(b));
+      total();
+    } else if (rc != GSOFA_OK) {
+      return rc;
+    }
+  }
+  if (ncond_ > 0) {
+    const int32_t K = ccfg_.chain_block;
+    std::vector<int64_t> cbase((size_t)nmats_ + 1, 0), cblk_base;
+    std::vector<int32_t> order;
+    for (int b = 0; b < nmats_; ++b) {
+      cbase[b + 1] = cbase[b] + (cond_[b] ? (int64_t)sizes[b] : 0);
+      if (cond_[b]) order.push_back(b);
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return sizes[x] > sizes[y]; });
+    cblk_base.push_back(0);
+    for (int32_t b : order) cblk_base.push_back(cblk_base.back() + ((int64_t)sizes[b] + K - 1) / K);
+    cnblk_ = cblk_base.back();
+    cut_divisor_ = opt_in_.split_blocks == -1 ? 0 : opt_in_.split_blocks > 0 ? opt_in_.split_blocks : kCutDivisor;
+    int32_t *orig = nullptr, *wt = nullptr, *ell[2] = {nullptr, nullptr}, *rp[2] = {nullptr, nullptr};
+    int32_t* adj[2] = {nullptr, nullptr};
+    uint8_t* esc = nullptr;
+    GSOFA_TRY(alloc(orig, (size_t)cnodes_, "condensed nodes"));
+    GSOFA_TRY(alloc(wt, (size_t)(2 * cnodes_), "condensed weights"));
+    GSOFA_TRY(alloc(esc, (size_t)(2 * cnodes_), "condensed escalations"));
+    for (int d = 0; d < (mirror_all_ ? 1 : 2); ++d) {
+      GSOFA_TRY(alloc(ell[d], (size_t)(cnodes_ * kEll), "condensed ELL"));
+      GSOFA_TRY(alloc(rp[d], (size_t)(cnodes_ + 1), "condensed row ends"));
+      GSOFA_TRY(alloc(adj[d], (size_t)nnz_, "condensed tails"));
+    }
+    GSOFA_HIP(launch_fill_i32(orig, cnodes_, 0, s), "clear condensed nodes");
+    GSOFA_TRY(alloc(cmats_d_, (size_t)nmats_, "condensed table"));
+    GSOFA_TRY(alloc(cbase_d_, cbase.size(), "condensed node base"));
+    GSOFA_TRY(alloc(cblk_base_d_, cblk_base.size(), "condensed block base"));
+    GSOFA_TRY(alloc(cblk_mat_d_, order.size(), "condensed order"));
+    GSOFA_TRY(alloc(citems_, (size_t)(4 * cnblk_), "condensed items"));
+    GSOFA_TRY(alloc(cspill_, (size_t)ccfg_.heavy_grid * (size_t)heavy_region_ints(cn_max_, false), "condensed spill regions"));
+    GSOFA_TRY(upload(cbase_d_, cbase.data(), cbase.size() * 8, "upload"));
+    GSOFA_TRY(upload(cblk_base_d_, cblk_base.data(), cblk_base.size() * 8, "upload"));
+    GSOFA_TRY(upload(cblk_mat_d_, order.data(), order.size() * 4, "upload"));
+    cmats_h_ = mats_h_;
+    for (int b = 0; b < nmats_; ++b) {
+      MatDev& C = cmats_h_[b];
+      C.n = (int32_t)(cbase[b + 1] - cbase[b]);
+      for (int d = 0; d < 2; ++d) {
+        C.ell[d] = ell[d] ? ell[d] + cbase[b] * kEll : nullptr;
+        C.rowptr[d] = rp[d] ? rp[d] + cbase[b] : nullptr;
+        C.adj[d] = adj[d];
+        C.esc[d] = esc + d * cnodes_ + cbase[b];
+      }
+      C.chain_block = K;
+      C.split = nullptr;
+      C.paired = 0;
+      C.orig = orig + cbase[b];
+      C.wt = wt + 2 * cbase[b];
+    }
+    GSOFA_TRY(upload(cmats_d_, cmats_h_.data(), sizeof(MatDev) * nmats_, "upload condensed table"));
+    if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(condensed tables)");
+  } else {
+    cond_words_ = 0;
+  }
+  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(condensed graphs)");
   return GSOFA_OK;
 }
 
@@ -692,7 +983,11 @@ int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Opt
   b += 4 * (heavy_grid + kTopMaxItems) * heavy_region_ints(nmax, paired);  // spill (and the early launch's)
   if (place_bitmaps_in_hbm(nmax, opt, info)) b += 4 * (int64_t)cus * (((int64_t)nmax + 31) / 32);  // one per CU
   if (dup) b += 8 * nrows;
-  if (opt.pre_escalate != -1) b += 4 * nrows;  // subtree sizes (at most one per row)
+  // subtree sizes, and the condensed graphs (roots, nodes, marks; lists of at most kLightLimitBig per
+  // kCondMinRoot rows and direction; nodes of at most kCondMaxShare + 0.1 of the rows)
+  if (opt.pre_escalate != -1)
+    b += 14 * nrows + 8 * nrows / kCondMinRoot * kLightLimitBig + 8 * nnz + (int64_t)(0.7 * 150.0 * (double)nrows) +
+         4 * heavy_grid * heavy_region_ints(nmax, false);
   if (opt.structure) b += 16 * (nrows + (int64_t)mats.size());  // offsets; pools are sized later
   b += 1 << 20;                       // tables, accumulators, scan scratch
   *out_bytes = b;
@@ -754,6 +1049,22 @@ Sequence DeviceSet::sequence() const {
   q.row_base = row_base_d_;
   q.blk_base = blk_base_d_;
   q.blkq_base = blkq_base_d_;
+  q.ncond = ncond_;
+  q.nplain = nplain_;
+  q.cmats = cmats_d_;
+  q.cbase = cbase_d_;
+  q.cblk_base = cblk_base_d_;
+  q.cblk_mat = cblk_mat_d_;
+  q.cnodes = cnodes_;
+  q.cnblk = cnblk_;
+  q.cond_words = cond_words_;
+  q.cn_max = cn_max_;
+  q.cut_divisor = cut_divisor_;
+  q.cond_zero = cond_zero_;
+  q.citems = citems_;
+  q.ws_cond = ws_ + 1;
+  q.cspill = cspill_;
+  q.ccfg = ccfg_;
   q.n_top = n_top_;
   q.top_grid = top_grid_;
   q.top_items = top_items_;
@@ -772,7 +1083,8 @@ int DeviceSet::read_results(std::vector<MatResult>& out) {
   for (int b = 0; b < nmats_; ++b) {
     const unsigned long long* a = acc.data() + (size_t)b * kAccSlots;
     if (a[kAccOverflow]) return fail(GSOFA_ERR_STATE, "structure offsets do not match this run's counts");
-    if (a[kAccScheduleError]) return fail(GSOFA_ERR_STATE, "wave path: a wave stopped waiting for its sibling's item");
+    if (a[kAccScheduleError]) return fail(GSOFA_ERR_STATE, "the run's schedule broke (a wave stopped waiting for its sibling's item, or a condensed "
+                                    "graph changed its size)");
     MatResult& r = out[b];
     r.fill = a[kAccFill];
     r.W = a[kAccW];
@@ -856,8 +1168,14 @@ int DeviceSet::size_pools_from_counts() {
     M.list_ptr[1] = list_ptr_l_ + ptr_base_h_[b];
     M.pool[0] = pool_u_ + pool_base_u_[b];
     M.pool[1] = pool_l_ + pool_base_l_[b];
+    if (ncond_ > 0)
+      for (int d = 0; d < 2; ++d) {
+        cmats_h_[b].list_ptr[d] = M.list_ptr[d];
+        cmats_h_[b].pool[d] = M.pool[d];
+      }
   }
   GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  if (ncond_ > 0) GSOFA_TRY(upload(cmats_d_, cmats_h_.data(), sizeof(MatDev) * nmats_, "upload condensed table"));
   if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(offsets)");
   pools_sized_ = true;
   return GSOFA_OK;

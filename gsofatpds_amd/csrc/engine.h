@@ -26,6 +26,7 @@ struct Prepared {
   // Subtree sizes of the elimination tree of A + A^T (|T[s]| bounds |R_s| + 1), computed on
   // first use (block cuts) and kept.
   mutable std::vector<int32_t> subtree;
+  mutable std::vector<int32_t> parent;  // that tree's parents (-1: a root), with the sizes
 };
 
 // Rows where chain blocks are cut into two workgroup-path items: in each block the row s whose
@@ -49,6 +50,17 @@ int32_t top_separator_rows(const Prepared& P, const std::vector<int32_t>& cut);
 constexpr double kPreSymmetry = 0.75;
 // The wave path's escalation limit for a matrix of n rows under a hash-set variant.
 int32_t light_limit_for(int32_t n, int light_bits);
+// The roots of a matrix's condensed graph (kernels.hip): the rows of at least kCondMinRoot vertices
+// whose elimination subtree has at most T vertices while their parent's has more. T is the share of
+// the wave path's limit that lets the most vertices be contracted: a root's reached set and its U
+// list must both fit the limit (surfaces are larger in 3-D than in 2-D), estimated on sampled
+// vertices. vroot[v] becomes the index of the root whose subtree holds v, or -1, and is_root[v] 1 for
+// the roots. Returns the number of roots, or 0 where the graph would keep more than kCondMaxShare of
+// the vertices (little to gain: natural-order bands, whose subtrees are long chains).
+int32_t condensation_roots(const Prepared& P, int32_t limit, std::vector<int32_t>& vroot, std::vector<uint8_t>& is_root);
+constexpr int32_t kCondMinRoot = 32;
+constexpr double kCondMaxShare = 0.6;
+
 // At most this many items go to the early launch (one workgroup each), and this many per
 // direction of a matrix (each over several chain blocks).
 constexpr int64_t kTopMaxItems = 32;
@@ -114,6 +126,9 @@ struct LaunchConfig {
   bool hbm_bitmap = false;
   size_t heavy_lds = 0;  // dynamic LDS bytes of k_heavy
 };
+// The same for the workgroup path on condensed graphs (`nodes` in all, at most cn_max in one).
+// GSOFA_ERR_CAPACITY: they do not fit (the matrices then run uncondensed).
+int configure_condensed(int32_t cn_max, int64_t nodes, const Options& opt, const DeviceInfo& info, LaunchConfig& out);
 // Picks the configuration for a set whose largest matrix has n_max rows (nrows in all) and sets
 // k_heavy's LDS limit. max_heavy_grid > 0 caps the bitmap-path workgroups (each holds a spill
 // region of heavy_region_ints(n_max) ints), for callers whose regions live in a fixed buffer.
@@ -141,6 +156,19 @@ struct Sequence {
   uint32_t *blk_flag = nullptr, *hbm_bm = nullptr;
   MatDev* mats = nullptr;
   int64_t *item_base = nullptr, *row_base = nullptr, *blk_base = nullptr, *blkq_base = nullptr;
+  // The condensed graphs (ncond > 0 matrices, built after the wave path by launch_condense) and their
+  // workgroup-path launch; nplain: matrices that run uncondensed (none: no such launch).
+  int ncond = 0, nplain = 0;
+  MatDev* cmats = nullptr;
+  int64_t *cbase = nullptr, *cblk_base = nullptr;
+  int32_t* cblk_mat = nullptr;
+  int64_t cnodes = 0, cnblk = 0, cond_words = 0;
+  int32_t cn_max = 0, cut_divisor = 0;
+  int32_t* cond_zero = nullptr;  // marks and lists, cleared by every run
+  uint64_t* citems = nullptr;
+  WorkState* ws_cond = nullptr;
+  int32_t* cspill = nullptr;
+  LaunchConfig ccfg;
   // The early launch (n_top > 0): top_grid workgroups of k_heavy over the fixed items top_items
   // on `side`, forked from the run's stream after its clears and joined before k_mirror and
   // k_supernodes; its own work state and spill regions. top_ev (optional, 2 events) brackets it.
@@ -208,6 +236,7 @@ class DeviceSet {
   int hip_fail(hipError_t e, const char* what);
 
   Options opt_;
+  Options opt_in_;  // as given to create() (opt_ carries the chosen block size)
   int nmats_ = 0;
   std::vector<int32_t> ns_;
   std::vector<int64_t> row_base_h_, item_base_h_, blk_base_h_;
@@ -255,6 +284,20 @@ class DeviceSet {
   std::vector<int64_t> pool_base_u_, pool_base_l_;        // per matrix, into the pools
   std::vector<std::vector<int64_t>> u_ptr_h_, l_ptr_h_;    // host copies of the offsets
   std::vector<MatDev> mats_h_;
+  // the condensed graphs (Sequence)
+  int create_condensed(const DeviceInfo& info);
+  int ncond_ = 0, nplain_ = 0;
+  std::vector<uint8_t> cond_;         // per matrix: its workgroup path runs on the condensed graph
+  std::vector<MatDev> cmats_h_;
+  MatDev* cmats_d_ = nullptr;
+  int64_t *cbase_d_ = nullptr, *cblk_base_d_ = nullptr;
+  int32_t* cblk_mat_d_ = nullptr;
+  int64_t cnodes_ = 0, cnblk_ = 0, cond_words_ = 0;
+  int32_t cn_max_ = 0, cut_divisor_ = 0;
+  int32_t *vroot_ = nullptr, *nid_ = nullptr, *cond_zero_ = nullptr, *root_list_ = nullptr, *root_wri_ = nullptr;
+  uint64_t* citems_ = nullptr;
+  int32_t* cspill_ = nullptr;
+  LaunchConfig ccfg_;
   std::vector<void*> owned_;
   hipStream_t alloc_stream_ = nullptr;
   // the early launch of top-separator items (top_separator_rows)

@@ -75,9 +75,27 @@ struct MatDev {
                                   // (a top separator's, n: none) are fixed workgroup-path items of
                                   // an early launch, escalated from the start
   int32_t light_limit;            // reached vertices before the wave path escalates a row
-  const int32_t* subtree;         // n: elimination-subtree sizes of A + A^T (null: none)
+  const int32_t* subtree;         // n: elimination-subtree sizes of A + A^T (null: none); the sign
+                                  // bit marks a condensation root
   int32_t pre_size;               // a row whose subtree exceeds this escalates without a
                                   // wave-path attempt (its reached set would exceed the limit)
+  // Condensation (kernels.hip, "condensed graph"). Of a matrix whose workgroup path runs on the
+  // condensed graph; vroot is null otherwise.
+  const int32_t* vroot;           // n: the root whose elimination subtree holds the vertex, or -1
+  uint8_t* mark[2];               // n: 1 where the vertex is in its root's R (per direction)
+  int32_t* root_cnt[2];           // per root: 1 + entries of its list, 0 while it has not finished
+  int32_t* root_list[2];          // per root, list_cap entries: U of the root, then the vertices of
+                                  // its R that the contraction leaves out
+  int32_t* root_bad;              // per root: 1 when some row of its subtree escalated
+  int32_t *root_w, *root_r;       // per root: sum of degrees of, and vertices in, {root} + R (dir. 0)
+  int32_t* root_id;               // per root: its node
+  int32_t* nid;                   // n: the vertex's node, -1 where it is part of its root's
+  int32_t list_cap;
+  // A condensed graph as k_heavy sees it (n nodes; ell, rowptr, adj, esc by node).
+  const int32_t* orig;            // n: the node's vertex, or -(r + 1): a list node of root r
+  const int32_t* wt;              // 2 n: what to add to the node's entry count for its input degree,
+                                  // and to 1 for its vertices (direction 0's totals)
+  int32_t rows;                   // vertices of the matrix
 };
 
 // Scheduler state of one launch set (plain matrix or batch).
@@ -85,7 +103,7 @@ struct WorkState {
   unsigned long long light_next;   // next pair of wave-path items
   unsigned long long heavy_count;  // items escalated to the workgroup path
   unsigned long long heavy_next;   // next escalated item
-  unsigned long long pad;
+  unsigned long long cut_count;    // condensed graphs: items before a cut (they go first)
 };
 
 // Item encoding for the escalation list: rows before a cut (bit 63), extra blocks e (bits
@@ -94,6 +112,7 @@ struct WorkState {
 // chain_block rows (v is the block's first row, or a cut; e > 0 only for the early launch's
 // items), or, with bit 63, the rows of v's block before v.
 constexpr int kItemExtraMax = 1023;
+constexpr uint64_t kNoItem = ~0ull;  // condensed graphs: a block without an escalated row
 __host__ __device__ inline uint64_t encode_item(uint32_t mat, uint32_t dir, uint32_t row, uint32_t before_cut,
                                                 uint32_t extra = 0) {
   return ((uint64_t)before_cut << 63) | ((uint64_t)extra << 53) | ((uint64_t)mat << 33) | ((uint64_t)dir << 32) |
@@ -108,11 +127,11 @@ __host__ __device__ inline uint64_t encode_item(uint32_t mat, uint32_t dir, uint
 
 namespace gsofa {
 hipError_t launch_fill_u64(unsigned long long* p, int64_t count, unsigned long long v, hipStream_t s);
-// A run's clears in one launch (all to zero): nacc u64 at acc, nws u64 at ws, nesc, nblk and
-// nbucket i32 words at esc, blk_flag and bucket.
+// A run's clears in one launch (all to zero): nacc u64 at acc, nws u64 at ws, nesc, nblk, nbucket
+// and ncond i32 words at esc, blk_flag, bucket and cond.
 hipError_t launch_clear_run(unsigned long long* acc, int64_t nacc, unsigned long long* ws, int64_t nws, int32_t* esc,
                             int64_t nesc, int32_t* blk_flag, int64_t nblk, int32_t* bucket, int64_t nbucket,
-                            hipStream_t s);
+                            int32_t* cond, int64_t ncond, hipStream_t s);
 hipError_t launch_fill_i32(int32_t* p, int64_t count, int32_t v, hipStream_t s);
 hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* ell, hipStream_t s);
@@ -121,9 +140,10 @@ hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, c
 hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* col_cnt, int32_t* rowptr_t, int32_t* cursor,
                             int32_t* adj_t, int32_t* block_sums, int32_t* total, hipStream_t s);
-// bits: kLightBits, or kLightBitsBig (a hash set of 2,048 slots and an escalation limit of 1,024)
+// bits: kLightBits, or kLightBitsBig (a hash set of 2,048 slots and an escalation limit of 1,024);
+// roots: some matrix has condensation roots (vroot)
 hipError_t launch_light(const MatDev* mats, int nmats, const int64_t* item_base, int64_t nitems, WorkState* ws, int grid, int bits,
-                        hipStream_t s);
+                        bool roots, hipStream_t s);
 // The escalated blocks (blk_flag, 2 * nblk_total slots) into heavy_items in descending block
 // order; sets ws->heavy_count. bucket has nb_max entries, cursor nb_max + 1, block_sums
 // ceil(nb_max / 4096), total one int.
@@ -159,6 +179,23 @@ constexpr int64_t heavy_region_ints(int64_t n_max, bool paired_any) {
 hipError_t launch_heavy(int threads, int grid, const MatDev* mats, WorkState* ws, const uint64_t* heavy_items,
                         int32_t bw_max, int32_t qcap, int64_t n_max, int32_t paired_any, int32_t* spill,
                         uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, hipStream_t s);
+// The condensed graphs (kernels.hip): sizes[b] += nodes of matrix b, after a wave path over zeroed
+// marks, lists and sizes.
+hipError_t launch_cond_sizes(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows,
+                             unsigned long long* sizes, hipStream_t s);
+// Builds them after the wave path: cmats the condensed matrices (by matrix index), cbase[b] the first
+// of the set's `nodes` nodes that is matrix b's, cblk_base / cblk_mat the ncond condensed matrices'
+// blocks in item order. Items: 2 nblk, then at most 2 nblk before cuts (cut_divisor 0: no cuts).
+hipError_t launch_condense(const MatDev* mats, const MatDev* cmats, int nmats, const int64_t* row_base, int64_t nrows,
+                           const int64_t* cbase, int64_t nodes, const int64_t* cblk_base, const int32_t* cblk_mat,
+                           int ncond, int64_t nblk, int32_t cut_divisor, int32_t* block_sums, int32_t* total,
+                           WorkState* ws, uint64_t* items, hipStream_t s);
+// k_heavy on the condensed matrices (256, 512 or 1024 threads).
+hipError_t launch_heavy_cond(int threads, int grid, const MatDev* cmats, WorkState* ws, const uint64_t* items,
+                             int32_t bw_max, int32_t qcap, int64_t n_max, int32_t* spill, int32_t ucap, hipStream_t s);
+// Sets its LDS limit and returns its resident workgroups per CU (0: it cannot run).
+int heavy_cond_occupancy(int threads, size_t bytes);
+constexpr size_t kHeavyCondLdsReserve = 4096;  // its static LDS plus margin
 // Before the early launch: every matrix's rows [light_end, n) escalated (both directions), and
 // ws->heavy_count = count, ws->heavy_next = 0 (one block per matrix).
 hipError_t launch_top_setup(const MatDev* mats, int nmats, WorkState* ws, int64_t count, hipStream_t s);

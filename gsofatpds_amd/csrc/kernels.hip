@@ -48,6 +48,7 @@ __device__ __forceinline__ void gstore(T* p, T v) {
   *(GSOFA_GLOBAL T*)(p) = v;
 }
 typedef int32_t v4i32 __attribute__((ext_vector_type(4)));
+typedef int32_t v2i32 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ v4i32 gload_v4(const int32_t* p) { return *(const GSOFA_GLOBAL v4i32*)(p); }
 
 __device__ __forceinline__ uint32_t rank_below(uint64_t mask) {
@@ -142,18 +143,21 @@ __global__ void k_fill_i32(int32_t* p, int64_t count, int32_t v) {
     p[i] = v;
 }
 
-// A run's clears in one launch: accumulators and work state (u64), escalation and block flags
-// and the workgroup-path queue's buckets (i32 words), all to zero.
+// A run's clears in one launch: accumulators and work state (u64), escalation and block flags,
+// the workgroup-path queue's buckets and the condensation's marks and lists (i32 words), all to
+// zero.
 __global__ void k_clear_run(unsigned long long* __restrict__ acc, int64_t nacc, unsigned long long* __restrict__ ws,
                             int64_t nws, int32_t* __restrict__ esc, int64_t nesc, int32_t* __restrict__ blk_flag,
-                            int64_t nblk, int32_t* __restrict__ bucket, int64_t nbucket) {
-  const int64_t total = nacc + nws + nesc + nblk + nbucket;
+                            int64_t nblk, int32_t* __restrict__ bucket, int64_t nbucket, int32_t* __restrict__ cond,
+                            int64_t ncond) {
+  const int64_t total = nacc + nws + nesc + nblk + nbucket + ncond;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
     if (i < nacc) acc[i] = 0ull;
     else if (i < nacc + nws) ws[i - nacc] = 0ull;
     else if (i < nacc + nws + nesc) esc[i - nacc - nws] = 0;
     else if (i < nacc + nws + nesc + nblk) blk_flag[i - nacc - nws - nesc] = 0;
-    else bucket[i - nacc - nws - nesc - nblk] = 0;
+    else if (i < nacc + nws + nesc + nblk + nbucket) bucket[i - nacc - nws - nesc - nblk] = 0;
+    else cond[i - nacc - nws - nesc - nblk - nbucket] = 0;
   }
 }
 
@@ -438,7 +442,9 @@ __device__ __forceinline__ bool hash_has(const int32_t* H, int32_t m) {
 // X_s). A row that holds an escalated u < s escalates without an attempt: X_u, already over the
 // limit, is part of X_s.
 
-template <int kBits>
+// kRoots: some matrix of the set has condensation roots (the extra code costs the 1,024-slot variant
+// registers: 1 % on a 1,024-row matrix).
+template <int kBits, bool kRoots>
 __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_eu(kBits == kLightBitsBig ? 3 : 5))) void k_light(
     const MatDev* __restrict__ mats, int nmats, const int64_t* __restrict__ item_base, int64_t nitems,
     WorkState* __restrict__ ws) {
@@ -601,7 +607,8 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
       const int32_t chunk_end = min(M.n, (src / M.chunk + 1) * M.chunk);
       // A row whose elimination subtree exceeds pre_size escalates at once: its reached set holds
       // its whole subtree (mirrored matrices), or nearly (pre_size leaves a margin otherwise).
-      const bool pre = M.subtree != nullptr && gload(M.subtree + src) > M.pre_size;
+      const int32_t sub = M.subtree != nullptr ? gload(M.subtree + src) : 0;
+      const bool pre = (kRoots ? sub & INT32_MAX : sub) > M.pre_size;
       RowCursor rc;
       // the source row, one ELL slot per lane (lanes 0..15); slot 15 <= -2 encodes a CSR tail
       const int32_t sm = lane < kEll ? gload(M.ell[dir] + (int64_t)src * kEll + lane) : kPad;
@@ -895,6 +902,26 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
               for (int i = lane; i < uq; i += 64) gstore(M.pool[dir] + off + i, Q[kLightQ - 1 - i]);
             }
           }
+          // A condensation root: its reached vertices are marked and its U list is kept.
+          if (kRoots && sub < 0) {
+            const int32_t r = gload(M.vroot + src);
+            int32_t* const list = M.root_list[dir] + (int64_t)r * M.list_cap;
+            int32_t nl = 0;
+            for (int i = lane; i < kHash; i += 64) {
+              const int32_t m = H[i];
+              if (m >= 0 && m < src) gstore(M.mark[dir] + m, (uint8_t)1);
+              const uint64_t mu = __ballot(m > src);
+              if (m > src) gstore(list + nl + (int32_t)rank_below(mu), m);
+              nl += __popcll(mu);
+            }
+            if (lane == 0) {
+              gstore(M.root_cnt[dir] + r, nl + 1);
+              if (dir == 0) {
+                gstore(M.root_w + r, (int32_t)(wr + deg0));
+                gstore(M.root_r + r, (int32_t)rr + 1);
+              }
+            }
+          }
           carry_ok = true;
           prev_esc = false;
           u_prev = U;
@@ -906,7 +933,12 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
       if (esc) {
         if (lane == 0) {
           gstore(M.esc[dir] + src, (uint8_t)1);
-          gstore(M.blk_flag[dir] + src / M.chain_block, 1u);  // the block goes to the workgroup path
+          if (!kRoots || M.vroot == nullptr) {
+            gstore(M.blk_flag[dir] + src / M.chain_block, 1u);  // the block goes to the workgroup path
+          } else if (!pre) {  // its root's subtree stays as it is (a pre-escalated row lies in none)
+            const int32_t r = gload(M.vroot + src);
+            if (r >= 0) gstore(M.root_bad + r, 1);
+          }
         }
         carry_ok = false;
         prev_esc = true;
@@ -1000,6 +1032,298 @@ __global__ void k_heavy_scatter(const MatDev* __restrict__ mats, int64_t nblk_to
     } else {
       const int32_t pos = atomicAdd(&cursor[nb_max - 1 - b], 1);
       heavy_items[pos] = encode_item((uint32_t)m, dir, (uint32_t)(b * mats[m].chain_block), 0u);
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------
+// The condensed graph of a matrix, on which the workgroup path runs.
+//
+// Every block of the workgroup path begins with a traversal of its first row's whole reached set,
+// most of which lies in small subtrees that the wave path has finished already. Let c be a root: a
+// row whose elimination subtree T(c) of A + A^T is small enough for the wave path while its
+// parent's is not. R_c lies in T(c), and S(c) = {c} + (R_c of A, R_c of A^T) is strongly connected
+// through vertices up to c. A source s outside T(c) reaches, through vertices below s, all of S(c)
+// or none of it (T(c) lies below s when s reaches it at all), so S(c) may be contracted into the
+// node c: its edges are U_c and the vertices of R_c outside S(c), its weights |S(c)| and the sum of
+// S(c)'s degrees. Roots whose subtree holds an escalated row stay as they are. Nodes keep the order
+// of their vertices (a contracted set takes its root's place), so every rule of k_heavy (chaining,
+// imports, cuts) holds on the condensed graph as on the matrix, and the U lists are the same.
+//
+// A root's edges do not fit one 16-entry row: they are held by list nodes right below the root
+// (leaves of up to 16 edges, then nodes over up to 16 leaves when there are more than 16 leaves),
+// which have no vertices and no degree of their own.
+//
+// 659,033-row 2-D stencil: 57 k nodes for 659 k vertices (a 7 KB bitmap instead of 82 KB, so
+// several workgroups per CU).
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ int32_t cond_leaves(int32_t len) { return len <= kEll ? 0 : (len + kEll - 1) / kEll; }
+__device__ __forceinline__ int32_t cond_mids(int32_t leaves) {
+  return leaves <= kEll ? 0 : (leaves + kEll - 1) / kEll;
+}
+__device__ __forceinline__ int32_t cond_list_len(const MatDev& M, int d, int32_t r) {
+  return M.sym && d == 1 ? 0 : min(gload(M.root_cnt[d] + r) - 1, M.list_cap);
+}
+__device__ __forceinline__ int32_t cond_list_nodes(const MatDev& M, int32_t r) {
+  const int32_t l0 = cond_leaves(cond_list_len(M, 0, r)), l1 = cond_leaves(cond_list_len(M, 1, r));
+  return max(l0 + cond_mids(l0), l1 + cond_mids(l1));
+}
+// Whether root r is contracted: finished in both directions, and no row of its subtree escalated.
+__device__ __forceinline__ bool cond_valid(const MatDev& M, int32_t r) {
+  return gload(M.root_cnt[0] + r) != 0 && (M.sym || gload(M.root_cnt[1] + r) != 0) && gload(M.root_bad + r) == 0;
+}
+// The nodes vertex v brings: itself, a contracted root's list nodes and itself, or none (contracted).
+__device__ __forceinline__ int32_t cond_nodes(const MatDev& M, int32_t v) {
+  if (M.vroot == nullptr) return 0;
+  const int32_t r = gload(M.vroot + v);
+  if (r < 0) return 1;
+  const bool in = gload(M.mark[0] + v) != 0 && (M.sym || gload(M.mark[1] + v) != 0);
+  const bool root = gload(M.subtree + v) < 0;
+  if ((!in && !root) || !cond_valid(M, r)) return 1;
+  return root ? 1 + cond_list_nodes(M, r) : 0;
+}
+
+// The vertices of R_c outside S(c) join the root's list of their direction and leave its weights.
+__global__ __launch_bounds__(256) void k_cond_append(const MatDev* __restrict__ mats, int nmats,
+                                                     const int64_t* __restrict__ row_base, int64_t nrows) {
+  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < nrows; g += (int64_t)gridDim.x * blockDim.x) {
+    const int mb = nmats == 1 ? 0 : find_segment(row_base, nmats, g);
+    const MatDev& M = mats[mb];
+    if (M.vroot == nullptr || M.sym) continue;  // mirrored: both directions reach the same
+    const int32_t v = (int32_t)(g - row_base[mb]);
+    const int32_t r = gload(M.vroot + v);
+    if (r < 0) continue;
+    const bool m0 = gload(M.mark[0] + v) != 0, m1 = gload(M.mark[1] + v) != 0;
+    if (m0 == m1 || gload(M.subtree + v) < 0 || !cond_valid(M, r)) continue;
+    const int d = m0 ? 0 : 1;
+    const int32_t pos = atomicAdd(M.root_cnt[d] + r, 1) - 1;
+    if (pos < M.list_cap) gstore(M.root_list[d] + (int64_t)r * M.list_cap + pos, v);
+    else atomicOr(&M.acc[kAccScheduleError], 1ull);  // cannot happen: |X_c| is at most the limit
+    if (d == 0) {
+      const int32_t deg = gload(M.rowptr[0] + v + 1) - gload(M.rowptr[0] + v) + (M.dup_all ? gload(M.dup_all + v) : 0);
+      atomicAdd(M.root_w + r, -deg);
+      atomicAdd(M.root_r + r, -1);
+    }
+  }
+}
+
+// Nodes per matrix (when a set is created: they size the condensed graph).
+__global__ __launch_bounds__(256) void k_cond_sizes(const MatDev* __restrict__ mats, int nmats,
+                                                    const int64_t* __restrict__ row_base, int64_t nrows,
+                                                    unsigned long long* __restrict__ sizes) {
+  for (int64_t g0 = (int64_t)blockIdx.x * blockDim.x; g0 < nrows; g0 += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t g = g0 + threadIdx.x;
+    const int mb = nmats == 1 ? 0 : find_segment(row_base, nmats, min(g, nrows - 1));
+    const int32_t c = g < nrows ? cond_nodes(mats[mb], (int32_t)(g - row_base[mb])) : 0;
+    const int mb0 = __builtin_amdgcn_readfirstlane(mb);
+    if (__ballot(mb != mb0) == 0) {
+      const uint32_t sum = wave_sum_u32((uint32_t)c);
+      if (lane_id() == 0 && sum) atomicAdd(&sizes[mb0], (unsigned long long)sum);
+    } else if (c) {
+      atomicAdd(&sizes[mb], (unsigned long long)c);
+    }
+  }
+}
+
+// Node numbers: an exclusive scan of cond_nodes over the set's rows (block sums, k_scan_blocks,
+// k_cond_apply).
+__global__ __launch_bounds__(kScanBlock) void k_cond_reduce(const MatDev* __restrict__ mats, int nmats,
+                                                            const int64_t* __restrict__ row_base, int64_t nrows,
+                                                            int32_t* __restrict__ block_sums) {
+  __shared__ int32_t s[kScanBlock / 64];
+  const int64_t base = (int64_t)blockIdx.x * kScanBlock * kScanItems;
+  int32_t acc = 0;
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    const int64_t i = base + (int64_t)k * kScanBlock + threadIdx.x;
+    if (i < nrows) {
+      const int mb = nmats == 1 ? 0 : find_segment(row_base, nmats, i);
+      acc += cond_nodes(mats[mb], (int32_t)(i - row_base[mb]));
+    }
+  }
+  const uint32_t w = wave_sum_u32((uint32_t)acc);
+  if (lane_id() == 0) s[threadIdx.x >> 6] = (int32_t)w;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int32_t t = 0;
+    for (int k = 0; k < kScanBlock / 64; ++k) t += s[k];
+    block_sums[blockIdx.x] = t;
+  }
+}
+
+__global__ __launch_bounds__(kScanBlock) void k_cond_apply(const MatDev* __restrict__ mats,
+                                                           const MatDev* __restrict__ cmats, int nmats,
+                                                           const int64_t* __restrict__ row_base, int64_t nrows,
+                                                           const int32_t* __restrict__ block_off,
+                                                           const int64_t* __restrict__ cbase) {
+  __shared__ int32_t s_wave[kScanItems][kScanBlock / 64];
+  const int64_t base = (int64_t)blockIdx.x * kScanBlock * kScanItems;
+  int32_t c[kScanItems], incl[kScanItems], mbs[kScanItems];
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    const int64_t i = base + (int64_t)k * kScanBlock + threadIdx.x;
+    mbs[k] = i < nrows ? (nmats == 1 ? 0 : find_segment(row_base, nmats, i)) : 0;
+    c[k] = i < nrows ? cond_nodes(mats[mbs[k]], (int32_t)(i - row_base[mbs[k]])) : 0;
+  }
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    incl[k] = (int32_t)wave_incl_scan_u32((uint32_t)c[k]);
+    if (lane_id() == 63) s_wave[k][threadIdx.x >> 6] = incl[k];
+  }
+  __syncthreads();
+  int32_t carry = block_off[blockIdx.x];
+#pragma unroll
+  for (int k = 0; k < kScanItems; ++k) {
+    int32_t off = 0, all = 0;
+    for (int w = 0; w < kScanBlock / 64; ++w) {
+      if (w < (int)(threadIdx.x >> 6)) off += s_wave[k][w];
+      all += s_wave[k][w];
+    }
+    const int64_t i = base + (int64_t)k * kScanBlock + threadIdx.x;
+    const int64_t first = (int64_t)carry + off + incl[k] - c[k];
+    carry += all;
+    if (i >= nrows) continue;
+    const MatDev& M = mats[mbs[k]];
+    if (M.vroot == nullptr) continue;
+    const int32_t v = (int32_t)(i - row_base[mbs[k]]);
+    // the nodes were counted when the set was created; a run that counts others reports an error
+    // (and stays inside the graph's buffers)
+    const int64_t lo = cbase[mbs[k]], hi = cbase[mbs[k] + 1];
+    if (first < lo || first + c[k] > hi || (v == M.n - 1 && first + c[k] != hi)) {
+      atomicOr(&M.acc[kAccScheduleError], 1ull);
+      gstore(M.nid + v, 0);
+      continue;
+    }
+    int32_t* const orig = const_cast<int32_t*>(cmats[mbs[k]].orig);
+    const int32_t id = (int32_t)(first - lo);
+    gstore(M.nid + v, c[k] ? id + c[k] - 1 : -1);
+    if (c[k]) gstore(orig + id + c[k] - 1, v);
+    if (gload(M.subtree + v) < 0) {
+      const int32_t r = gload(M.vroot + v);
+      gstore(M.root_id + r, id + c[k] - 1);
+      for (int32_t j = 0; j < c[k] - 1; ++j) gstore(orig + id + j, -(r + 1));
+    }
+  }
+}
+
+// The condensed graph's rows, 16 lanes per node and direction (blocks [0, 2 ell_blocks), direction
+// 1 after direction 0), and its workgroup-path items, one wave per block of chain_block nodes (the
+// blocks after them). Items go by descending block (cblk_base / cblk_mat: the condensed matrices,
+// largest first), both directions of a block together; a block without an escalated row keeps
+// kNoItem. A block is cut at the node whose subtree is at least 1.5 times its predecessor's and at
+// least rows / cut_divisor vertices (the largest such): its rows before the cut are items of their
+// own, after the others.
+__global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mats, const MatDev* __restrict__ cmats,
+                                                  int nmats, const int64_t* __restrict__ cbase, int64_t nodes,
+                                                  int64_t ell_blocks, const int64_t* __restrict__ cblk_base,
+                                                  const int32_t* __restrict__ cblk_mat, int ncond, int64_t nblk,
+                                                  int32_t cut_divisor, WorkState* __restrict__ ws,
+                                                  uint64_t* __restrict__ items) {
+  const int lane = lane_id();
+  if ((int64_t)blockIdx.x >= 2 * ell_blocks) {
+    const int64_t k = ((int64_t)blockIdx.x - 2 * ell_blocks) * 4 + (threadIdx.x >> 6);
+    if (k == 0 && lane == 0) ws->heavy_count = 2ull * (unsigned long long)nblk;
+    if (k >= nblk) return;
+    const int o = find_segment(cblk_base, ncond, k);
+    const int mb = cblk_mat[o];
+    const MatDev& M = mats[mb];
+    const MatDev& C = cmats[mb];
+    const int32_t K = C.chain_block;
+    const int32_t b = (int32_t)(cblk_base[o + 1] - 1 - k);
+    const int32_t r0 = b * K, r1 = (int32_t)min((int64_t)C.n, (int64_t)r0 + K);
+    uint64_t any0 = 0, any1 = 0;
+    int32_t best = 0, cut = -1;
+    for (int32_t j0 = r0; j0 < r1; j0 += 64) {
+      const int32_t j = j0 + lane;
+      const int32_t v = j < r1 ? gload(C.orig + j) : -1;
+      any0 |= __ballot(v >= 0 && gload(M.esc[0] + v) != 0);
+      any1 |= __ballot(v >= 0 && !M.sym && gload(M.esc[1] + v) != 0);
+      if (cut_divisor > 0) {
+        const int32_t u = j > r0 && j < r1 ? gload(C.orig + j - 1) : -1;
+        int32_t size = 0;
+        if (v >= 0 && u >= 0) {
+          const int32_t sv = gload(M.subtree + v) & INT32_MAX, su = gload(M.subtree + u) & INT32_MAX;
+          if (2 * (int64_t)sv >= 3 * (int64_t)su && sv >= M.rows / cut_divisor) size = sv;
+        }
+        int32_t most = size;
+        for (int x = 32; x > 0; x >>= 1) most = max(most, __shfl_xor(most, x, 64));
+        if (most > best) {
+          best = most;
+          cut = j0 + __ffsll((unsigned long long)__ballot(size == most)) - 1;
+        }
+      }
+    }
+    if (lane < 2) {
+      const bool any = lane == 0 ? any0 != 0 : any1 != 0;
+      items[2 * k + lane] = any ? encode_item((uint32_t)mb, (uint32_t)lane, (uint32_t)(cut >= 0 ? cut : r0), 0u) : kNoItem;
+      if (any && cut >= 0) {
+        const unsigned long long pos = atomicAdd(&ws->cut_count, 1ull);
+        items[2 * nblk + (int64_t)pos] = encode_item((uint32_t)mb, (uint32_t)lane, (uint32_t)cut, 1u);
+      }
+    }
+    return;
+  }
+  const int d = (int64_t)blockIdx.x < ell_blocks ? 0 : 1;
+  const int64_t g = (((int64_t)blockIdx.x - (d ? ell_blocks : 0)) * 256 + threadIdx.x) / kEll;
+  if (g >= nodes) return;  // a node's 16 lanes leave together
+  const int l = lane & (kEll - 1);
+  const int mb = nmats == 1 ? 0 : find_segment(cbase, nmats, g);
+  const MatDev& M = mats[mb];
+  const MatDev& C = cmats[mb];
+  if (d == 1 && M.sym) return;
+  const int32_t j = (int32_t)(g - cbase[mb]);
+  auto node_of = [&](int32_t m) -> int32_t {
+    const int32_t id = gload(M.nid + m);
+    return id >= 0 ? id : gload(M.root_id + gload(M.vroot + m));
+  };
+  const int32_t v = gload(C.orig + j);
+  int32_t e = kPad;
+  int32_t wt_deg = 0, wt_r = 0;
+  uint8_t esc = 0;
+  const int32_t r = v >= 0 ? gload(M.vroot + v) : -(v + 1);
+  const bool root = v >= 0 && r >= 0 && gload(M.subtree + v) < 0 && cond_valid(M, r);
+  if (v >= 0 && !root) {
+    e = gload(M.ell[d] + (int64_t)v * kEll + l);
+    const bool tail = l == kEll - 1 && e <= -2;
+    if (e >= 0) e = node_of(e);
+    if (tail) {
+      const int32_t pe = gload(M.rowptr[d] + v + 1);
+      for (int32_t p = -(e + 2); p < pe; ++p)
+        gstore(const_cast<int32_t*>(C.adj[d]) + p, node_of(gload(M.adj[d] + p)));
+      gstore(const_cast<int32_t*>(C.rowptr[d]) + j + 1, pe);
+    }
+    if (d == 0 && M.dup_all) wt_deg = gload(M.dup_all + v);
+    esc = gload(M.esc[d] + v);
+  } else {
+    // a contracted root, or one of its list nodes
+    const int32_t len = cond_list_len(M, d, r);
+    const int32_t leaves = cond_leaves(len), mids = cond_mids(leaves);
+    const int32_t first = gload(M.root_id + r) - cond_list_nodes(M, r);  // the root's first list node
+    const int32_t i = j - first;
+    int32_t at = -1, node = kPad;  // a list entry, or a list node
+    if (root) {
+      if (leaves == 0) at = l < len ? l : -1;
+      else if (mids == 0) node = l < leaves ? first + l : kPad;
+      else node = l < mids ? first + leaves + l : kPad;
+    } else if (i < leaves) {
+      at = i * kEll + l < len ? i * kEll + l : -1;
+    } else if (i < leaves + mids) {
+      const int32_t q = (i - leaves) * kEll + l;
+      node = q < leaves ? first + q : kPad;
+    }
+    e = at >= 0 ? node_of(gload(M.root_list[d] + (int64_t)r * M.list_cap + at)) : node;
+    // its entries are not input entries, and a list node is no vertex
+    const int32_t entries = __popcll((__ballot(e >= 0) >> (lane & 48)) & 0xFFFFull);
+    wt_deg = (root ? gload(M.root_w + r) : 0) - entries;
+    wt_r = root ? gload(M.root_r + r) - 1 : -1;
+  }
+  gstore(const_cast<int32_t*>(C.ell[d]) + (int64_t)j * kEll + l, e);
+  if (l == 0) {
+    gstore(C.esc[d] + j, esc);
+    if (d == 0) {
+      int32_t* const wt = const_cast<int32_t*>(C.wt) + 2 * (int64_t)j;
+      gstore(wt, wt_deg);
+      gstore(wt + 1, wt_r);
     }
   }
 }
@@ -1121,7 +1445,9 @@ struct LeaderState {
 };
 
 // kPairedAny: some matrix of the set runs paired items (otherwise that code is compiled out).
-template <int kThreads, bool kPairedAny, bool kHbmBitmap>
+// kCond: the matrices are condensed graphs (below k_cond_ell): rows are nodes, results go to the
+// nodes' vertices, and the items before a cut come first.
+template <int kThreads, bool kPairedAny, bool kHbmBitmap, bool kCond = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_heavy(const MatDev* __restrict__ mats,
                                                     WorkState* __restrict__ ws,
                                                     const uint64_t* __restrict__ heavy_items,
@@ -1130,6 +1456,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                                                     uint32_t* __restrict__ hbm_bitmaps, int32_t ucap,
                                                     int32_t exec_slot) {
   static_assert(kEll == 16, "the window scan maps one row to 16 lanes");
+  static_assert(!kCond || (!kPairedAny && !kHbmBitmap), "condensed graphs run plain items with LDS bitmaps");
   extern __shared__ uint32_t dyn[];
   constexpr int kPfRounds = ((kHeavyWin + 1) * kEll + kThreads - 1) / kThreads;
   constexpr int kStash = (kHeavyWin + 1) * kEll;  // ELL slots of a window's rows, per direction
@@ -1143,11 +1470,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   __shared__ int32_t s_esc[2][kHeavyWin + 1];   // row w0 + i was escalated (per direction)
   __shared__ int32_t s_hold[2][kHeavyWin + 1];  // row w0 + i holds w0 + i - 1
   __shared__ int64_t s_lp[2][kHeavyWin + 2];    // structure offsets of rows w0 .. w0 + np
+  __shared__ int32_t s_orig[kCond ? kHeavyWin + 1 : 1];  // condensed: the rows' vertices
+  __shared__ int32_t s_ulen[kCond ? kHeavyWin + 1 : 1];  // and the lengths of their structure lists
   __shared__ unsigned long long s_escm[2];      // rows w0 .. w0 + 63 escalated, as bits (per direction)
   __shared__ HeavyCtl s_ctl;
   __shared__ LeaderState s_ls;
   // The slots some lane of the wave sets (push loops skip the others). Sets with paired items
   // (unstructured rows, which fill most slots) keep every slot: measured faster there.
+  // What a vertex adds to the totals beyond its entries: the duplicate surplus of its input row, or a
+  // condensed node's weights (dupv to its entry count, rv vertices). Nothing for v < 0.
+  auto node_weight = [](const MatDev& M, int d, int32_t v, uint32_t& dupv, uint32_t& rv) {
+    if constexpr (kCond) {
+      if (v >= 0 && d == 0) {
+        const v2i32 t = gload(reinterpret_cast<const v2i32*>(M.wt) + v);
+        dupv = (uint32_t)t.x;
+        rv = 1u + (uint32_t)t.y;
+      }
+    } else {
+      if (v >= 0 && d == 0 && M.dup_all) dupv = (uint32_t)gload(M.dup_all + v);
+    }
+  };
   auto row_any = [](uint32_t mask) -> uint32_t {
     if constexpr (kPairedAny) return ~0u;
     else return wave_or_u32(mask);
@@ -1202,13 +1544,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   __shared__ Totals tot;  // thread 0 only (in LDS: keeps the registers for the traversal)
   if (tid == 0) tot = Totals{};
 
-  const unsigned long long total = ws->heavy_count;
+  const unsigned long long ncut = kCond ? ws->cut_count : 0ull;
+  const unsigned long long total = ws->heavy_count + ncut;
   while (true) {
     if (tid == 0) s_idx = atomicAdd(&ws->heavy_next, 1ull);
     bsync();
     const unsigned long long idx = s_idx;
     if (idx >= total) break;
-    const uint64_t item = heavy_items[idx];
+    // condensed: the items before a cut (after the others in the array) go first
+    const uint64_t item = heavy_items[kCond ? (idx < ncut ? total - ncut + idx : idx - ncut) : idx];
+    if (kCond && item == kNoItem) {
+      bsync();
+      continue;
+    }
     const int mb = (int)((item >> 33) & 0xfffffu);
     const int item_dir = (int)((item >> 32) & 1);
     const int32_t v = (int32_t)(item & 0xffffffffu);
@@ -1217,6 +1565,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const bool paired = kPairedAny && M.paired != 0;
     const int ndir = paired ? 2 : 1;
     const int32_t n = M.n;
+    const int32_t rows = kCond ? M.rows : n;  // rows of the matrix (chunks, window bits)
     const int32_t bw = (n + 31) >> 5;
     // rows [r0, r1): from v to the end of its block, or, before a cut, from the block's start to
     // v (decoded from the item alone: a table read here costs the traversal registers)
@@ -1256,7 +1605,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         int32_t esc_v = 0;
         int64_t lp_v = 0;
         if (tid < np) esc_v = gload(M.esc[dd] + w0 + tid);
-        if (want_list && tid <= np) lp_v = gload(M.list_ptr[dd] + w0 + tid);
+        if constexpr (kCond) {
+          if (tid < np) {
+            const int32_t o = gload(M.orig + w0 + tid);
+            s_orig[tid] = o;
+            if (want_list && o >= 0) {
+              lp_v = gload(M.list_ptr[dd] + o);
+              s_ulen[tid] = (int32_t)(gload(M.list_ptr[dd] + o + 1) - lp_v);
+            }
+          }
+        } else {
+          if (want_list && tid <= np) lp_v = gload(M.list_ptr[dd] + w0 + tid);
+        }
         int32_t ev[kPfRounds];
 #pragma unroll
         for (int q = 0; q < kPfRounds; ++q) {
@@ -1298,11 +1658,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           if (i < np * kEll && li2 >= 1 && s_esc[dd][li2] != 0 && s_esc[dd][li2 - 1] != 0 && s_hold[dd][li2] == 0) {
             const int32_t u = stash[i];
             if (u >= 0 && u < row - 1) {
-              const int32_t* const ur = M.ell[dd] + (int64_t)u * kEll;
+              // condensed: u in row - 1 of the other direction (a root's entries are in list nodes);
+              // 16 lanes read the same line, where the entries' own rows are 16 lines
+              const int32_t* const ur = kCond ? M.ell[M.sym ? dd : 1 - dd] + (int64_t)(row - 1) * kEll
+                                              : M.ell[dd] + (int64_t)u * kEll;
+              const int32_t want = kCond ? u : row - 1;
 #pragma unroll
               for (int q4 = 0; q4 < 4; ++q4) {
                 const v4i32 t4 = gload_v4(ur + 4 * q4);
-                hit = hit || t4.x == row - 1 || t4.y == row - 1 || t4.z == row - 1 || t4.w == row - 1;
+                hit = hit || t4.x == want || t4.y == want || t4.z == want || t4.w == want;
               }
             }
           }
@@ -1361,7 +1725,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 break;
               }
               src = w0 + li;
-              chunk_end = min(n, (src / M.chunk + 1) * M.chunk);
+              {
+                const int32_t o = kCond ? s_orig[li] : src;
+                chunk_end = min(rows, (o / M.chunk + 1) * M.chunk);
+              }
               const int32_t prev_d = s_ls.prev[d];
               // t1: the last row traversed here in this direction, even with wave-path rows in
               // between (plain items: s-1 only)
@@ -1562,7 +1929,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   if (v >= 0) m = seed ? stash[li * kEll + sl] : gload(M.ell[d] + (int64_t)v * kEll + sl);
                   const bool chk = v >= 0 && !seed && has_prev;
                   const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
-                  uint32_t dupv = (v >= 0 && sl == 0 && d == 0 && M.dup_all) ? (uint32_t)gload(M.dup_all + v) : 0u;
+                  uint32_t dupv = 0, rv = 1;
+                  node_weight(M, d, sl == 0 ? v : -1, dupv, rv);
                   const bool in_prev = chk && ((pword >> (v & 31)) & 1u) != 0;
                   if (in_prev && imported) {  // covered by the imported X_{s-1}
                     v = -1;
@@ -1585,8 +1953,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     w_all += valid + dupv;
                     if (in_prev) w_ovl += valid + dupv;
                     if (v >= 0 && sl == 0) {
-                      r_all += 1;
-                      if (in_prev) r_ovl += 1;
+                      r_all += rv;
+                      if (in_prev) r_ovl += rv;
                     }
                   }
                   x_e += valid;
@@ -1620,7 +1988,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
                   RowCursor rc;
                   load_row(M, d, v, rc);
-                  uint32_t dupv = (v >= 0 && d == 0 && M.dup_all) ? (uint32_t)gload(M.dup_all + v) : 0u;
+                  uint32_t dupv = 0, rv = 1;
+                  node_weight(M, d, v, dupv, rv);
                   const bool in_prev = chk && ((pword >> (v & 31)) & 1u) != 0;
                   if (in_prev && imported) {
                     v = -1;
@@ -1685,10 +2054,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   if (v >= 0) {
                     deg += dupv;
                     w_all += deg;
-                    r_all += 1;
+                    r_all += rv;
                     if (in_prev) {
                       w_ovl += deg;
-                      r_ovl += 1;
+                      r_ovl += rv;
                     }
                   }
                 }
@@ -1743,7 +2112,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               if (want_list) {
                 const uint32_t len = ubase + s_ust;
                 const int64_t off = s_lp[d][li];
-                const bool lp_ok = s_lp[d][li + 1] - off == (int64_t)U;
+                const bool lp_ok = kCond ? s_ulen[li] == (int32_t)U : s_lp[d][li + 1] - off == (int64_t)U;
                 int32_t* const dst = M.pool[d] + off;
                 // 256 entries per round, all read before any is written: an entry moves to a
                 // position at or below its own, so a round never overwrites what it still reads
@@ -1773,7 +2142,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     const uint64_t mk = __ballot(keep);
                     const uint32_t pos = kept + rank_below(mk);
                     if (keep) {
-                      if (lp_ok && pos < U) gstore(dst + pos, e[q]);
+                      if (lp_ok && pos < U) gstore(dst + pos, kCond ? gload(M.orig + e[q]) : e[q]);
                       if (in_lds) ul[pos] = e[q];  // pos <= i0 + 255 < ucap
                       else uput(pos, e[q]);
                     }
@@ -1792,6 +2161,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               const bool save = paired ? next_in
                                        : !M.sym && next_in && s_esc[d][li + 1] != 0 && s_hold[d][li + 1] == 0;
               const int wslot = s_ls.wp[d];  // the ring slot this row's save takes
+              const int32_t vsrc = kCond ? s_orig[li] : src;
+              if (kCond && (d == 1 || M.sym)) {
+                // window bits of a node: its next 128 nodes hold every vertex vsrc + 1 .. vsrc + 128
+                // of the graph; a set bit stands for its node's vertex
+                uint32_t win[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                  const int32_t j = src + 1 + 64 * q + lane;
+                  if (j < n && ((bm_get(j >> 5) >> (j & 31)) & 1u) != 0) window_bit(win, vsrc, gload(M.orig + j), chunk_end);
+                }
+                const uint32_t w0 = wave_or_u32(win[0]), w1 = wave_or_u32(win[1]);
+                const uint32_t w2 = wave_or_u32(win[2]), w3 = wave_or_u32(win[3]);
+                if (lane == 0) reinterpret_cast<uint4*>(M.win)[vsrc] = make_uint4(w0, w1, w2, w3);
+              }
               if (lane == 0) {
                 const RowFacts f{wr, dg0, rr, U, want_list ? kept : 0u};
                 s_facts[d][kSavedRing] = f;
@@ -1800,7 +2183,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   flush_totals(mats, last_mat, tot, exec_slot);
                   last_mat = mb;
                 }
-                gstore(M.cnt[d] + src, (int32_t)U);
+                gstore(M.cnt[d] + vsrc, (int32_t)U);
                 tot.fill += U - a_us;
                 tot.heavy += 1;
                 tot.x_edges += a_x;
@@ -1813,7 +2196,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 } else {
                   tot.nnz_l += U;
                 }
-                if (d == 1 || M.sym) {
+                if (!kCond && (d == 1 || M.sym)) {
                   // window bits straight from the bitmap: rows src+1 .. src+128 of this column's
                   // chunk (a mirrored matrix: L's column src is U's row src)
                   uint32_t win[4];
@@ -2027,7 +2410,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
                 RowCursor rc;
                 load_row(CM, cd, v, rc);
-                const uint32_t dupv = (v >= 0 && cd == 0 && CM.dup_all) ? (uint32_t)gload(CM.dup_all + v) : 0u;
+                uint32_t dupv = 0, rv = 1;
+                node_weight(CM, cd, v, dupv, rv);
                 const bool in_prev = chk && ((pword >> (v & 31)) & 1u) != 0;
                 if (in_prev && cimported) {  // covered by the imported X_{s-1}
                   v = -1;
@@ -2138,10 +2522,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 if (v >= 0) {
                   deg += dupv;
                   p_w += deg;
-                  p_r += 1;
+                  p_r += rv;
                   if (in_prev) {
                     p_wo += deg;
-                    p_ro += 1;
+                    p_ro += rv;
                   }
                 }
               }
@@ -2314,9 +2698,9 @@ hipError_t launch_fill_u64(unsigned long long* p, int64_t count, unsigned long l
 
 hipError_t launch_clear_run(unsigned long long* acc, int64_t nacc, unsigned long long* ws, int64_t nws, int32_t* esc,
                             int64_t nesc, int32_t* blk_flag, int64_t nblk, int32_t* bucket, int64_t nbucket,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(k_clear_run, dim3(grid_for(nacc + nws + nesc + nblk + nbucket, 256, 8192)), dim3(256), 0, s, acc,
-                     nacc, ws, nws, esc, nesc, blk_flag, nblk, bucket, nbucket);
+                            int32_t* cond, int64_t ncond, hipStream_t s) {
+  hipLaunchKernelGGL(k_clear_run, dim3(grid_for(nacc + nws + nesc + nblk + nbucket + ncond, 256, 8192)), dim3(256), 0,
+                     s, acc, nacc, ws, nws, esc, nesc, blk_flag, nblk, bucket, nbucket, cond, ncond);
   return hipGetLastError();
 }
 
@@ -2349,13 +2733,12 @@ hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, c
 }
 
 hipError_t launch_light(const MatDev* mats, int nmats, const int64_t* item_base, int64_t nitems, WorkState* ws, int grid,
-                        int bits, hipStream_t s) {
-  if (bits == kLightBitsBig)
-    hipLaunchKernelGGL(k_light<kLightBitsBig>, dim3(grid), dim3(kLightWaves * 64), 0, s, mats, nmats, item_base, nitems,
-                       ws);
-  else
-    hipLaunchKernelGGL(k_light<kLightBits>, dim3(grid), dim3(kLightWaves * 64), 0, s, mats, nmats, item_base, nitems, ws);
-  return hipGetLastError();
+                        int bits, bool roots, hipStream_t s) {
+  const void* f = bits == kLightBitsBig
+                      ? (roots ? (const void*)k_light<kLightBitsBig, true> : (const void*)k_light<kLightBitsBig, false>)
+                      : (roots ? (const void*)k_light<kLightBits, true> : (const void*)k_light<kLightBits, false>);
+  void* args[] = {&mats, &nmats, &item_base, &nitems, &ws};
+  return hipLaunchKernel(f, dim3(grid), dim3(kLightWaves * 64), args, 0, s);
 }
 
 hipError_t launch_heavy_order(const MatDev* mats, int64_t nblk_total, int nmats, const int64_t* blkq_base,
@@ -2405,6 +2788,16 @@ const void* heavy_fn(int threads) {
   }
 }
 
+// Condensed graphs: plain items, bitmaps in LDS.
+const void* heavy_cond_fn(int threads) {
+  switch (threads) {
+    case 1024: return (const void*)k_heavy<1024, false, false, true>;
+    case 512: return (const void*)k_heavy<512, false, false, true>;
+    case 256: return (const void*)k_heavy<256, false, false, true>;
+    default: return nullptr;
+  }
+}
+
 const void* heavy_fn(int threads, bool paired, bool hbm) {
   if (paired) return hbm ? heavy_fn<true, true>(threads) : heavy_fn<true, false>(threads);
   return hbm ? heavy_fn<false, true>(threads) : heavy_fn<false, false>(threads);
@@ -2429,6 +2822,51 @@ hipError_t launch_heavy(int threads, int grid, const MatDev* mats, WorkState* ws
   void* args[] = {&mats, &ws, &heavy_items, &bw_max, &qcap, &n_max, &spill, &hbm_bitmaps, &ucap, &exec_slot};
   return hipLaunchKernel(f, dim3(grid), dim3(threads), args,
                          heavy_lds_bytes(bw_max, qcap, hbm, ucap, paired_any != 0), s);
+}
+
+hipError_t launch_heavy_cond(int threads, int grid, const MatDev* cmats, WorkState* ws, const uint64_t* items,
+                             int32_t bw_max, int32_t qcap, int64_t n_max, int32_t* spill, int32_t ucap, hipStream_t s) {
+  const void* f = heavy_cond_fn(threads);
+  if (!f) return hipErrorInvalidValue;
+  uint32_t* none = nullptr;
+  int32_t exec_slot = kAccHeavyExecEdges;
+  void* args[] = {&cmats, &ws, &items, &bw_max, &qcap, &n_max, &spill, &none, &ucap, &exec_slot};
+  return hipLaunchKernel(f, dim3(grid), dim3(threads), args, heavy_lds_bytes(bw_max, qcap, false, ucap, false), s);
+}
+
+int heavy_cond_occupancy(int threads, size_t bytes) {
+  const void* f = heavy_cond_fn(threads);
+  int nb = 0;
+  if (!f || hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, f, threads, bytes) != hipSuccess)
+    return 0;
+  return nb;
+}
+
+hipError_t launch_cond_sizes(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows,
+                             unsigned long long* sizes, hipStream_t s) {
+  const int g = grid_for(nrows, 256, 16384);
+  hipLaunchKernelGGL(k_cond_append, dim3(g), dim3(256), 0, s, mats, nmats, row_base, nrows);
+  hipLaunchKernelGGL(k_cond_sizes, dim3(g), dim3(256), 0, s, mats, nmats, row_base, nrows, sizes);
+  return hipGetLastError();
+}
+
+hipError_t launch_condense(const MatDev* mats, const MatDev* cmats, int nmats, const int64_t* row_base, int64_t nrows,
+                           const int64_t* cbase, int64_t nodes, const int64_t* cblk_base, const int32_t* cblk_mat,
+                           int ncond, int64_t nblk, int32_t cut_divisor, int32_t* block_sums, int32_t* total,
+                           WorkState* ws, uint64_t* items, hipStream_t s) {
+  const int64_t per = (int64_t)kScanBlock * kScanItems;
+  const int64_t nb = (nrows + per - 1) / per;
+  hipLaunchKernelGGL(k_cond_append, dim3(grid_for(nrows, 256, 16384)), dim3(256), 0, s, mats, nmats, row_base, nrows);
+  hipLaunchKernelGGL(k_cond_reduce, dim3((unsigned)nb), dim3(kScanBlock), 0, s, mats, nmats, row_base, nrows, block_sums);
+  hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScanBlock), 0, s, block_sums, nb, total);
+  hipLaunchKernelGGL(k_cond_apply, dim3((unsigned)nb), dim3(kScanBlock), 0, s, mats, cmats, nmats, row_base, nrows,
+                     block_sums, cbase);
+  const int64_t ell_blocks = (nodes * kEll + 255) / 256;
+  const int64_t item_blocks = (nblk + 3) / 4;
+  hipLaunchKernelGGL(k_cond_ell, dim3((unsigned)(2 * ell_blocks + item_blocks)), dim3(256), 0, s, mats, cmats, nmats,
+                     cbase, nodes, ell_blocks, cblk_base, cblk_mat, ncond, nblk, cut_divisor, ws, items);
+  return hipGetLastError();
 }
 
 hipError_t launch_supernodes(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s) {
@@ -2467,8 +2905,8 @@ int heavy_occupancy(int threads, size_t lds_bytes, bool hbm_bitmap) {
 int light_occupancy(int bits) {
   int nb = 0;
   const hipError_t e = bits == kLightBitsBig
-                           ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBitsBig>, kLightWaves * 64, 0)
-                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBits>, kLightWaves * 64, 0);
+                           ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBitsBig, true>, kLightWaves * 64, 0)
+                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBits, true>, kLightWaves * 64, 0);
   return e == hipSuccess ? nb : 0;
 }
 }  // namespace gsofa

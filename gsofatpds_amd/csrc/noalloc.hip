@@ -288,6 +288,7 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   M.light_end = n;
   M.subtree = nullptr;  // no pre-escalation: the subtree sizes need the host's elimination tree
   M.pre_size = INT32_MAX;
+  M.rows = n;
   M.light_limit = n <= kLightSmallRows ? kLightLimitSmall
                   : cfg.light_bits == kLightBitsBig ? kLightLimitBig : kLightLimitMax;
   const int64_t bases[8] = {0, nitems, 0, n, 0, nblocks_sup, 0, nblk};
@@ -335,6 +336,7 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   q.esc = L.esc;
   q.blk_flag = L.blk_flag;
   q.hbm_bm = nullptr;
+  q.nplain = 1;
   q.mats = L.mats;
   q.item_base = item_base;
   q.row_base = row_base;
