@@ -444,7 +444,7 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
     if (e_ != hipSuccess) return hf(e_, what);  \
   } while (0)
   if (ev) GSOFA_SEQ(hipEventRecord(ev[0], s), "hipEventRecord");
-  GSOFA_SEQ(launch_clear_run(q.acc, (int64_t)q.nmats * kAccSlots, reinterpret_cast<unsigned long long*>(q.ws),
+  GSOFA_SEQ(launch_clear_run(q.acc, (int64_t)q.nmats * kAccSlots * acc_copies(q.nmats), reinterpret_cast<unsigned long long*>(q.ws),
                              q.ncond > 0 ? 8 : 4, reinterpret_cast<int32_t*>(q.esc), q.esc_words,
                              reinterpret_cast<int32_t*>(q.blk_flag), 2 * q.nblk_total, q.bucket, q.nb_max,
                              q.cond_zero, q.cond_words, s),
@@ -487,6 +487,7 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
   if (q.n_top > 0) GSOFA_SEQ(hipStreamWaitEvent(s, q.join, 0), "hipStreamWaitEvent(join)");
   if (q.mirror_any) GSOFA_SEQ(launch_mirror(q.mats, q.nmats, q.blk_base, q.nblocks_sup, s), "k_mirror");
   GSOFA_SEQ(launch_supernodes(q.mats, q.nmats, q.blk_base, q.nblocks_sup, s), "k_supernodes");
+  if (q.sum_totals) GSOFA_SEQ(launch_totals(q.mats, q.nmats, s), "k_totals");
   if (ev) GSOFA_SEQ(hipEventRecord(ev[4], s), "hipEventRecord");
 #undef GSOFA_SEQ
   return GSOFA_OK;
@@ -630,7 +631,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   GSOFA_TRY(alloc(cnt_l_, nrows_, "L counts"));
   GSOFA_TRY(alloc(win_, nrows_ * 4, "window bits"));
   GSOFA_TRY(alloc(sup_flag_, nrows_, "supernode flags"));
-  GSOFA_TRY(alloc(acc_, (size_t)nmats_ * kAccSlots, "accumulators"));
+  GSOFA_TRY(alloc(acc_, (size_t)nmats_ * kAccSlots * acc_copies(nmats_), "accumulators"));
   GSOFA_TRY(alloc(mats_d_, nmats_, "matrix table"));
   GSOFA_TRY(alloc(item_base_d_, nmats_ + 1, "item base"));
   GSOFA_TRY(alloc(row_base_d_, nmats_ + 1, "row base"));
@@ -784,6 +785,8 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     M.pool[0] = M.pool[1] = nullptr;
     M.sup_flag = sup_flag_ + rb;
     M.acc = acc_ + (size_t)b * kAccSlots;
+    M.acc_stride = (int64_t)nmats_ * kAccSlots;
+    M.acc_mask = acc_copies(nmats_) - 1;
     M.esc[0] = esc_ + rb;
     M.esc[1] = esc_ + nrows_ + rb;
     M.blk_flag[0] = blk_flag_ + blkq_base_h_[b];
@@ -848,7 +851,7 @@ int DeviceSet::create_condensed(const DeviceInfo& info) {
   unsigned long long* sizes_d = nullptr;
   GSOFA_TRY(alloc(sizes_d, (size_t)nmats_, "condensed sizes"));
   Sequence q = sequence();
-  GSOFA_HIP(launch_clear_run(q.acc, (int64_t)nmats_ * kAccSlots, reinterpret_cast<unsigned long long*>(ws_), 8,
+  GSOFA_HIP(launch_clear_run(q.acc, (int64_t)nmats_ * kAccSlots * acc_copies(nmats_), reinterpret_cast<unsigned long long*>(ws_), 8,
                              reinterpret_cast<int32_t*>(esc_), esc_words_, reinterpret_cast<int32_t*>(blk_flag_),
                              2 * nblk_total_, bucket_, nb_max_, cond_zero_, cond_words_, s),
             "clear the run's state");
@@ -989,7 +992,7 @@ int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Opt
     b += 14 * nrows + 8 * nrows / kCondMinRoot * kLightLimitBig + 8 * nnz + (int64_t)(0.7 * 150.0 * (double)nrows) +
          4 * heavy_grid * heavy_region_ints(nmax, false);
   if (opt.structure) b += 16 * (nrows + (int64_t)mats.size());  // offsets; pools are sized later
-  b += 1 << 20;                       // tables, accumulators, scan scratch
+  b += (1 << 20) + (int64_t)mats.size() * kAccSlots * 8 * acc_copies((int)mats.size());  // tables, accumulators, scan scratch
   *out_bytes = b;
   return GSOFA_OK;
 }

@@ -143,6 +143,7 @@ struct Sequence {
   int32_t nb_max = 0, n_max = 0;
   int32_t paired_any = 0;
   int32_t prepare = 1;         // 0: the ELL rows and A^T are already built (enqueue_preparation)
+  int32_t sum_totals = 1;      // end with k_totals
   int32_t mirror_any = 0;      // some matrix is mirrored (k_mirror runs)
   int32_t mirror_all = 0;      // every matrix is mirrored (A^T is not built)
   LaunchConfig cfg;

@@ -43,8 +43,18 @@ enum : int {
   kAccTopExecEdges = 20,
   kAccTopExecVerts = 21,
   kAccTopExecOut = 22,
-  kAccSlots = 24
+  kAccSlots = 32     // a copy is whole cache lines
 };
+// Totals are added to one of several copies of a matrix's accumulators, chosen by workgroup: atomic
+// adds to one address take 13 ns each, one after the other, whatever the rest of the device does
+// (k_supernodes: one add per 256 rows, 35 us at 659,033 rows). k_totals sums them into copy 0.
+constexpr int kAccCopies = 64;  // at most a wave (k_noalloc_totals)
+// A power of two: as many as keep a set's copies at 4,096.
+inline int acc_copies(int nmats) {
+  int c = kAccCopies;
+  while (c > 1 && (int64_t)c * nmats > 4096) c /= 2;
+  return c;
+}
 
 // One matrix as the kernels see it. Direction 0 traverses A (rows, gives U), direction 1
 // traverses A^T (columns of A, gives L by columns).
@@ -61,7 +71,9 @@ struct MatDev {
   const int64_t* list_ptr[2];     // n + 1: row/column offsets into pool (null: no structure)
   int32_t* pool[2];               // strict U rows (dir 0) / strict L columns (dir 1)
   uint8_t* sup_flag;              // n: 1 where the supernode count increments
-  unsigned long long* acc;        // kAccSlots
+  unsigned long long* acc;        // kAccSlots: copy 0
+  int64_t acc_stride;             // slots from one copy to the next
+  int32_t acc_mask;               // copies - 1
   uint8_t* esc[2];                // n: 1 where the wave path escalated the source
   uint32_t* blk_flag[2];          // ceil(n / chain_block): 1 where the block has an escalated row
   const int32_t* split;           // ceil(n / chain_block): a row where the block is cut into two
@@ -199,8 +211,10 @@ constexpr size_t kHeavyCondLdsReserve = 4096;  // its static LDS plus margin
 // Before the early launch: every matrix's rows [light_end, n) escalated (both directions), and
 // ws->heavy_count = count, ws->heavy_next = 0 (one block per matrix).
 hipError_t launch_top_setup(const MatDev* mats, int nmats, WorkState* ws, int64_t count, hipStream_t s);
-// Mirrored matrices: L counts = U counts, fill and workgroup-path entries doubled, nnz_L = nnz_U
-// (one thread per row, blocks as for launch_supernodes).
+// After the last kernel that counts: every matrix's copies summed into copy 0 (one block per matrix);
+// a mirrored matrix's fill and workgroup-path entries doubled, nnz_L = nnz_U.
+hipError_t launch_totals(const MatDev* mats, int nmats, hipStream_t s);
+// Mirrored matrices: L counts = U counts (one thread per row, blocks as for launch_supernodes).
 hipError_t launch_mirror(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 hipError_t launch_supernodes(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 constexpr int kLightThreads = 256;

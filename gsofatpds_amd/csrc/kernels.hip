@@ -312,6 +312,39 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_apply(const int32_t* __rest
 }
 
 // ------------------------------------------------------------------------------------------
+// totals
+// ------------------------------------------------------------------------------------------
+// The copy of a matrix's accumulators that this workgroup adds to.
+__device__ __forceinline__ unsigned long long* acc_of(const MatDev& M) {
+  return M.acc + (int64_t)((int32_t)blockIdx.x & M.acc_mask) * M.acc_stride;
+}
+
+// Sums a matrix's copies into copy 0, and completes a mirrored matrix's: it was traversed from A
+// only, and L's column s holds what U's row s holds.
+__global__ __launch_bounds__(256) void k_totals(const MatDev* __restrict__ mats) {
+  static_assert(kAccSlots == 32, "eight copies per round");
+  __shared__ unsigned long long s_sum[8][kAccSlots];
+  const MatDev& M = mats[blockIdx.x];
+  const int slot = threadIdx.x & (kAccSlots - 1), part = threadIdx.x / kAccSlots;
+  unsigned long long x = 0;
+  for (int k = part; k <= M.acc_mask; k += 8) x += M.acc[k * M.acc_stride + slot];
+  s_sum[part][slot] = x;
+  __syncthreads();
+  if (part == 0) {
+    for (int k = 1; k < 8; ++k) x += s_sum[k][slot];
+    s_sum[0][slot] = x;
+  }
+  __syncthreads();
+  if (part == 0) {
+    if (M.sym) {
+      if (slot == kAccFill || slot == kAccHeavyNnz) x *= 2;
+      if (slot == kAccNnzL) x = s_sum[0][kAccNnzU];
+    }
+    M.acc[slot] = x;
+  }
+}
+
+// ------------------------------------------------------------------------------------------
 // traversal: shared pieces
 // ------------------------------------------------------------------------------------------
 struct RowCursor {
@@ -496,7 +529,7 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
   auto flush = [&](int mb) {
     if (mb < 0) return;
     if (lane == 0) {
-      unsigned long long* acc = mats[mb].acc;
+      unsigned long long* acc = acc_of(mats[mb]);
       if (t_fill) atomicAdd(&acc[kAccFill], t_fill);
       if (t_w) atomicAdd(&acc[kAccW], t_w);
       if (t_r) atomicAdd(&acc[kAccR], t_r);
@@ -1366,7 +1399,7 @@ struct Totals {  // cleared with Totals{}
 
 __device__ __forceinline__ void flush_totals(const MatDev* mats, int mb, Totals& t, int32_t exec_slot) {
   if (mb < 0) return;
-  unsigned long long* acc = mats[mb].acc;
+  unsigned long long* acc = acc_of(mats[mb]);
   if (t.fill) atomicAdd(&acc[kAccFill], t.fill);
   if (t.w) atomicAdd(&acc[kAccW], t.w);
   if (t.r) atomicAdd(&acc[kAccR], t.r);
@@ -2632,13 +2665,12 @@ __global__ __launch_bounds__(256) void k_supernodes(const MatDev* __restrict__ m
   const uint64_t c = wave_sum_u64(flag);
   if (lane_id() == 0 && c) atomicAdd(&s_sum, (uint32_t)c);
   __syncthreads();
-  if (threadIdx.x == 0 && s_sum) atomicAdd(&M.acc[kAccNsup], (unsigned long long)s_sum);
+  if (threadIdx.x == 0 && s_sum) atomicAdd(&acc_of(M)[kAccNsup], (unsigned long long)s_sum);
 }
 
 // k_mirror: a mirrored matrix was traversed from A only. From source s, A^T reaches exactly what
 // A reaches (the pattern is its own transpose), so L's column s holds U's row s: its count is
-// copied, the fill and the workgroup path's entries (both triangles) double, nnz_L = nnz_U.
-// Runs after both traversal kernels, before k_supernodes.
+// copied (the totals: k_totals). Runs after both traversal kernels, before k_supernodes.
 __global__ __launch_bounds__(256) void k_mirror(const MatDev* __restrict__ mats, int nmats,
                                                 const int64_t* __restrict__ blk_base) {
   const int mb = find_segment(blk_base, nmats, (int64_t)blockIdx.x);
@@ -2646,12 +2678,6 @@ __global__ __launch_bounds__(256) void k_mirror(const MatDev* __restrict__ mats,
   if (!M.sym) return;
   const int64_t r = ((int64_t)blockIdx.x - blk_base[mb]) * 256 + threadIdx.x;
   if (r < M.n) M.cnt[1][r] = M.cnt[0][r];
-  if ((int64_t)blockIdx.x == blk_base[mb] && threadIdx.x == 0) {
-    unsigned long long* acc = M.acc;
-    acc[kAccFill] *= 2;
-    acc[kAccNnzL] = acc[kAccNnzU];
-    acc[kAccHeavyNnz] *= 2;
-  }
 }
 
 // Before the early launch of the top separators' items: their rows escalated in both directions
@@ -2683,6 +2709,11 @@ static int grid_for(int64_t work, int block, int cap) {
 hipError_t launch_mirror(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s) {
   if (nblocks <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_mirror, dim3((unsigned)nblocks), dim3(256), 0, s, mats, nmats, blk_base);
+  return hipGetLastError();
+}
+
+hipError_t launch_totals(const MatDev* mats, int nmats, hipStream_t s) {
+  hipLaunchKernelGGL(k_totals, dim3((unsigned)nmats), dim3(256), 0, s, mats);
   return hipGetLastError();
 }
 

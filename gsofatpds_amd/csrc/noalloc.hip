@@ -99,7 +99,7 @@ void carve_layout(unsigned char* base, int32_t n, int64_t nnz, int64_t nblk, int
   L.total = c.take<int32_t>(1);
   L.cnt_l = c.take<int32_t>(n);
   L.win = c.take<uint32_t>((int64_t)n * 4);
-  L.acc = c.take<unsigned long long>(kAccSlots);
+  L.acc = c.take<unsigned long long>(kAccSlots * acc_copies(1));
   L.mats = c.take<MatDev>(1);
   L.bases = c.take<int64_t>(8);
   L.ws = c.take<WorkState>(1);
@@ -160,19 +160,30 @@ __global__ void k_noalloc_tables(Tables t, MatDev* __restrict__ mats, int64_t* _
 }
 
 // Totals in the order gsofa_run_noalloc documents: fill, nnz_F, nnz_L, nnz_U, W, |R|, reported
-// supernodes, counted supernodes, input error.
-__global__ void k_noalloc_totals(const unsigned long long* __restrict__ acc, const uint32_t* __restrict__ bad,
-                                 int32_t n, int32_t n_processes, uint64_t* __restrict__ totals) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    totals[0] = acc[kAccFill];
-    totals[1] = acc[kAccNnzL] + acc[kAccNnzU] + (uint64_t)n;
-    totals[2] = acc[kAccNnzL];
-    totals[3] = acc[kAccNnzU];
-    totals[4] = acc[kAccW];
-    totals[5] = acc[kAccR];
-    totals[6] = acc[kAccNsup] + (uint64_t)(int64_t)n_processes;
-    totals[7] = acc[kAccNsup];
-    totals[8] = *bad;
+// supernodes, counted supernodes, input error. One wave; lane k sums over the accumulators' copy k.
+__global__ __launch_bounds__(64) void k_noalloc_totals(const unsigned long long* __restrict__ acc, int copies,
+                                                       const uint32_t* __restrict__ bad, int32_t n,
+                                                       int32_t n_processes, uint64_t* __restrict__ totals) {
+  const int slots[6] = {kAccFill, kAccNnzL, kAccNnzU, kAccW, kAccR, kAccNsup};
+  unsigned long long x[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) x[k] = (int)threadIdx.x < copies ? acc[threadIdx.x * kAccSlots + slots[k]] : 0ull;
+  const uint32_t error = *bad;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)  // six independent sums per step
+#pragma unroll
+    for (int k = 0; k < 6; ++k) x[k] += __shfl_xor(x[k], o, 64);
+  const uint64_t fill = x[0], l = x[1], u = x[2], w = x[3], r = x[4], sup = x[5];
+  if (threadIdx.x == 0) {
+    totals[0] = fill;
+    totals[1] = l + u + (uint64_t)n;
+    totals[2] = l;
+    totals[3] = u;
+    totals[4] = w;
+    totals[5] = r;
+    totals[6] = sup + (uint64_t)(int64_t)n_processes;
+    totals[7] = sup;
+    totals[8] = error;
   }
 }
 
@@ -278,6 +289,8 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   M.pool[0] = M.pool[1] = nullptr;
   M.sup_flag = sup_flags;
   M.acc = L.acc;
+  M.acc_stride = kAccSlots;
+  M.acc_mask = acc_copies(1) - 1;
   M.esc[0] = L.esc;
   M.esc[1] = L.esc + n;
   M.blk_flag[0] = L.blk_flag;
@@ -337,6 +350,7 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   q.blk_flag = L.blk_flag;
   q.hbm_bm = nullptr;
   q.nplain = 1;
+  q.sum_totals = 0;  // k_noalloc_totals does
   q.mats = L.mats;
   q.item_base = item_base;
   q.row_base = row_base;
@@ -344,7 +358,7 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   q.blkq_base = blkq_base;
   rc = enqueue_sequence(q, s, nullptr);
   if (rc != GSOFA_OK) return rc;
-  hipLaunchKernelGGL(k_noalloc_totals, dim3(1), dim3(64), 0, s, L.acc, L.bad, n, o.n_processes, totals);
+  hipLaunchKernelGGL(k_noalloc_totals, dim3(1), dim3(64), 0, s, L.acc, acc_copies(1), L.bad, n, o.n_processes, totals);
   NA_HIP(hipGetLastError(), "k_noalloc_totals");
   return GSOFA_OK;
 }
