@@ -135,58 +135,52 @@ static double symmetric_share(const Prepared& P) {
   return seen ? (double)matched / (double)seen : 1.0;
 }
 
-int32_t condensation_roots(const Prepared& P, int32_t limit, std::vector<int32_t>& vroot, std::vector<uint8_t>& is_root) {
+bool front_units(const Prepared& P, std::vector<std::vector<std::pair<int32_t, int32_t>>>& levels) {
   const int32_t n = P.n;
   const std::vector<int32_t>&size = P.subtree, &parent = P.parent;
-  // Sampled vertices: their root under each share of the limit, and how much of a contracted vertex
-  // is left in the graph (its root's node and list nodes). In nested-dissection order a subtree is
-  // the rows before its root; elsewhere the list lengths below are estimates only (a root that does
-  // not fit escalates, and its subtree then stays uncontracted).
-  constexpr int kSamples = 64;
-  double best = 0.0;
-  int32_t best_t = 0;
-  std::vector<int32_t> up;
-  for (const double share : {0.9, 0.75, 0.6, 0.45, 0.35, 0.25}) {
-    const int32_t t = (int32_t)(share * limit);
-    if (t < kCondMinRoot) break;
-    double gone = 0.0, kept = 0.0;
-    int32_t last = -1;
-    for (int k = 0; k < kSamples; ++k) {
-      int32_t c = (int32_t)((int64_t)n * (2 * k + 1) / (2 * kSamples));
-      if (size[c] > t) continue;
-      while (parent[c] >= 0 && size[parent[c]] <= t) c = parent[c];
-      if (size[c] < kCondMinRoot) continue;
-      if (c != last) {
-        last = c;
-        up.clear();
-        for (int32_t v = std::max(0, c - size[c] + 1); v <= c; ++v)
-          for (int32_t p = P.rowptr[v + 1]; p > P.rowptr[v] && P.adj[p - 1] > c; --p) up.push_back(P.adj[p - 1]);
-        std::sort(up.begin(), up.end());
-        const double u = (double)(std::unique(up.begin(), up.end()) - up.begin());
-        // the directed lists of an unsymmetric pattern miss some of the surface
-        kept = size[c] + 1.1 * u <= limit ? 1.0 - (1.0 + u / kEll) / size[c] : 0.0;
+  levels.clear();
+  std::vector<int32_t> first((size_t)n), nodes((size_t)n);
+  for (int32_t v = 0; v < n; ++v) first[v] = v;
+  for (int32_t v = 0; v < n; ++v)
+    if (parent[v] >= 0) first[parent[v]] = std::min(first[parent[v]], first[v]);
+  // nodes[v]: the nodes T(v) has when the units so far are contracted
+  for (int32_t v = 0; v < n; ++v) nodes[v] = size[v];
+  int64_t left = n, open = n, units = 0, rows = 0;  // nodes, unfinished rows
+  std::vector<uint8_t> gone((size_t)n, 0);  // v is a unit's root
+  for (int l = 0; l < kFrontLevels; ++l) {
+    if (open < kFrontOpen[l]) break;
+    const int32_t cap = l == 0 ? kFrontMax[0].nodes : kFrontMax[l].nodes - kFrontMax[l].nodes / 7;
+    std::vector<std::pair<int32_t, int32_t>> u;
+    for (int32_t v = 0; v < n; ++v)
+      if (nodes[v] <= cap && nodes[v] >= kFrontMin && !gone[v] && (parent[v] < 0 || nodes[parent[v]] > cap) &&
+          first[v] == v - size[v] + 1)
+        u.push_back({first[v], v});
+    if (u.empty()) break;
+    for (const auto& x : u) {
+      gone[x.second] = 1;
+      left -= nodes[x.second] - 1;
+      if (l == 0) rows += size[x.second];
+    }
+    // rows of the level's units that no unit below holds
+    std::vector<int32_t> held((size_t)u.size(), 0);
+    if (l > 0) {
+      size_t k = 0;
+      for (const auto& x : levels[l - 1]) {  // both in ascending order, nested or disjoint
+        while (k < u.size() && u[k].second < x.first) ++k;
+        if (k < u.size() && u[k].first <= x.first && x.second <= u[k].second) held[k] += size[x.second];
       }
-      gone += kept;
     }
-    if (gone > best) {
-      best = gone;
-      best_t = t;
-    }
-  }
-  if (best < (1.0 - kCondMaxShare) * kSamples) return 0;
-  vroot.assign((size_t)n, -1);
-  is_root.assign((size_t)n, 0);
-  int32_t roots = 0;
-  for (int32_t v = n - 1; v >= 0; --v) {
-    if (size[v] > best_t) continue;
-    if (parent[v] >= 0 && size[parent[v]] <= best_t) {
-      vroot[v] = vroot[parent[v]];
-    } else if (size[v] >= kCondMinRoot) {
-      vroot[v] = roots++;
-      is_root[v] = 1;
+    for (size_t k = 0; k < u.size(); ++k) open -= size[u[k].second] - held[k];
+    if (l == 0) units = (int64_t)u.size();
+    levels.push_back(std::move(u));
+    if (l == 0 && (units == 0 || rows < kFrontMean * units)) return false;
+    std::fill(nodes.begin(), nodes.end(), 1);
+    for (int32_t v = 0; v < n; ++v) {
+      if (gone[v]) nodes[v] = 1;
+      if (parent[v] >= 0) nodes[parent[v]] += nodes[v];
     }
   }
-  return roots;
+  return !levels.empty() && (double)left <= kCondMaxShare * n;
 }
 
 int32_t light_limit_for(int32_t n, int light_bits) {
@@ -371,17 +365,25 @@ int configure_launch(int32_t n_max, int64_t nrows, bool paired_any, const Option
   return GSOFA_OK;
 }
 
-int configure_condensed(int32_t cn_max, int64_t nodes, const Options& opt, const DeviceInfo& info, LaunchConfig& out) {
+int configure_condensed(int32_t cn_max, int64_t open, const Options& opt, const DeviceInfo& info, LaunchConfig& out) {
   out = LaunchConfig();
   out.bw_max = (cn_max + 31) / 32;
   const size_t reserve = kHeavyCondLdsReserve + heavy_stash_bytes(false);
   const size_t bitmap_bytes = (size_t)out.bw_max * 4;
   auto lds_fits = [&](int wgs) { return (size_t)wgs * (bitmap_bytes + reserve + 512 * 8) <= info.lds_per_cu; };
-  // Four workgroups of 256 threads per compute unit while their bitmaps fit: measured (best block
-  // sizes) 128 / 256 / 512 threads: 57 k nodes 1466 / 865 / 919 us, 131 k 3237 / 1851 / 1922, 47 k (3-D)
-  // 2393 / 1266 / 1204, 5.6 k 233 / 181 / 162.
+  // Workgroup shape and nodes per item, by the rows that the graphs leave in one direction. An
+  // item's first row pays for a traversal of what lies below the item, so long items traverse less;
+  // short ones, and larger workgroups, end the few items of a small graph sooner. Measured, us of
+  // k_heavy for both directions (rows: 256 threads at 4 / 8 / 16 / 32 nodes; 512 threads at the same):
+  //   376: 50 / 61 / 83 / 129; 44 / 55 / 77 / 122        3,073: 130 / 140 / 157 / 206; 146 / 124 / 145 / 191
+  //   4,693 (3-D): 213 / 217 / 242 / 379; 267 / 204 / 199 / 325
+  //   17,738: 645 / 424 / 383 / 401; 993 / 624 / 447 / 383
+  //   17,983 (3-D): 869 / 576 / 510 / 653; 1222 / 787 / 606 / 563
+  //   36,525: 1654 / 992 / 713 / 696; 2470 / 1484 / 996 / 771
+  // and mirrored: 1,888: 94 / 102 / 122 / 168; 81 / 90 / 112 / 161, 6,620: 167 / 178 / 273 / 323;
+  // 199 / 159 / 233 / 289.
   int threads = opt.heavy_threads;
-  if (!threads) threads = lds_fits(4) ? 256 : lds_fits(2) ? 512 : 1024;
+  if (!threads) threads = open < 10000 && lds_fits(2) ? 512 : lds_fits(4) ? 256 : lds_fits(2) ? 512 : 1024;
   if (threads != 256 && threads != 512 && threads != 1024)
     return fail(GSOFA_ERR_INVALID_ARG, "heavy_threads must be 256, 512 or 1024");
   out.heavy_threads = threads;
@@ -407,12 +409,7 @@ int configure_condensed(int32_t cn_max, int64_t nodes, const Options& opt, const
   const int cus = opt.cu_share > 0 ? std::min(opt.cu_share, info.cus) : info.cus;
   out.heavy_grid = cus * occ;
   out.heavy_wgs_per_cu = occ;
-  // Nodes per item. A node's traversal starts from its block's earlier ones, so the first of a block
-  // pays for the block; with little left below it that costs less than an idle compute unit. Measured
-  // (256 threads, us of k_heavy at 8 / 16 / 32 / 64 nodes): 2.3 k nodes 164 / 168 / 218 / -, 5.6 k 187 /
-  // 181 / 225 / 318, 47 k (3-D) 1619 / 1266 / 1681 / 2176, 57 k - / 906 / 874 / 944, 131 k - / 2158 /
-  // 1851 / 1854 (24 and 48 nodes lie between their neighbours or above them).
-  out.chain_block = opt.chain_block ? opt.chain_block : nodes < 4096 ? 8 : nodes < 50000 ? 16 : 32;
+  out.chain_block = opt.chain_block ? opt.chain_block : open < 1250 ? 4 : open < 10000 ? 8 : 16;
   return GSOFA_OK;
 }
 
@@ -429,6 +426,14 @@ int enqueue_preparation(const Sequence& q, hipStream_t s) {
     if (e != hipSuccess) return hf(e, "transpose");
     e = launch_ell_build(q.nrows, q.nmats, q.row_base, q.rowptr_t, q.adj_t, q.ell_t, s);
     if (e != hipSuccess) return hf(e, "ell A^T");
+  }
+  return GSOFA_OK;
+}
+
+int enqueue_fronts(const Sequence& q, hipStream_t s, FrontSize* most) {
+  for (int l = 0; l < kFrontLevels; ++l) {
+    const hipError_t e = launch_front(l, q.fronts[l], q.mats, q.units, most ? most + l : nullptr, s);
+    if (e != hipSuccess) return fail(GSOFA_ERR_HIP, std::string("k_front: ") + hipGetErrorString(e));
   }
   return GSOFA_OK;
 }
@@ -463,8 +468,9 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
     if (q.top_ev) GSOFA_SEQ(hipEventRecord(q.top_ev[1], q.side), "hipEventRecord");
     GSOFA_SEQ(hipEventRecord(q.join, q.side), "hipEventRecord(join)");
   }
-  GSOFA_SEQ(launch_light(q.mats, q.nmats, q.item_base, q.nitems, q.ws, q.cfg.light_grid, q.cfg.light_bits, q.ncond > 0, s),
-            "k_light");
+  if (q.nplain > 0)
+    GSOFA_SEQ(launch_light(q.mats, q.nmats, q.item_base, q.nitems, q.ws, q.cfg.light_grid, q.cfg.light_bits, s), "k_light");
+  if (q.ncond > 0) GSOFA_TRY(enqueue_fronts(q, s));
   // cursor, block_sums and total are free again once the transpose is built
   if (q.ncond > 0)
     GSOFA_SEQ(launch_condense(q.mats, q.cmats, q.nmats, q.row_base, q.nrows, q.cbase, q.cnodes, q.cblk_base, q.cblk_mat,
@@ -665,8 +671,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   // reaches almost nothing below its rows, whatever the subtree) and paired matrices
   // (unstructured: reaches far smaller than their subtrees) keep every attempt. Only matrices
   // with more rows than the limit carry the subtree sizes.
-  std::vector<int32_t> pre_size((size_t)nmats_, INT32_MAX), nroots((size_t)nmats_, 0);
-  int32_t list_cap = 0;
+  std::vector<int32_t> pre_size((size_t)nmats_, INT32_MAX);
   bool any_pre = false;
   if (opt.pre_escalate != -1) {
     for (int b = 0; b < nmats_; ++b) {
@@ -680,50 +685,15 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   }
   if (any_pre) {
     GSOFA_TRY(alloc(subtree_d_, (size_t)nrows_, "subtree sizes"));
-    std::vector<int32_t> sub((size_t)nrows_, 0), vroot_all, vroot;
-    std::vector<uint8_t> is_root;
+    std::vector<int32_t> sub((size_t)nrows_, 0);
     for (int b = 0; b < nmats_; ++b) {
       if (pre_size[b] == INT32_MAX) continue;
       const Prepared& P = *mats[b];
       if (P.subtree.empty()) elimination_tree(P);
       std::copy(P.subtree.begin(), P.subtree.end(), sub.begin() + row_base_h_[b]);
-      // the workgroup path on the condensed graph, except where the early launch's fixed items or
-      // HBM bitmaps were asked for
-      if (opt.early_top > 0 || opt.bitmap_in_hbm == 1) continue;
-      nroots[b] = condensation_roots(P, pre_size[b], vroot, is_root);
-      if (nroots[b] == 0) continue;
-      if (vroot_all.empty()) vroot_all.assign((size_t)nrows_, -1);
-      std::copy(vroot.begin(), vroot.end(), vroot_all.begin() + row_base_h_[b]);
-      for (int32_t v = 0; v < P.n; ++v)
-        if (is_root[v]) sub[row_base_h_[b] + v] |= INT32_MIN;
-      list_cap = std::max(list_cap, pre_size[b]);
     }
     GSOFA_TRY(upload(subtree_d_, sub.data(), sub.size() * 4, "upload subtree sizes"));
-    if (!vroot_all.empty()) {
-      GSOFA_TRY(alloc(vroot_, (size_t)nrows_, "condensation roots"));
-      GSOFA_TRY(upload(vroot_, vroot_all.data(), vroot_all.size() * 4, "upload condensation roots"));
-    }
     if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(subtree sizes)");
-  }
-  int64_t roots_all = 0;
-  std::vector<int64_t> root_base((size_t)nmats_ + 1, 0);
-  for (int b = 0; b < nmats_; ++b) root_base[b + 1] = root_base[b] + nroots[b];
-  roots_all = root_base[nmats_];
-  cond_.assign((size_t)nmats_, 0);
-  uint8_t* marks = nullptr;
-  int32_t *root_cnt = nullptr, *root_bad = nullptr;
-  if (roots_all > 0) {
-    // cleared by every run: the marks of both directions (bytes), then per root its two counts and
-    // whether its subtree holds an escalated row
-    const int64_t mark_words = (2 * nrows_ + 3) / 4;
-    cond_words_ = mark_words + 3 * roots_all;
-    GSOFA_TRY(alloc(cond_zero_, (size_t)cond_words_, "condensation marks"));
-    marks = reinterpret_cast<uint8_t*>(cond_zero_);
-    root_cnt = cond_zero_ + mark_words;
-    root_bad = root_cnt + 2 * roots_all;
-    GSOFA_TRY(alloc(root_list_, (size_t)(2 * roots_all * list_cap), "condensation lists"));
-    GSOFA_TRY(alloc(root_wri_, (size_t)(3 * roots_all), "condensation root weights"));
-    GSOFA_TRY(alloc(nid_, (size_t)nrows_, "condensation nodes"));
   }
   if (any_dup) {
     GSOFA_TRY(alloc(dup_u_, nrows_, "duplicate surplus (upper)"));
@@ -801,28 +771,18 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     M.subtree = pre_size[b] != INT32_MAX ? subtree_d_ + rb : nullptr;
     M.pre_size = pre_size[b];
     M.rows = ns_[b];
-    if (nroots[b] > 0) {
-      cond_[b] = 1;
-      const int64_t r0 = root_base[b];
-      M.vroot = vroot_ + rb;
-      M.nid = nid_ + rb;
-      for (int d = 0; d < 2; ++d) {
-        M.mark[d] = marks + d * nrows_ + rb;
-        M.root_cnt[d] = root_cnt + d * roots_all + r0;
-        M.root_list[d] = root_list_ + (d * roots_all + r0) * list_cap;
-      }
-      M.root_bad = root_bad + r0;
-      M.root_w = root_wri_ + r0;
-      M.root_r = root_wri_ + roots_all + r0;
-      M.root_id = root_wri_ + 2 * roots_all + r0;
-      M.list_cap = list_cap;
-    }
   }
   GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
   // The pattern is fixed for the set's lifetime, and so are its device forms (ELL rows, A^T): built
   // here once, like the upload, not on every run.
   GSOFA_TRY(enqueue_preparation(sequence(), alloc_stream_));
-  if (roots_all > 0) GSOFA_TRY(create_condensed(info));
+  // by fronts: the matrices with subtree sizes, except where the early launch's fixed items or HBM
+  // bitmaps were asked for
+  if (any_pre && opt.early_top <= 0 && opt.bitmap_in_hbm != 1) {
+    std::vector<uint8_t> tree((size_t)nmats_, 0);
+    for (int b = 0; b < nmats_; ++b) tree[b] = pre_size[b] != INT32_MAX;
+    GSOFA_TRY(create_fronts(mats, tree, info));
+  }
   GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(preparation)");
   nplain_ = nmats_ - ncond_;
   if (nplain_ > 0) {
@@ -843,44 +803,99 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   return GSOFA_OK;
 }
 
-// The condensed graphs' buffers. Their sizes are counted by one wave path over the set (nothing
-// else of that run is kept; every run builds its graphs anew, and reports an error should it count
-// other sizes).
-int DeviceSet::create_condensed(const DeviceInfo& info) {
+// The fronts' units and the condensed graphs' buffers. The graphs' sizes are counted by one run of the
+// fronts (nothing else of it is kept; every run builds its graphs anew, and reports an error should
+// it count other sizes).
+int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree,
+                             const DeviceInfo& info) {
   hipStream_t s = alloc_stream_;
+  cond_.assign((size_t)nmats_, 0);
+  std::vector<FrontUnit> units[kFrontLevels];
+  std::vector<std::vector<std::pair<int32_t, int32_t>>> levels;
+  bool any = false;
+  for (int b = 0; b < nmats_; ++b) {
+    if (!tree[b] || ns_[b] >= kStRoot || !front_units(*mats[b], levels)) continue;
+    cond_[b] = 1;
+    any = true;
+    for (size_t l = 0; l < levels.size(); ++l)
+      for (const auto& x : levels[l]) units[l].push_back({b, x.second, x.first, kFrontMax[l].nodes + kFrontMax[l].ext, 0});
+  }
+  if (!any) return GSOFA_OK;
+  const int cus = opt_in_.cu_share > 0 ? std::min(opt_in_.cu_share, info.cus) : info.cus;
+  std::vector<FrontUnit> all;
+  int64_t list_len = 0;
+  for (int l = 0; l < kFrontLevels; ++l) {
+    FrontLaunch& L = fronts_[l];
+    L.size = kFrontMax[l];
+    const int occ = front_occupancy(l, L.size);
+    if (occ <= 0) return fail(GSOFA_ERR_HIP, "k_front cannot be resident");
+    L.grid = cus * occ;
+    L.u0 = (int32_t)all.size();
+    for (FrontUnit& u : units[l]) {
+      u.off = list_len;
+      list_len += 2 * (int64_t)u.cap;
+      all.push_back(u);
+    }
+    L.u1 = (int32_t)all.size();
+  }
+  const int64_t nu = (int64_t)all.size();
+  if (nu >= kStUnit) return fail(GSOFA_ERR_CAPACITY, "too many front units");
+  int32_t *ulist = nullptr, *ulen = nullptr, *uwt = nullptr, *uid = nullptr;
+  uint32_t* umsg = nullptr;
+  cond_words_ = nrows_ + nu;  // the vertices' states, the units' counters
+  GSOFA_TRY(alloc(cond_zero_, (size_t)cond_words_, "vertex states"));
+  GSOFA_TRY(alloc(umsg, (size_t)(2 * kFrontMsg * nu), "front messages"));
+  GSOFA_TRY(alloc(nid_, (size_t)nrows_, "condensation nodes"));
+  GSOFA_TRY(alloc(units_, (size_t)nu, "front units"));
+  GSOFA_TRY(alloc(ulist, (size_t)list_len, "front lists"));
+  GSOFA_TRY(alloc(ulen, (size_t)(2 * nu), "front list lengths"));
+  GSOFA_TRY(alloc(uwt, (size_t)(2 * nu), "front weights"));
+  GSOFA_TRY(alloc(uid, (size_t)nu, "front nodes"));
+  GSOFA_TRY(upload(units_, all.data(), all.size() * sizeof(FrontUnit), "upload front units"));
+  if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(front units)");
+  for (int b = 0; b < nmats_; ++b) {
+    if (!cond_[b]) continue;
+    MatDev& M = mats_h_[b];
+    M.st = cond_zero_ + row_base_h_[b];
+    M.nid = nid_ + row_base_h_[b];
+    M.units = units_;
+    M.ulist = ulist;
+    M.ulen = ulen;
+    M.uwt = uwt;
+    M.uid = uid;
+    M.umsg = umsg;
+    M.uctr = reinterpret_cast<uint32_t*>(cond_zero_ + nrows_);
+  }
+  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  // per matrix its nodes and its unfinished rows, then per level the largest units (FrontSize)
   unsigned long long* sizes_d = nullptr;
-  GSOFA_TRY(alloc(sizes_d, (size_t)nmats_, "condensed sizes"));
+  GSOFA_TRY(alloc(sizes_d, (size_t)(2 * nmats_ + 2 * kFrontLevels), "condensed sizes"));
   Sequence q = sequence();
   GSOFA_HIP(launch_clear_run(q.acc, (int64_t)nmats_ * kAccSlots * acc_copies(nmats_), reinterpret_cast<unsigned long long*>(ws_), 8,
-                             reinterpret_cast<int32_t*>(esc_), esc_words_, reinterpret_cast<int32_t*>(blk_flag_),
-                             2 * nblk_total_, bucket_, nb_max_, cond_zero_, cond_words_, s),
+                             reinterpret_cast<int32_t*>(esc_), 0, reinterpret_cast<int32_t*>(blk_flag_), 0, bucket_, 0,
+                             cond_zero_, cond_words_, s),
             "clear the run's state");
-  GSOFA_HIP(launch_fill_u64(sizes_d, nmats_, 0, s), "clear condensed sizes");
-  GSOFA_HIP(launch_light(q.mats, nmats_, q.item_base, nitems_, ws_, cfg_.light_grid, cfg_.light_bits, true, s),
-            "k_light");
+  GSOFA_HIP(launch_fill_u64(sizes_d, 2 * nmats_ + 2 * kFrontLevels, 0, s), "clear condensed sizes");
+  GSOFA_TRY(enqueue_fronts(q, s, reinterpret_cast<FrontSize*>(sizes_d + 2 * nmats_)));
   GSOFA_HIP(launch_cond_sizes(q.mats, nmats_, q.row_base, nrows_, sizes_d, s), "condensed sizes");
-  std::vector<unsigned long long> sizes((size_t)nmats_, 0);
+  std::vector<unsigned long long> sizes((size_t)(2 * nmats_ + 2 * kFrontLevels), 0);
   GSOFA_TRY(download(sizes.data(), sizes_d, sizes.size() * 8, "read condensed sizes"));
-  // a matrix whose graph keeps too many vertices (roots that did not fit the wave path) runs as it is
-  auto drop = [&](int b) -> int {
+  // a matrix whose graph keeps too many vertices (units that did not fit) runs without fronts
+  auto drop = [&](int b) {
     cond_[b] = 0;
-    std::vector<int32_t> sub((size_t)ns_[b]);
-    MatDev& M = mats_h_[b];
-    GSOFA_TRY(download(sub.data(), M.subtree, sub.size() * 4, "read subtree sizes"));
-    for (int32_t& x : sub) x &= INT32_MAX;
-    GSOFA_TRY(upload(const_cast<int32_t*>(M.subtree), sub.data(), sub.size() * 4, "upload subtree sizes"));
-    if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(subtree sizes)");
-    M.vroot = nullptr;
-    return GSOFA_OK;
+    mats_h_[b].st = nullptr;
   };
   for (int b = 0; b < nmats_; ++b)
-    if (cond_[b] && (double)sizes[b] > (kCondMaxShare + 0.1) * ns_[b]) GSOFA_TRY(drop(b));
+    if (cond_[b] && (double)sizes[b] > (kCondMaxShare + 0.1) * ns_[b]) drop(b);
+  int64_t open = 0;
   auto total = [&] {
     cn_max_ = 0;
     cnodes_ = 0;
     ncond_ = 0;
+    open = 0;
     for (int b = 0; b < nmats_; ++b)
       if (cond_[b]) {
+        open += (int64_t)sizes[nmats_ + b];
         cn_max_ = std::max(cn_max_, (int32_t)sizes[b]);
         cnodes_ += (int64_t)sizes[b];
         ++ncond_;
@@ -888,14 +903,41 @@ int DeviceSet::create_condensed(const DeviceInfo& info) {
   };
   total();
   if (ncond_ > 0) {
-    const int rc = configure_condensed(cn_max_, cnodes_, opt_in_, info, ccfg_);
+    const int rc = configure_condensed(cn_max_, open, opt_in_, info, ccfg_);
     if (rc == GSOFA_ERR_CAPACITY) {
       for (int b = 0; b < nmats_; ++b)
-        if (cond_[b]) GSOFA_TRY(drop(b));
+        if (cond_[b]) drop(b);
       total();
     } else if (rc != GSOFA_OK) {
       return rc;
     }
+  }
+  // the units of the matrices that keep their fronts, and the wave path's items of the others
+  {
+    std::vector<FrontUnit> kept;
+    for (int l = 0; l < kFrontLevels; ++l) {
+      FrontLaunch& L = fronts_[l];
+      const int32_t base = (int32_t)kept.size();
+      for (int32_t u = L.u0; u < L.u1; ++u)
+        if (cond_[all[u].mat]) kept.push_back(all[u]);
+      L.u0 = base;
+      L.u1 = (int32_t)kept.size();
+      if (l == 0) continue;
+      // the level's LDS holds what its units need: more of them are resident
+      std::memcpy(&L.size, &sizes[2 * nmats_ + 2 * l], sizeof(FrontSize));
+      if (L.size.nodes == 0) L.u1 = L.u0;  // it took none
+      const int occ = front_occupancy(l, L.size);
+      if (occ <= 0) return fail(GSOFA_ERR_HIP, "k_front cannot be resident");
+      L.grid = cus * occ;
+    }
+    if (!kept.empty()) GSOFA_TRY(upload(units_, kept.data(), kept.size() * sizeof(FrontUnit), "upload front units"));
+    for (int b = 0; b < nmats_; ++b) {
+      const int64_t nb = cond_[b] ? 0 : ((int64_t)light_end_[b] + light_block_ - 1) / light_block_;
+      item_base_h_[b + 1] = item_base_h_[b] + (mirror_[b] ? nb + (nb & 1) : 2 * nb);
+    }
+    nitems_ = item_base_h_[nmats_];
+    GSOFA_TRY(upload(item_base_d_, item_base_h_.data(), item_base_h_.size() * 8, "upload"));
+    if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(front units)");
   }
   if (ncond_ > 0) {
     const int32_t K = ccfg_.chain_block;
@@ -986,11 +1028,11 @@ int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Opt
   b += 4 * (heavy_grid + kTopMaxItems) * heavy_region_ints(nmax, paired);  // spill (and the early launch's)
   if (place_bitmaps_in_hbm(nmax, opt, info)) b += 4 * (int64_t)cus * (((int64_t)nmax + 31) / 32);  // one per CU
   if (dup) b += 8 * nrows;
-  // subtree sizes, and the condensed graphs (roots, nodes, marks; lists of at most kLightLimitBig per
-  // kCondMinRoot rows and direction; nodes of at most kCondMaxShare + 0.1 of the rows)
+  // subtree sizes; fronts (states, nodes, units of at least kFrontMean rows on average with their lists)
+  // and the condensed graphs (at most kCondMaxShare + 0.1 of the rows)
   if (opt.pre_escalate != -1)
-    b += 14 * nrows + 8 * nrows / kCondMinRoot * kLightLimitBig + 8 * nnz + (int64_t)(0.7 * 150.0 * (double)nrows) +
-         4 * heavy_grid * heavy_region_ints(nmax, false);
+    b += 12 * nrows + (nrows / kFrontMean + 1) * (int64_t)(sizeof(FrontUnit) + 24 + 8 * kFrontMsg + 8 * (kFrontMax[0].nodes + kFrontMax[0].ext) * 2) +
+         8 * nnz + (int64_t)(0.7 * 150.0 * (double)nrows) + 4 * heavy_grid * heavy_region_ints(nmax, false);
   if (opt.structure) b += 16 * (nrows + (int64_t)mats.size());  // offsets; pools are sized later
   b += (1 << 20) + (int64_t)mats.size() * kAccSlots * 8 * acc_copies((int)mats.size());  // tables, accumulators, scan scratch
   *out_bytes = b;
@@ -1064,6 +1106,8 @@ Sequence DeviceSet::sequence() const {
   q.cn_max = cn_max_;
   q.cut_divisor = cut_divisor_;
   q.cond_zero = cond_zero_;
+  q.units = units_;
+  for (int l = 0; l < kFrontLevels; ++l) q.fronts[l] = fronts_[l];
   q.citems = citems_;
   q.ws_cond = ws_ + 1;
   q.cspill = cspill_;

@@ -50,15 +50,21 @@ int32_t top_separator_rows(const Prepared& P, const std::vector<int32_t>& cut);
 constexpr double kPreSymmetry = 0.75;
 // The wave path's escalation limit for a matrix of n rows under a hash-set variant.
 int32_t light_limit_for(int32_t n, int light_bits);
-// The roots of a matrix's condensed graph (kernels.hip): the rows of at least kCondMinRoot vertices
-// whose elimination subtree has at most T vertices while their parent's has more. T is the share of
-// the wave path's limit that lets the most vertices be contracted: a root's reached set and its U
-// list must both fit the limit (surfaces are larger in 3-D than in 2-D), estimated on sampled
-// vertices. vroot[v] becomes the index of the root whose subtree holds v, or -1, and is_root[v] 1 for
-// the roots. Returns the number of roots, or 0 where the graph would keep more than kCondMaxShare of
-// the vertices (little to gain: natural-order bands, whose subtrees are long chains).
-int32_t condensation_roots(const Prepared& P, int32_t limit, std::vector<int32_t>& vroot, std::vector<uint8_t>& is_root);
-constexpr int32_t kCondMinRoot = 32;
+// The front units of a matrix (kernels.hip, k_front): levels[l] receives the (lo, c) row ranges of the
+// elimination subtrees that level l's kernel takes. A level takes the largest subtrees whose rows,
+// with one node for every unit of the levels below, come to at most kFrontMax[l].nodes (above level 0
+// somewhat fewer: vertices that a contraction leaves out are nodes too, which only a run can tell),
+// and at least kFrontMin. Only subtrees that are row ranges (a postorder, as nested dissection
+// gives) are units. Returns whether it pays: at most kCondMaxShare of the vertices left as nodes,
+// units of at least kFrontMean rows on average (natural-order bands, whose subtrees are long chains,
+// and stars have few or tiny ones).
+bool front_units(const Prepared& P, std::vector<std::vector<std::pair<int32_t, int32_t>>>& levels);
+constexpr int32_t kFrontMin = 8, kFrontMean = 24;
+// A level runs when the levels below it leave this many rows: its launch takes the time of one of its
+// units, whatever their number. Measured, us with and without level 2 (fronts and k_heavy): 3,073 rows
+// left 261 / 245, 4,693 (3-D) 370 / 343, 6,620 (mirrored) 334 / 266, 30,413 (3-D) 899 / 1143, 49,371
+// 752 / 1166; with and without level 1: 1,981 rows left 176 / 184.
+constexpr int64_t kFrontOpen[kFrontLevels] = {0, 1500, 7000};
 constexpr double kCondMaxShare = 0.6;
 
 // At most this many items go to the early launch (one workgroup each), and this many per
@@ -126,9 +132,10 @@ struct LaunchConfig {
   bool hbm_bitmap = false;
   size_t heavy_lds = 0;  // dynamic LDS bytes of k_heavy
 };
-// The same for the workgroup path on condensed graphs (`nodes` in all, at most cn_max in one).
+// The same for the workgroup path on condensed graphs of at most cn_max nodes, with `open` unfinished
+// rows in all (in direction 0).
 // GSOFA_ERR_CAPACITY: they do not fit (the matrices then run uncondensed).
-int configure_condensed(int32_t cn_max, int64_t nodes, const Options& opt, const DeviceInfo& info, LaunchConfig& out);
+int configure_condensed(int32_t cn_max, int64_t open, const Options& opt, const DeviceInfo& info, LaunchConfig& out);
 // Picks the configuration for a set whose largest matrix has n_max rows (nrows in all) and sets
 // k_heavy's LDS limit. max_heavy_grid > 0 caps the bitmap-path workgroups (each holds a spill
 // region of heavy_region_ints(n_max) ints), for callers whose regions live in a fixed buffer.
@@ -157,15 +164,18 @@ struct Sequence {
   uint32_t *blk_flag = nullptr, *hbm_bm = nullptr;
   MatDev* mats = nullptr;
   int64_t *item_base = nullptr, *row_base = nullptr, *blk_base = nullptr, *blkq_base = nullptr;
-  // The condensed graphs (ncond > 0 matrices, built after the wave path by launch_condense) and their
-  // workgroup-path launch; nplain: matrices that run uncondensed (none: no such launch).
+  // The matrices with fronts (ncond of them): their units' launches, the condensed graphs these leave
+  // (launch_condense) and the workgroup path on them. nplain: the others, which the wave path and the
+  // plain workgroup path run (none: no such launches).
   int ncond = 0, nplain = 0;
   MatDev* cmats = nullptr;
   int64_t *cbase = nullptr, *cblk_base = nullptr;
   int32_t* cblk_mat = nullptr;
   int64_t cnodes = 0, cnblk = 0, cond_words = 0;
   int32_t cn_max = 0, cut_divisor = 0;
-  int32_t* cond_zero = nullptr;  // marks and lists, cleared by every run
+  int32_t* cond_zero = nullptr;  // the vertices' states, cleared by every run
+  const FrontUnit* units = nullptr;
+  FrontLaunch fronts[kFrontLevels];
   uint64_t* citems = nullptr;
   WorkState* ws_cond = nullptr;
   int32_t* cspill = nullptr;
@@ -188,6 +198,8 @@ struct Sequence {
 // path and the workgroup-path queue, after the main workgroup-path launch, after the join,
 // k_mirror and supernodes.
 int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev);
+// The fronts of the matrices that have them, level by level (after the states' clears).
+int enqueue_fronts(const Sequence& q, hipStream_t s, FrontSize* most = nullptr);
 // The input's device forms: ELL rows of A, and A^T with its ELL rows unless every matrix is
 // mirrored. Part of enqueue_sequence when q.prepare is set.
 int enqueue_preparation(const Sequence& q, hipStream_t s);
@@ -285,17 +297,19 @@ class DeviceSet {
   std::vector<int64_t> pool_base_u_, pool_base_l_;        // per matrix, into the pools
   std::vector<std::vector<int64_t>> u_ptr_h_, l_ptr_h_;    // host copies of the offsets
   std::vector<MatDev> mats_h_;
-  // the condensed graphs (Sequence)
-  int create_condensed(const DeviceInfo& info);
+  // fronts and condensed graphs (Sequence)
+  int create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree, const DeviceInfo& info);
   int ncond_ = 0, nplain_ = 0;
-  std::vector<uint8_t> cond_;         // per matrix: its workgroup path runs on the condensed graph
+  std::vector<uint8_t> cond_;         // per matrix: it runs by fronts and a condensed graph
   std::vector<MatDev> cmats_h_;
   MatDev* cmats_d_ = nullptr;
   int64_t *cbase_d_ = nullptr, *cblk_base_d_ = nullptr;
   int32_t* cblk_mat_d_ = nullptr;
   int64_t cnodes_ = 0, cnblk_ = 0, cond_words_ = 0;
   int32_t cn_max_ = 0, cut_divisor_ = 0;
-  int32_t *vroot_ = nullptr, *nid_ = nullptr, *cond_zero_ = nullptr, *root_list_ = nullptr, *root_wri_ = nullptr;
+  int32_t *nid_ = nullptr, *cond_zero_ = nullptr;
+  FrontUnit* units_ = nullptr;
+  FrontLaunch fronts_[kFrontLevels];
   uint64_t* citems_ = nullptr;
   int32_t* cspill_ = nullptr;
   LaunchConfig ccfg_;

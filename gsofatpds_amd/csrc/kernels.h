@@ -56,6 +56,17 @@ inline int acc_copies(int nmats) {
   return c;
 }
 
+// A front unit: the elimination subtree (of A + A^T) of row c of matrix `mat`, rows lo .. c. Its list
+// of direction d (the edges of its contracted root) starts at ulist + off + d * cap.
+struct FrontUnit {
+  int32_t mat, c, lo, cap;
+  int64_t off;
+};
+constexpr int kFrontMsg = 17;  // a bit per node of a unit, and a length
+// A vertex's state: which directions of its row are finished (a mirrored matrix has direction 0
+// only), and u + 1 where it is contracted into the root of unit u; with kStRoot it is that root.
+constexpr int32_t kStDone0 = 1 << 30, kStDone1 = 1 << 28, kStRoot = 1 << 29, kStUnit = kStDone1 - 1;
+
 // One matrix as the kernels see it. Direction 0 traverses A (rows, gives U), direction 1
 // traverses A^T (columns of A, gives L by columns).
 struct MatDev {
@@ -87,22 +98,21 @@ struct MatDev {
                                   // (a top separator's, n: none) are fixed workgroup-path items of
                                   // an early launch, escalated from the start
   int32_t light_limit;            // reached vertices before the wave path escalates a row
-  const int32_t* subtree;         // n: elimination-subtree sizes of A + A^T (null: none); the sign
-                                  // bit marks a condensation root
+  const int32_t* subtree;         // n: elimination-subtree sizes of A + A^T (null: none)
   int32_t pre_size;               // a row whose subtree exceeds this escalates without a
                                   // wave-path attempt (its reached set would exceed the limit)
-  // Condensation (kernels.hip, "condensed graph"). Of a matrix whose workgroup path runs on the
-  // condensed graph; vroot is null otherwise.
-  const int32_t* vroot;           // n: the root whose elimination subtree holds the vertex, or -1
-  uint8_t* mark[2];               // n: 1 where the vertex is in its root's R (per direction)
-  int32_t* root_cnt[2];           // per root: 1 + entries of its list, 0 while it has not finished
-  int32_t* root_list[2];          // per root, list_cap entries: U of the root, then the vertices of
-                                  // its R that the contraction leaves out
-  int32_t* root_bad;              // per root: 1 when some row of its subtree escalated
-  int32_t *root_w, *root_r;       // per root: sum of degrees of, and vertices in, {root} + R (dir. 0)
-  int32_t* root_id;               // per root: its node
-  int32_t* nid;                   // n: the vertex's node, -1 where it is part of its root's
-  int32_t list_cap;
+  // Fronts and the condensed graph (kernels.hip, k_front); st is null for a matrix without them.
+  int32_t* st;                    // n: state of the vertex (kSt*)
+  int32_t* nid;                   // n: the vertex's node in the condensed graph, -1 if contracted
+  // of every front unit of the set (k_front)
+  const FrontUnit* units;
+  int32_t* ulist;                 // the units' lists (FrontUnit::off)
+  int32_t* ulen;                  // 2 per unit: entries of its list, per direction
+  int32_t* uwt;                   // 2 per unit: sum of degrees and number of vertices of its S
+  int32_t* uid;                   // per unit: its root's node
+  uint32_t* umsg;                 // kFrontMsg per unit and direction: its root's reached nodes as bits,
+                                  // and in the last word the length of its list above the root
+  uint32_t* uctr;                 // per unit: directions ended, 1 for each that fitted, 16 for the others
   // A condensed graph as k_heavy sees it (n nodes; ell, rowptr, adj, esc by node).
   const int32_t* orig;            // n: the node's vertex, or -(r + 1): a list node of root r
   const int32_t* wt;              // 2 n: what to add to the node's entry count for its input degree,
@@ -140,7 +150,7 @@ __host__ __device__ inline uint64_t encode_item(uint32_t mat, uint32_t dir, uint
 namespace gsofa {
 hipError_t launch_fill_u64(unsigned long long* p, int64_t count, unsigned long long v, hipStream_t s);
 // A run's clears in one launch (all to zero): nacc u64 at acc, nws u64 at ws, nesc, nblk, nbucket
-// and ncond i32 words at esc, blk_flag, bucket and cond.
+// and ncond i32 words at esc, blk_flag, bucket and cond (the vertices' states).
 hipError_t launch_clear_run(unsigned long long* acc, int64_t nacc, unsigned long long* ws, int64_t nws, int32_t* esc,
                             int64_t nesc, int32_t* blk_flag, int64_t nblk, int32_t* bucket, int64_t nbucket,
                             int32_t* cond, int64_t ncond, hipStream_t s);
@@ -152,10 +162,9 @@ hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, c
 hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* col_cnt, int32_t* rowptr_t, int32_t* cursor,
                             int32_t* adj_t, int32_t* block_sums, int32_t* total, hipStream_t s);
-// bits: kLightBits, or kLightBitsBig (a hash set of 2,048 slots and an escalation limit of 1,024);
-// roots: some matrix has condensation roots (vroot)
+// bits: kLightBits, or kLightBitsBig (a hash set of 2,048 slots and an escalation limit of 1,024)
 hipError_t launch_light(const MatDev* mats, int nmats, const int64_t* item_base, int64_t nitems, WorkState* ws, int grid, int bits,
-                        bool roots, hipStream_t s);
+                        hipStream_t s);
 // The escalated blocks (blk_flag, 2 * nblk_total slots) into heavy_items in descending block
 // order; sets ws->heavy_count. bucket has nb_max entries, cursor nb_max + 1, block_sums
 // ceil(nb_max / 4096), total one int.
@@ -191,11 +200,32 @@ constexpr int64_t heavy_region_ints(int64_t n_max, bool paired_any) {
 hipError_t launch_heavy(int threads, int grid, const MatDev* mats, WorkState* ws, const uint64_t* heavy_items,
                         int32_t bw_max, int32_t qcap, int64_t n_max, int32_t paired_any, int32_t* spill,
                         uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, hipStream_t s);
-// The condensed graphs (kernels.hip): sizes[b] += nodes of matrix b, after a wave path over zeroed
-// marks, lists and sizes.
+// What a front level holds per unit: alive nodes (its rows not yet contracted), surface vertices (rows
+// above the unit that its rows hold), words of one direction's bit matrix and of one of its rows. A
+// unit with more is left to the next level or to k_heavy.
+struct FrontSize {
+  int32_t nodes, ext, words, width;
+};
+constexpr int kFrontLevels = 3;
+// At most (the kernels' registers; level 2: the LDS of a CU).
+constexpr FrontSize kFrontMax[kFrontLevels] = {{64, 128, 0, 0}, {256, 768, 256 * 36, 36}, {512, 1536, 512 * 48, 68}};
+// One level's launch: its units, its resident workgroups (front_occupancy), and what its LDS holds.
+struct FrontLaunch {
+  int32_t u0 = 0, u1 = 0;
+  int grid = 0;
+  FrontSize size = {0, 0, 0, 0};
+};
+// Finishes the rows of the level's units and contracts their roots; the vertices' states are zero
+// before level 0. most (levels 1 and up, may be null): the largest of the units that it took.
+hipError_t launch_front(int level, const FrontLaunch& L, const MatDev* mats, const FrontUnit* units, FrontSize* most,
+                        hipStream_t s);
+// Sets the LDS limit of a level's kernel and returns its resident workgroups per CU (0: error).
+int front_occupancy(int level, const FrontSize& z);
+// The condensed graphs (kernels.hip): sizes[b] += nodes of matrix b, sizes[nmats + b] += its unfinished
+// rows of direction 0, after the fronts.
 hipError_t launch_cond_sizes(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows,
                              unsigned long long* sizes, hipStream_t s);
-// Builds them after the wave path: cmats the condensed matrices (by matrix index), cbase[b] the first
+// Builds them after the fronts: cmats the condensed matrices (by matrix index), cbase[b] the first
 // of the set's `nodes` nodes that is matrix b's, cblk_base / cblk_mat the ncond condensed matrices'
 // blocks in item order. Items: 2 nblk, then at most 2 nblk before cuts (cut_divisor 0: no cuts).
 hipError_t launch_condense(const MatDev* mats, const MatDev* cmats, int nmats, const int64_t* row_base, int64_t nrows,

@@ -19,13 +19,17 @@
 //   k_ell_build                 pack rows into 64-byte ELL-16 slots
 //   k_col_hist, scan, k_transpose_scatter, k_ell_build   build A^T in the same layout
 //   k_light                     one wave per block of rows, LDS hash set; escalates big sources
+//   k_front_leaf, k_front       (matrices with fronts, instead) elimination subtrees as bit matrices
+//   k_cond_*                    (these) the graph of what the fronts left, and its items
 //   k_heavy_hist, scan, k_heavy_scatter   the workgroup path's queue, costliest blocks first
-//   k_heavy                     one workgroup per block of escalated rows, n-bit bitmap
+//   k_heavy                     one workgroup per block of escalated (or left) rows, n-bit bitmap
 //   k_supernodes                the reference's supernode rule, one thread per row
+//   k_totals                    sums the accumulators' copies
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kernels.h"
 
@@ -50,6 +54,11 @@ __device__ __forceinline__ void gstore(T* p, T v) {
 typedef int32_t v4i32 __attribute__((ext_vector_type(4)));
 typedef int32_t v2i32 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ v4i32 gload_v4(const int32_t* p) { return *(const GSOFA_GLOBAL v4i32*)(p); }
+typedef uint32_t v4u32 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void gstore_v4(uint32_t* p, uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  const v4u32 v = {a, b, c, d};
+  *(GSOFA_GLOBAL v4u32*)(p) = v;
+}
 
 __device__ __forceinline__ uint32_t rank_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
@@ -108,6 +117,11 @@ __device__ __forceinline__ uint32_t wave_or_u32(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
 }
 
+// Sum over the wave of values below 2^50, the same in every lane (two scans of 24 and 26 bits).
+__device__ __forceinline__ uint64_t wave_sum_u50(uint64_t x) {
+  return wave_sum_u32((uint32_t)x & 0xFFFFFFu) + ((uint64_t)wave_sum_u32((uint32_t)(x >> 24)) << 24);
+}
+
 // Lanes of one wave hand data to each other through LDS (one lane writes a count, others read
 // it; lanes read queue entries other lanes wrote) between steps that no workgroup barrier
 // separates. Release and acquire at wavefront scope around a wave barrier: every access of the
@@ -144,8 +158,7 @@ __global__ void k_fill_i32(int32_t* p, int64_t count, int32_t v) {
 }
 
 // A run's clears in one launch: accumulators and work state (u64), escalation and block flags,
-// the workgroup-path queue's buckets and the condensation's marks and lists (i32 words), all to
-// zero.
+// the workgroup-path queue's buckets and the vertices' states (i32 words), all to zero.
 __global__ void k_clear_run(unsigned long long* __restrict__ acc, int64_t nacc, unsigned long long* __restrict__ ws,
                             int64_t nws, int32_t* __restrict__ esc, int64_t nesc, int32_t* __restrict__ blk_flag,
                             int64_t nblk, int32_t* __restrict__ bucket, int64_t nbucket, int32_t* __restrict__ cond,
@@ -475,9 +488,7 @@ __device__ __forceinline__ bool hash_has(const int32_t* H, int32_t m) {
 // X_s). A row that holds an escalated u < s escalates without an attempt: X_u, already over the
 // limit, is part of X_s.
 
-// kRoots: some matrix of the set has condensation roots (the extra code costs the 1,024-slot variant
-// registers: 1 % on a 1,024-row matrix).
-template <int kBits, bool kRoots>
+template <int kBits>
 __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_eu(kBits == kLightBitsBig ? 3 : 5))) void k_light(
     const MatDev* __restrict__ mats, int nmats, const int64_t* __restrict__ item_base, int64_t nitems,
     WorkState* __restrict__ ws) {
@@ -640,8 +651,7 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
       const int32_t chunk_end = min(M.n, (src / M.chunk + 1) * M.chunk);
       // A row whose elimination subtree exceeds pre_size escalates at once: its reached set holds
       // its whole subtree (mirrored matrices), or nearly (pre_size leaves a margin otherwise).
-      const int32_t sub = M.subtree != nullptr ? gload(M.subtree + src) : 0;
-      const bool pre = (kRoots ? sub & INT32_MAX : sub) > M.pre_size;
+      const bool pre = M.subtree != nullptr && gload(M.subtree + src) > M.pre_size;
       RowCursor rc;
       // the source row, one ELL slot per lane (lanes 0..15); slot 15 <= -2 encodes a CSR tail
       const int32_t sm = lane < kEll ? gload(M.ell[dir] + (int64_t)src * kEll + lane) : kPad;
@@ -935,26 +945,6 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
               for (int i = lane; i < uq; i += 64) gstore(M.pool[dir] + off + i, Q[kLightQ - 1 - i]);
             }
           }
-          // A condensation root: its reached vertices are marked and its U list is kept.
-          if (kRoots && sub < 0) {
-            const int32_t r = gload(M.vroot + src);
-            int32_t* const list = M.root_list[dir] + (int64_t)r * M.list_cap;
-            int32_t nl = 0;
-            for (int i = lane; i < kHash; i += 64) {
-              const int32_t m = H[i];
-              if (m >= 0 && m < src) gstore(M.mark[dir] + m, (uint8_t)1);
-              const uint64_t mu = __ballot(m > src);
-              if (m > src) gstore(list + nl + (int32_t)rank_below(mu), m);
-              nl += __popcll(mu);
-            }
-            if (lane == 0) {
-              gstore(M.root_cnt[dir] + r, nl + 1);
-              if (dir == 0) {
-                gstore(M.root_w + r, (int32_t)(wr + deg0));
-                gstore(M.root_r + r, (int32_t)rr + 1);
-              }
-            }
-          }
           carry_ok = true;
           prev_esc = false;
           u_prev = U;
@@ -966,12 +956,7 @@ __global__ __launch_bounds__(kLightWaves * 64) __attribute__((amdgpu_waves_per_e
       if (esc) {
         if (lane == 0) {
           gstore(M.esc[dir] + src, (uint8_t)1);
-          if (!kRoots || M.vroot == nullptr) {
-            gstore(M.blk_flag[dir] + src / M.chain_block, 1u);  // the block goes to the workgroup path
-          } else if (!pre) {  // its root's subtree stays as it is (a pre-escalated row lies in none)
-            const int32_t r = gload(M.vroot + src);
-            if (r >= 0) gstore(M.root_bad + r, 1);
-          }
+          gstore(M.blk_flag[dir] + src / M.chain_block, 1u);  // the block goes to the workgroup path
         }
         carry_ok = false;
         prev_esc = true;
@@ -1070,90 +1055,971 @@ __global__ void k_heavy_scatter(const MatDev* __restrict__ mats, int64_t nblk_to
 }
 
 // ------------------------------------------------------------------------------------------
-// The condensed graph of a matrix, on which the workgroup path runs.
+// Fronts: whole elimination subtrees in bit matrices, and the condensed graph they leave.
 //
-// Every block of the workgroup path begins with a traversal of its first row's whole reached set,
-// most of which lies in small subtrees that the wave path has finished already. Let c be a root: a
-// row whose elimination subtree T(c) of A + A^T is small enough for the wave path while its
-// parent's is not. R_c lies in T(c), and S(c) = {c} + (R_c of A, R_c of A^T) is strongly connected
-// through vertices up to c. A source s outside T(c) reaches, through vertices below s, all of S(c)
-// or none of it (T(c) lies below s when s reaches it at all), so S(c) may be contracted into the
-// node c: its edges are U_c and the vertices of R_c outside S(c), its weights |S(c)| and the sum of
-// S(c)'s degrees. Roots whose subtree holds an escalated row stay as they are. Nodes keep the order
-// of their vertices (a contracted set takes its root's place), so every rule of k_heavy (chaining,
-// imports, cuts) holds on the condensed graph as on the matrix, and the U lists are the same.
+// A unit is the elimination subtree T(c) of A + A^T of a row c, a range of rows (postorder). A row
+// v of T(c) reaches only vertices of T(c) and, above c, a few more (its surface), so a workgroup
+// holds the whole subtree as a bit matrix in LDS: row i has a bit per vertex of the unit and per
+// vertex above it that some row holds. Boolean elimination in ascending order (row i takes in row k
+// for every bit k < i) leaves in row i R_i below the diagonal and U_i above it, for all rows at
+// once: for 100 rows of a 2-D stencil some 10^4 word operations, where the wave path takes two
+// traversals of some 700 instructions each per row.
 //
-// A root's edges do not fit one 16-entry row: they are held by list nodes right below the root
-// (leaves of up to 16 edges, then nodes over up to 16 leaves when there are more than 16 leaves),
-// which have no vertices and no degree of their own.
+// The unit's root is then contracted. S(c) = {c} + (R_c of A, R_c of A^T) is strongly connected
+// through vertices up to c, and a source s outside T(c) reaches, through vertices below s, all of
+// it or nothing (T(c) lies below s when s reaches it at all): S(c) becomes the node c, whose edges
+// are U_c and the vertices of R_c outside S(c) (the unit's list) and whose weights are |S(c)| and
+// S(c)'s degrees. The rows of a larger subtree hold a node for each unit inside it, so the next
+// level takes subtrees of thousands of rows as a matrix of a few hundred nodes, and what no level
+// takes runs on k_heavy over the condensed graph of the remaining nodes (below k_front): U lists,
+// |R| and degree sums come out the same, on a graph a tenth of the matrix (659,033-row 2-D stencil).
+// A unit that does not fit (more nodes or surface than the level's matrices hold) is left as it is.
 //
-// 659,033-row 2-D stencil: 57 k nodes for 659 k vertices (a 7 KB bitmap instead of 82 KB, so
-// several workgroups per CU).
+// In LDS the elimination goes by blocks of 32 pivots: the block's own closure in registers, each
+// row's coefficients (the block's pivots it reaches) by one thread per row, then every (row, word)
+// ORs the pivot rows its coefficients name, held in registers. Two barriers per block instead of
+// one per pivot, and no chain of dependent LDS reads.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ int32_t cond_leaves(int32_t len) { return len <= kEll ? 0 : (len + kEll - 1) / kEll; }
-__device__ __forceinline__ int32_t cond_mids(int32_t leaves) {
-  return leaves <= kEll ? 0 : (leaves + kEll - 1) / kEll;
-}
-__device__ __forceinline__ int32_t cond_list_len(const MatDev& M, int d, int32_t r) {
-  return M.sym && d == 1 ? 0 : min(gload(M.root_cnt[d] + r) - 1, M.list_cap);
-}
-__device__ __forceinline__ int32_t cond_list_nodes(const MatDev& M, int32_t r) {
-  const int32_t l0 = cond_leaves(cond_list_len(M, 0, r)), l1 = cond_leaves(cond_list_len(M, 1, r));
-  return max(l0 + cond_mids(l0), l1 + cond_mids(l1));
-}
-// Whether root r is contracted: finished in both directions, and no row of its subtree escalated.
-__device__ __forceinline__ bool cond_valid(const MatDev& M, int32_t r) {
-  return gload(M.root_cnt[0] + r) != 0 && (M.sym || gload(M.root_cnt[1] + r) != 0) && gload(M.root_bad + r) == 0;
-}
-// The nodes vertex v brings: itself, a contracted root's list nodes and itself, or none (contracted).
-__device__ __forceinline__ int32_t cond_nodes(const MatDev& M, int32_t v) {
-  if (M.vroot == nullptr) return 0;
-  const int32_t r = gload(M.vroot + v);
-  if (r < 0) return 1;
-  const bool in = gload(M.mark[0] + v) != 0 && (M.sym || gload(M.mark[1] + v) != 0);
-  const bool root = gload(M.subtree + v) < 0;
-  if ((!in && !root) || !cond_valid(M, r)) return 1;
-  return root ? 1 + cond_list_nodes(M, r) : 0;
-}
+// Level 0: one wave per unit of at most 64 rows, a row per lane, its bits in registers (64 for the
+// unit, 128 for the surface): a pivot is a handful of lane reads and ORs, without LDS or a barrier.
+constexpr int kLeafWaves = 4, kLeafSlots = 256, kLeafExtWords = kFrontMax[0].ext / 32;
 
-// The vertices of R_c outside S(c) join the root's list of their direction and leave its weights.
-__global__ __launch_bounds__(256) void k_cond_append(const MatDev* __restrict__ mats, int nmats,
-                                                     const int64_t* __restrict__ row_base, int64_t nrows) {
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < nrows; g += (int64_t)gridDim.x * blockDim.x) {
-    const int mb = nmats == 1 ? 0 : find_segment(row_base, nmats, g);
-    const MatDev& M = mats[mb];
-    if (M.vroot == nullptr || M.sym) continue;  // mirrored: both directions reach the same
-    const int32_t v = (int32_t)(g - row_base[mb]);
-    const int32_t r = gload(M.vroot + v);
-    if (r < 0) continue;
-    const bool m0 = gload(M.mark[0] + v) != 0, m1 = gload(M.mark[1] + v) != 0;
-    if (m0 == m1 || gload(M.subtree + v) < 0 || !cond_valid(M, r)) continue;
-    const int d = m0 ? 0 : 1;
-    const int32_t pos = atomicAdd(M.root_cnt[d] + r, 1) - 1;
-    if (pos < M.list_cap) gstore(M.root_list[d] + (int64_t)r * M.list_cap + pos, v);
-    else atomicOr(&M.acc[kAccScheduleError], 1ull);  // cannot happen: |X_c| is at most the limit
-    if (d == 0) {
-      const int32_t deg = gload(M.rowptr[0] + v + 1) - gload(M.rowptr[0] + v) + (M.dup_all ? gload(M.dup_all + v) : 0);
-      atomicAdd(M.root_w + r, -deg);
-      atomicAdd(M.root_r + r, -1);
+__global__ __launch_bounds__(kLeafWaves * 64) void k_front_leaf(const MatDev* __restrict__ mats,
+                                                                const FrontUnit* __restrict__ units, int32_t u0,
+                                                                int32_t u1) {
+  static_assert(kFrontMax[0].nodes == 64 && kLeafExtWords == 4, "a row per lane, four surface words");
+  static_assert(kFrontMax[0].ext + 64 < kLeafSlots, "the hash must never fill");
+  __shared__ int32_t s_keys[kLeafWaves][kLeafSlots];
+  __shared__ uint8_t s_vals[kLeafWaves][kLeafSlots];
+  __shared__ int32_t s_ext[kLeafWaves][kFrontMax[0].ext];
+  const int lane = lane_id(), wave = threadIdx.x >> 6;
+  int32_t* const keys = s_keys[wave];
+  uint8_t* const vals = s_vals[wave];
+  int32_t* const ext = s_ext[wave];
+  auto home = [](int32_t key) { return (((uint32_t)key * 0x9E3779B1u) >> 24) & (kLeafSlots - 1); };
+
+  uint64_t t_w = 0, t_r = 0;
+  uint32_t t_fill = 0, t_u = 0, t_l = 0, t_e = 0, t_v = 0;  // of one matrix and lane: below 2^32
+  int last_mat = -1;
+  auto flush = [&]() {
+    if (last_mat < 0) return;
+    unsigned long long* acc = acc_of(mats[last_mat]);
+    const uint64_t f = wave_sum_u50(t_fill), w = wave_sum_u50(t_w), r = wave_sum_u50(t_r), u = wave_sum_u50(t_u),
+                   l = wave_sum_u50(t_l), e = wave_sum_u50(t_e), v = wave_sum_u50(t_v);
+    if (lane == 0) {
+      if (f) atomicAdd(&acc[kAccFill], f);
+      if (w) atomicAdd(&acc[kAccW], w);
+      if (r) atomicAdd(&acc[kAccR], r);
+      if (u) atomicAdd(&acc[kAccNnzU], u);
+      if (l) atomicAdd(&acc[kAccNnzL], l);
+      if (e) atomicAdd(&acc[kAccLightExecEdges], e);
+      if (v) atomicAdd(&acc[kAccLightExecVerts], v);
+      if (u + l) atomicAdd(&acc[kAccLightExecOut], u + l);
+    }
+    t_fill = t_w = t_r = t_u = t_l = t_e = t_v = 0;
+  };
+
+  const int32_t stride = (int32_t)gridDim.x * kLeafWaves;
+  for (int32_t u = u0 + (int32_t)blockIdx.x * kLeafWaves + wave; u < u1; u += stride) {
+    const FrontUnit F = units[u];
+    if (F.mat != last_mat) {
+      flush();
+      last_mat = F.mat;
+    }
+    const MatDev& M = mats[F.mat];
+    const bool sym = M.sym != 0;
+    const int32_t c = F.c, lo = F.lo, m = c - lo + 1;
+    const bool on = lane < m;
+    const int32_t v = lo + lane;
+    RowCursor rc[2];
+    load_row(M, 0, on ? v : -1, rc[0]);
+    load_row(M, 1, on && !sym ? v : -1, rc[1]);
+    uint32_t deg = 0;
+    if (on) deg = (uint32_t)(gload(M.rowptr[0] + v + 1) - gload(M.rowptr[0] + v) + (M.dup_all ? gload(M.dup_all + v) : 0));
+    wave_sync();
+    for (int i = lane; i < kLeafSlots; i += 64) keys[i] = -1;
+    wave_sync();
+    // ---- the surface: every entry above c ----
+    int ne = 0;
+    auto add_ext = [&](int32_t x) {  // wave-uniform call; stops when the surface is too large
+      bool fresh = false;
+      if (x > c && ne <= kFrontMax[0].ext) {
+        uint32_t h = home(x);
+        while (true) {
+          const int32_t old = atomicCAS(&keys[h], -1, x);
+          fresh = old == -1;
+          if (fresh || old == x) break;
+          h = (h + 1) & (kLeafSlots - 1);
+        }
+      }
+      ne += __popcll(__ballot(fresh));
+    };
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+#pragma unroll
+      for (int k = 0; k < kEll; ++k)
+        if (__ballot(rc[d].e[k] > c) != 0) add_ext(rc[d].e[k]);
+      for (int32_t p = rc[d].ov_pos; __ballot(p < rc[d].ov_end) != 0; ++p)
+        add_ext(p < rc[d].ov_end ? gload(M.adj[d] + p) : kPad);
+    }
+    if (ne > kFrontMax[0].ext) continue;  // too large a surface: left to the next level
+    wave_sync();
+    uint64_t near0 = 0, near1 = 0;  // surface vertices within 128 of c
+    {
+      int base = 0;
+#pragma unroll
+      for (int q = 0; q < kLeafSlots / 64; ++q) {
+        const int32_t key = keys[q * 64 + lane];
+        const uint64_t mk = __ballot(key >= 0);
+        if (key >= 0) {
+          const int x = base + (int)rank_below(mk);
+          vals[q * 64 + lane] = (uint8_t)x;
+          ext[x] = key;
+        }
+        base += __popcll(mk);
+      }
+      wave_sync();
+      near0 = __ballot(lane < ne && ext[lane] <= c + 128);
+      near1 = __ballot(lane + 64 < ne && ext[lane + 64] <= c + 128);
+    }
+    uint64_t in_last[2] = {0, 0}, ext_last[2][2] = {{0, 0}, {0, 0}};  // the root's row, per direction
+    const int32_t chunk_end = min(M.n, (v / M.chunk + 1) * M.chunk);
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      if (d == 1 && sym) break;
+      // ---- the row's bits ----
+      uint64_t in = 0;
+      uint32_t x0 = 0, x1 = 0, x2 = 0, x3 = 0, seed = 0;
+      auto set = [&](int32_t e) {
+        if (e < 0) return;
+        ++t_e;
+        seed += e > v;
+        if (e <= c) {
+          in |= 1ull << ((e - lo) & 63);  // a row of T(c) holds no vertex below c outside it
+        } else {
+          uint32_t h = home(e);
+          while (keys[h] != e) h = (h + 1) & (kLeafSlots - 1);  // it was inserted above
+          const int x = vals[h];
+          const uint32_t b = 1u << (x & 31);
+          const int w = x >> 5;
+          x0 |= w == 0 ? b : 0u;
+          x1 |= w == 1 ? b : 0u;
+          x2 |= w == 2 ? b : 0u;
+          x3 |= w == 3 ? b : 0u;
+        }
+      };
+#pragma unroll
+      for (int k = 0; k < kEll; ++k)
+        if (__ballot(rc[d].e[k] >= 0) != 0) set(rc[d].e[k]);
+      for (int32_t p = rc[d].ov_pos; p < rc[d].ov_end; ++p) set(gload(M.adj[d] + p));
+      // ---- elimination: the rows above k that hold k take in row k ----
+      uint32_t i0 = (uint32_t)in, i1 = (uint32_t)(in >> 32);
+      const uint64_t below = (1ull << lane) - 1;
+      const uint32_t b0 = (uint32_t)below, b1 = (uint32_t)(below >> 32);
+      auto pivots = [&](auto wide) {
+        for (int k = 0; k < min(m, 32); ++k) {
+          const uint32_t hold = 0u - (((i0 & b0) >> k) & 1u);
+          i0 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)i0, k);
+          i1 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)i1, k);
+          x0 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x0, k);
+          x1 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x1, k);
+          if constexpr (decltype(wide)::value) {
+            x2 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x2, k);
+            x3 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x3, k);
+          }
+        }
+        for (int k = 32; k < m; ++k) {
+          const uint32_t hold = 0u - (((i1 & b1) >> (k - 32)) & 1u);
+          i0 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)i0, k);
+          i1 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)i1, k);
+          x0 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x0, k);
+          x1 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x1, k);
+          if constexpr (decltype(wide)::value) {
+            x2 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x2, k);
+            x3 |= hold & (uint32_t)__builtin_amdgcn_readlane((int)x3, k);
+          }
+        }
+      };
+      if (ne <= 64) pivots(std::false_type{});
+      else pivots(std::true_type{});
+      // ---- the row's results ----
+      in = ((uint64_t)i1 << 32) | i0;
+      const uint64_t r = in & below, up = in & ~below & ~(1ull << lane);
+      const uint64_t e0 = ((uint64_t)x1 << 32) | x0, e1 = ((uint64_t)x3 << 32) | x2;
+      const uint32_t U = (uint32_t)(__popcll(up) + __popcll(e0) + __popcll(e1));
+      if (d == 0) {
+        // the degrees of R: a count per bit of the degrees
+        uint64_t nd = 0;
+        for (int b = 0; __ballot((deg >> b) != 0) != 0; ++b)
+          nd += (uint64_t)(uint32_t)__popcll(r & __ballot(((deg >> b) & 1u) != 0)) << b;
+        if (on) {
+          t_w += deg + nd;
+          t_r += (uint32_t)__popcll(r);
+          t_u += U;
+          ++t_v;
+        }
+      } else if (on) {
+        t_l += U;
+      }
+      if (on) {
+        t_fill += U - seed;
+        gstore(M.cnt[d] + v, (int32_t)U);
+      }
+      if (d == 1 || sym) {
+        // rows v + 1 .. v + 128: the unit's rows follow v; then the near surface
+        uint32_t win[4] = {0, 0, 0, 0};
+        uint64_t y = up >> lane >> 1;
+        const int32_t room = chunk_end - v - 1;
+        if (room < 64) y &= (1ull << (room < 0 ? 0 : room)) - 1;
+        win[0] = (uint32_t)y;
+        win[1] = (uint32_t)(y >> 32);
+        for (uint64_t nb = near0; nb; nb &= nb - 1) {
+          const int j = __ffsll((unsigned long long)nb) - 1;
+          if ((e0 >> j) & 1ull) window_bit(win, v, ext[j], chunk_end);
+        }
+        for (uint64_t nb = near1; nb; nb &= nb - 1) {
+          const int j = __ffsll((unsigned long long)nb) - 1;
+          if ((e1 >> j) & 1ull) window_bit(win, v, ext[64 + j], chunk_end);
+        }
+        if (on) gstore_v4(M.win + 4 * (int64_t)v, win[0], win[1], win[2], win[3]);
+      }
+      if (M.list_ptr[d] != nullptr && on) {
+        const int64_t off = gload(M.list_ptr[d] + v);
+        if (gload(M.list_ptr[d] + v + 1) - off != (int64_t)U) {
+          atomicOr(&M.acc[kAccOverflow], 1ull);
+        } else {
+          int32_t* p = M.pool[d] + off;
+          for (uint64_t y = up; y; y &= y - 1) gstore(p++, lo + __ffsll((unsigned long long)y) - 1);
+          for (uint64_t y = e0; y; y &= y - 1) gstore(p++, ext[__ffsll((unsigned long long)y) - 1]);
+          for (uint64_t y = e1; y; y &= y - 1) gstore(p++, ext[64 + __ffsll((unsigned long long)y) - 1]);
+        }
+      }
+      auto of_root = [&](uint64_t x) -> uint64_t {
+        return ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), m - 1) << 32) |
+               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, m - 1);
+      };
+      in_last[d] = of_root(r);
+      ext_last[d][0] = of_root(e0);
+      ext_last[d][1] = of_root(e1);
+    }
+    // ---- contract the root ----
+    const uint64_t s = (sym ? in_last[0] : in_last[0] & in_last[1]) | (1ull << (m - 1));
+    const bool inside = (s >> lane) & 1ull;
+    if (on) gstore(M.st + v, kStDone0 | kStDone1 | (inside ? (lane == m - 1 ? kStRoot : 0) | (u + 1) : 0));
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      if (d == 1 && sym) break;
+      int32_t* const list = M.ulist + F.off + (int64_t)d * F.cap;
+      const uint64_t out = in_last[d] & ~s;  // reached, but not in S(c)
+      const uint64_t a = ext_last[d][0], b = ext_last[d][1];
+      const int na = __popcll(a), nb = __popcll(b);
+      if ((a >> lane) & 1ull) gstore(list + rank_below(a), ext[lane]);
+      if ((b >> lane) & 1ull) gstore(list + na + rank_below(b), ext[64 + lane]);
+      if ((out >> lane) & 1ull) gstore(list + na + nb + rank_below(out), v);
+      if (lane == 0) gstore(M.ulen + 2 * (int64_t)u + d, (int32_t)(na + nb + __popcll(out)));
+    }
+    if (sym && lane == 0) gstore(M.ulen + 2 * (int64_t)u + 1, 0);
+    const uint32_t sdeg = wave_sum_u32(inside ? deg : 0u);
+    if (lane == 0) {
+      gstore(M.uwt + 2 * (int64_t)u, (int32_t)sdeg);
+      gstore(M.uwt + 2 * (int64_t)u + 1, (int32_t)__popcll(s));
     }
   }
+  flush();
 }
 
-// Nodes per matrix (when a set is created: they size the condensed graph).
+// Levels 1 and up: one workgroup per unit and direction, the bit matrix in LDS; the direction that
+// ends last contracts the root. Bound by the latency of the steps on the few units a level has: the
+// 64 units of a 49,729-row matrix run side by side, each some 20 barriers long.
+constexpr int kFrontThreads[kFrontLevels] = {kLeafWaves * 64, 256, 512};
+
+// The dynamic LDS of a level, for units that FrontSize holds.
+struct FrontLds {
+  uint32_t* B;         // row i at B + i * W (W: the unit's words per row)
+  uint32_t* P;         // the pivot rows of a block
+  uint32_t* coef;      // of the k-th row that takes in pivots of the block: which
+  uint16_t* act;       // and which row it is
+  int32_t* seed;       // entries of the row above its diagonal
+  int32_t* tail;       // where the row's entries beyond its slots start in the CSR, or -1
+  int32_t* keys;       // hash of the unit's vertices: vertex, -1 empty
+  uint16_t* vals;      // its number: node, or far surface vertex
+  int32_t* ids;        // vertex of a node
+  int32_t* unit;       // unit of a contracted node, -1 a vertex, -2 a vertex whose row is not finished
+  int32_t* ext;        // far surface vertices
+  int32_t* wdeg;       // degrees a node stands for
+  // degrees and vertices that the nodes stand for, as bit planes (plane b: the nodes whose number has
+  // bit b), so that a row's sums are population counts
+  uint32_t *pdeg, *pcnt;
+  uint32_t* run;       // 1: the word's nodes are consecutive vertices
+  size_t bytes;
+  static constexpr int kDegBits = 32, kCntBits = 31;
+  __host__ __device__ FrontLds(char* p, const FrontSize& z, int slots) {
+    const int wi = (z.nodes + 31) / 32;
+    char* const p0 = p;
+    auto take = [&](auto*& to, int n) {
+      to = reinterpret_cast<std::remove_reference_t<decltype(to)>>(p);
+      p += ((size_t)n * sizeof(*to) + 15) & ~size_t(15);
+    };
+    take(B, z.words);
+    take(P, 32 * z.width);
+    take(coef, z.nodes);
+    take(act, z.nodes);
+    take(seed, z.nodes);
+    take(tail, z.nodes);
+    take(keys, slots);
+    take(vals, slots);
+    take(ids, z.nodes);
+    take(unit, z.nodes);
+    take(ext, z.ext);
+    take(wdeg, z.nodes);
+    take(pdeg, kDegBits * wi);
+    take(pcnt, kCntBits * wi);
+    take(run, wi);
+    bytes = (size_t)(p - p0);
+  }
+};
+// Hash slots: more than a unit's vertices and each thread's insertion past the limit.
+__host__ __device__ constexpr int front_slots(int level) { return level == 1 ? 2048 : 4096; }
+static_assert(kFrontMax[1].nodes + kFrontMax[1].ext + kFrontThreads[1] < front_slots(1), "the hash must never fill");
+static_assert(kFrontMax[2].nodes + kFrontMax[2].ext + kFrontThreads[2] < front_slots(2), "the hash must never fill");
+
+template <int kLevel>
+__global__ __launch_bounds__(kFrontThreads[kLevel]) __attribute__((amdgpu_waves_per_eu(4))) void k_front(
+    const MatDev* __restrict__ mats, const FrontUnit* __restrict__ units, int32_t u0, int32_t u1, FrontSize Z,
+    FrontSize* __restrict__ most) {
+  constexpr int T = kFrontThreads[kLevel], kRows = T / kEll, kPer = kFrontMax[kLevel].nodes / kRows;
+  constexpr int kSlots = front_slots(kLevel), kScanPer = 4;
+  static_assert(T >= kFrontMax[kLevel].nodes && kFrontMax[kLevel].nodes <= 32 * kEll, "a row per thread, a word of it per lane");
+  extern __shared__ uint32_t dyn[];
+  const FrontLds S(reinterpret_cast<char*>(dyn), Z, kSlots);
+  const int nb = Z.nodes, eb = Z.ext, wi_max = (nb + 31) / 32;
+  __shared__ int32_t s_wave[T / 64];
+  __shared__ int32_t s_ne, s_num, s_fail, s_near, s_sdeg, s_scnt, s_len[2], s_nact[2], s_other;
+  __shared__ uint32_t s_bits[2];  // all degrees, all counts, OR-ed
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6, sl = tid & (kEll - 1);
+  uint32_t* const B = S.B;
+
+  auto home = [](int32_t key) { return ((uint32_t)key * 0x9E3779B1u) & (kSlots - 1); };
+  auto find = [&](int32_t key, uint32_t h) -> int32_t {  // its slot from h on, -1 if absent
+    for (int k = 0; k < kSlots; ++k) {
+      const int32_t x = S.keys[h];
+      if (x == key) return (int32_t)h;
+      if (x == -1) return -1;
+      h = (h + 1) & (kSlots - 1);
+    }
+    return -1;
+  };
+
+  uint64_t t_w = 0, t_r = 0;
+  uint32_t t_fill = 0, t_u = 0, t_l = 0, t_e = 0, t_v = 0;  // of one matrix and lane: below 2^32
+  int last_mat = -1;
+  auto flush = [&]() {
+    if (last_mat < 0) return;
+    unsigned long long* acc = acc_of(mats[last_mat]);
+    const uint64_t f = wave_sum_u50(t_fill), w = wave_sum_u50(t_w), r = wave_sum_u50(t_r), u = wave_sum_u50(t_u),
+                   l = wave_sum_u50(t_l), e = wave_sum_u50(t_e), v = wave_sum_u50(t_v);
+    if (lane == 0) {
+      if (f) atomicAdd(&acc[kAccFill], f);
+      if (w) atomicAdd(&acc[kAccW], w);
+      if (r) atomicAdd(&acc[kAccR], r);
+      if (u) atomicAdd(&acc[kAccNnzU], u);
+      if (l) atomicAdd(&acc[kAccNnzL], l);
+      if (e) atomicAdd(&acc[kAccLightExecEdges], e);
+      if (v) atomicAdd(&acc[kAccLightExecVerts], v);
+      if (u + l) atomicAdd(&acc[kAccLightExecOut], u + l);
+    }
+    t_fill = t_w = t_r = t_u = t_l = t_e = t_v = 0;
+  };
+
+  for (int32_t item = 2 * u0 + (int32_t)blockIdx.x; item < 2 * u1; item += (int32_t)gridDim.x) {
+    const int32_t u = item >> 1, d = item & 1;
+    const FrontUnit F = units[u];
+    if (F.mat != last_mat) {
+      flush();
+      last_mat = F.mat;
+    }
+    const MatDev& M = mats[F.mat];
+    const bool sym = M.sym != 0;
+    if (sym && d == 1) continue;
+    const int32_t c = F.c, lo = F.lo, done = d == 0 ? kStDone0 : kStDone1;
+    __syncthreads();  // the previous item's last reads
+    for (int i = tid; i < kSlots; i += T) S.keys[i] = -1;
+    if (tid == 0) {
+      s_ne = s_num = s_fail = s_near = s_sdeg = s_scnt = 0;
+      s_bits[0] = s_bits[1] = 0;
+      s_len[0] = s_len[1] = 0;
+      s_nact[0] = s_nact[1] = 0;
+    }
+    // ---- the unit's nodes, in ascending order: kScanPer vertices per thread and step ----
+    int32_t m = 0;
+    for (int32_t base = lo; base <= c; base += kScanPer * T) {
+      int32_t st[kScanPer];
+      uint32_t alive = 0;
+#pragma unroll
+      for (int j = 0; j < kScanPer; ++j) {
+        const int32_t v = base + kScanPer * tid + j;
+        st[j] = v <= c ? gload(M.st + v) : 1;
+      }
+#pragma unroll
+      for (int j = 0; j < kScanPer; ++j)
+        if ((st[j] & kStUnit) == 0 || (st[j] & kStRoot) != 0) alive |= 1u << j;
+      const uint32_t incl = wave_incl_scan_u32(__popc(alive));
+      if (lane == 63) s_wave[wave] = (int32_t)incl;
+      __syncthreads();
+      int32_t at = m, all = 0;
+#pragma unroll
+      for (int w = 0; w < T / 64; ++w) {
+        const int32_t x = s_wave[w];
+        at += w < wave ? x : 0;
+        all += x;
+      }
+      at += (int32_t)incl - __popc(alive);
+#pragma unroll
+      for (int j = 0; j < kScanPer; ++j)
+        if ((alive >> j) & 1u) {
+          if (at < nb) {
+            S.ids[at] = base + kScanPer * tid + j;
+            S.unit[at] = (st[j] & kStRoot) ? (st[j] & kStUnit) - 1 : (st[j] & done) ? -1 : -2;
+          }
+          ++at;
+        }
+      m += all;
+      __syncthreads();
+    }
+    if (m > nb) continue;  // uniform, and the same in the other direction: too many nodes
+    // ---- weights, and the rows' slots: all loads in flight together ----
+    int32_t wd = 0, wc = 0;
+    if (tid < m) {
+      const int32_t v = S.ids[tid], k = S.unit[tid];
+      if (k >= 0) {
+        wd = gload(M.uwt + 2 * (int64_t)k);
+        wc = gload(M.uwt + 2 * (int64_t)k + 1);
+      } else {
+        wd = gload(M.rowptr[0] + v + 1) - gload(M.rowptr[0] + v) + (M.dup_all ? gload(M.dup_all + v) : 0);
+        wc = 1;
+      }
+    }
+    int32_t e[kPer];
+    const int32_t* const ell = M.ell[d];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = k * kRows + (tid >> 4);
+      e[k] = kPad;
+      if (i < m && S.unit[i] < 0) e[k] = gload(ell + (int64_t)S.ids[i] * kEll + sl);
+    }
+    if (tid < m) {
+      const int32_t v = S.ids[tid];
+      uint32_t h = home(v);
+      while (atomicCAS(&S.keys[h], -1, v) != -1) h = (h + 1) & (kSlots - 1);  // every vertex once
+      S.vals[h] = (uint16_t)tid;
+      S.wdeg[tid] = wd;
+    }
+    if (wave * 64 < m) {
+      const uint32_t od = wave_or_u32((uint32_t)wd), oc = wave_or_u32((uint32_t)wc);
+      if (lane == 0) {
+        atomicOr(&s_bits[0], od);
+        atomicOr(&s_bits[1], oc);
+      }
+    }
+    // where the part of a long row beyond its slots starts in the CSR
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = k * kRows + (tid >> 4);
+      if (sl == kEll - 1 && i < m) S.tail[i] = e[k] <= -2 ? -(e[k] + 2) : -1;
+      if (e[k] < 0) e[k] = kPad;
+    }
+    // entries inside the unit: the vertex whose node they are now (a contracted vertex's root, level by
+    // level), all of a thread's at once. A row's entries keep their side of its diagonal.
+    for (bool more = true; more;) {
+      more = false;
+#pragma unroll
+      for (int k0 = 0; k0 < kPer; k0 += 8) {
+        int32_t st[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) st[k] = e[k0 + k] >= lo && e[k0 + k] <= c ? gload(M.st + e[k0 + k]) : 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if ((st[k] & kStUnit) != 0 && (st[k] & kStRoot) == 0) {
+            e[k0 + k] = gload(&units[(st[k] & kStUnit) - 1].c);
+            more = true;
+          }
+      }
+      more = __ballot(more) != 0;
+    }
+    __syncthreads();  // the hash holds the nodes
+    const int nbd = 32 - __clz((int)s_bits[0]), nbc = 32 - __clz((int)s_bits[1]);  // planes in use
+    if (wave * 64 < m) {
+      const int w0 = wave * 2 + lane;  // lanes 0 and 1: the wave's two words
+      const bool put = lane < 2 && w0 * 32 < m;
+      for (int q = 0; q < nbd; ++q) {
+        const uint64_t z = __ballot(((wd >> q) & 1) != 0);
+        if (put) S.pdeg[q * wi_max + w0] = (uint32_t)(z >> (32 * lane));
+      }
+      for (int q = 0; q < nbc; ++q) {
+        const uint64_t z = __ballot(((wc >> q) & 1) != 0);
+        if (put) S.pcnt[q * wi_max + w0] = (uint32_t)(z >> (32 * lane));
+      }
+      if (put) {
+        const int a = w0 * 32, z = min(m, a + 32) - 1;
+        S.run[w0] = S.ids[z] - S.ids[a] == z - a ? 1u : 0u;
+      }
+    }
+    // ---- the surface: every entry above c joins the hash. Entries become their slots. ----
+    auto add_ext = [&](int32_t x, uint32_t h) -> int32_t {  // its slot from h on, -1 once there are too many
+      if (__hip_atomic_load(&s_ne, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) > eb) return -1;
+      while (true) {
+        const int32_t old = atomicCAS(&S.keys[h], -1, x);
+        if (old == x) return (int32_t)h;
+        if (old == -1) {
+          atomicAdd(&s_ne, 1);
+          return (int32_t)h;
+        }
+        h = (h + 1) & (kSlots - 1);
+      }
+    };
+    // f(row, entry) for the entries that no slot holds: the lists of contracted nodes and the CSR tails of
+    // long rows, 16 lanes each
+    auto long_rows = [&](auto f) {
+      for (int i = tid >> 4; i < m; i += kRows) {
+        const int32_t k = S.unit[i], tail = S.tail[i];
+        if (k < 0 && tail < 0) continue;
+        const int32_t* list = M.adj[d] + tail;
+        int32_t len;
+        if (k >= 0) {
+          list = M.ulist + units[k].off + (int64_t)d * units[k].cap;
+          len = gload(M.ulen + 2 * (int64_t)k + d);
+        } else {
+          len = gload(M.rowptr[d] + S.ids[i] + 1) - tail;
+        }
+#pragma unroll 1
+        for (int32_t p = sl; p < len; p += 4 * kEll) {
+          int32_t x[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) x[q] = p + q * kEll < len ? gload(list + p + q * kEll) : kPad;
+#pragma unroll 1
+          for (int q = 0; q < 4; ++q) {
+            if (x[0] >= 0) f(i, x[0]);
+            x[0] = x[1];
+            x[1] = x[2];
+            x[2] = x[3];
+          }
+        }
+      }
+    };
+    // a thread's entries in turn, through the first register (the code of one instead of kPer)
+#pragma unroll 1
+    for (int k = 0; k < kPer; ++k) {
+      const int32_t x = e[0];
+      const int i = k * kRows + (tid >> 4);
+      const bool src = i < m && S.unit[i] == -2;
+      const uint64_t up = __ballot(x > (src ? S.ids[i] : INT32_MAX));  // entries above an unfinished row's diagonal
+      if (i < m && sl == 0) S.seed[i] = __popcll((up >> (lane & 48)) & 0xFFFFull);
+      int32_t slot = kPad;
+      if (x >= 0) {
+        const uint32_t h = home(x);
+        slot = S.keys[h] == x ? (int32_t)h : x > c ? add_ext(x, h) : find(x, h);
+        if (slot < 0 && x <= c) s_fail = 1;  // cannot happen: an alive vertex of T(c) is a node
+        ++t_e;
+      }
+#pragma unroll
+      for (int q = 0; q + 1 < kPer; ++q) e[q] = e[q + 1];
+      e[kPer - 1] = slot;
+    }
+    long_rows([&](int, int32_t x) {
+      if (x > c) add_ext(x, home(x));
+    });
+    __syncthreads();
+    const int32_t ne = s_ne;
+    bool fits = ne <= eb;  // uniform
+    // columns above c: the vertices within 128 of it by their distance (the window bits are shifts
+    // then), the others in any order
+    if (fits)
+      for (int i = tid; i < kSlots; i += T) {
+        const int32_t key = S.keys[i];
+        const bool far = key > c + 128;
+        const uint64_t mk = __ballot(far);
+        int at = 0;
+        if (lane == 0 && mk) at = atomicAdd(&s_num, (int)__popcll(mk));
+        at = __builtin_amdgcn_readfirstlane(at) + (int)rank_below(mk);
+        if (far) {
+          S.vals[i] = (uint16_t)at;
+          S.ext[at] = key;
+        } else if (key > c) {
+          atomicMax(&s_near, key - c);
+        }
+      }
+    __syncthreads();
+    const int nw = (s_near + 31) >> 5, nfar = s_num;
+    const int Wi = (m + 31) >> 5, Wn = Wi + nw, W = Wn + ((nfar + 31) >> 5);
+    fits = fits && W <= Z.width && m * W <= Z.words;
+    if (fits) {
+      if (tid == 0 && most) {
+        atomicMax(&most->nodes, m);
+        atomicMax(&most->ext, ne);
+        atomicMax(&most->words, m * W);
+        atomicMax(&most->width, W);
+      }
+      for (int i = tid; i < m * W; i += T) B[i] = 0;
+      __syncthreads();
+      // ---- the rows' bits ----
+      auto column = [&](int32_t key, int32_t x) {
+        return key <= c ? x : key <= c + 128 ? Wi * 32 + key - c - 1 : Wn * 32 + x;
+      };
+      auto put_bit = [&](int i, int32_t col) { atomicOr(&B[i * W + (col >> 5)], 1u << (col & 31)); };
+#pragma unroll
+      for (int k0 = 0; k0 < kPer; k0 += 8) {
+        int32_t key[8], x[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          key[k] = e[k0 + k] >= 0 ? S.keys[e[k0 + k]] : -1;
+          x[k] = e[k0 + k] >= 0 ? S.vals[e[k0 + k]] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (key[k] >= 0) put_bit((k0 + k) * kRows + (tid >> 4), column(key[k], x[k]));
+      }
+      long_rows([&](int i, int32_t x) {
+        if (S.unit[i] == -2 && x > S.ids[i]) atomicAdd(&S.seed[i], 1);
+        int32_t h = find(x, home(x));
+        while (h < 0) {  // contracted: its root's node
+          const int32_t st = x >= lo && x <= c ? gload(M.st + x) : 0;
+          if ((st & kStUnit) == 0 || (st & kStRoot) != 0) {
+            s_fail = 1;  // cannot happen
+            return;
+          }
+          x = gload(&units[(st & kStUnit) - 1].c);
+          h = find(x, home(x));
+        }
+        put_bit(i, column(S.keys[h], S.vals[h]));
+      });
+      __syncthreads();
+      // ---- elimination, 32 pivots at a time ----
+      const int gn = T / W, gi = tid / W, gl = tid - gi * W;  // rows side by side, this thread's row and word
+#pragma unroll 1
+      for (int kb = 0; kb < Wi; ++kb) {
+        const int p0 = kb * 32, np = min(32, m - p0);
+        for (int i = tid; i < np * W; i += T) S.P[i] = B[p0 * W + i];
+        if (p0 + wave * 64 < m) {
+          // the block's closure among its own columns (every wave that has rows, rows in lanes 0..31)
+          uint32_t x = lane < np ? B[(p0 + lane) * W + kb] : 0u;
+          const int i = p0 + tid;
+          uint32_t cf = i < m ? B[i * W + kb] : 0u;
+          const uint32_t below = lane < 32 ? (1u << lane) - 1u : 0u;
+          uint32_t lower = x & below;
+#pragma unroll
+          for (int q = 0; q < 31; ++q) {
+            const uint32_t xq = (uint32_t)__builtin_amdgcn_readlane((int)x, q);
+            x |= (uint32_t)((int32_t)(lower << (31 - q)) >> 31) & xq;
+            lower = x & below;
+          }
+          // a row's coefficients: the block's pivots it reaches; a pivot's, the pivots below it (every
+          // lane goes through the loop: a lane read needs its source lane active)
+#pragma unroll
+          for (int q = 0; q < 32; ++q)
+            cf |= (uint32_t)((int32_t)(cf << (31 - q)) >> 31) & (uint32_t)__builtin_amdgcn_readlane((int)x, q);
+          if (tid < 32) cf = lower;
+          const uint64_t some = __ballot(i < m && cf != 0);
+          int at = 0;
+          if (lane == 0 && some) at = atomicAdd(&s_nact[kb & 1], (int)__popcll(some));
+          at = __builtin_amdgcn_readfirstlane(at) + (int)rank_below(some);
+          if ((some >> lane) & 1ull) {
+            S.coef[at] = cf;
+            S.act[at] = (uint16_t)i;
+          }
+        }
+        __syncthreads();
+        const int na = s_nact[kb & 1];
+        if (tid == 0) s_nact[(kb + 1) & 1] = 0;
+        if (gi < gn && gi < na) {
+          uint32_t pr[32];
+#pragma unroll
+          for (int q = 0; q < 32; ++q) pr[q] = q < np ? S.P[q * W + gl] : 0u;
+#pragma unroll 1
+          for (int a = gi; a < na; a += 2 * gn) {  // two rows at a time
+            const bool two = a + gn < na;
+            const uint32_t c0 = S.coef[a], c1 = two ? S.coef[a + gn] : 0u;
+            uint32_t *const r0 = B + S.act[a] * W + gl, *const r1 = two ? B + S.act[a + gn] * W + gl : r0;
+            uint32_t x0 = *r0, x1 = *r1;
+#pragma unroll
+            for (int q = 0; q < 32; ++q) {
+              x0 |= (uint32_t)((int32_t)(c0 << (31 - q)) >> 31) & pr[q];
+              x1 |= (uint32_t)((int32_t)(c1 << (31 - q)) >> 31) & pr[q];
+            }
+            *r0 = x0;
+            if (two) *r1 = x1;
+          }
+        }
+        __syncthreads();
+      }
+      // ---- results of the unfinished rows, 16 lanes per row: lane w has word w of the nodes ----
+      const bool win_dir = d == 1 || sym;
+      const int fail = s_fail, chunk = M.chunk, n = M.n;
+      const int64_t* const list_ptr = M.list_ptr[d];
+      int32_t *const cnt = M.cnt[d], *const pool = M.pool[d];
+      uint32_t* const wins = M.win;
+      // the planes of this lane's word
+      constexpr int kPd = 14, kPc = 11;
+      uint32_t pd[kPd], pc[kPc];
+#pragma unroll
+      for (int q = 0; q < kPd; ++q) pd[q] = d == 0 && q < nbd && sl < Wi ? S.pdeg[q * wi_max + sl] : 0u;
+#pragma unroll
+      for (int q = 0; q < kPc; ++q) pc[q] = d == 0 && q < nbc && sl < Wi ? S.pcnt[q * wi_max + sl] : 0u;
+      const int first_id = sl < Wi ? S.ids[sl * 32] : c + 1 + 32 * (sl - Wi);  // the vertex of the word's bit 0
+      const bool run = sl >= Wi || S.run[sl] != 0;
+      // sums over a row's 16 lanes, in its last lane
+      auto sum16 = [&](uint32_t x) -> uint32_t {
+        x += dpp_u32<0x111>(x);
+        x += dpp_u32<0x112>(x);
+        x += dpp_u32<0x114>(x);
+        x += dpp_u32<0x118>(x);
+        return x;
+      };
+#pragma unroll 1
+      for (int i0 = 0; i0 < m; i0 += kRows) {
+        const int i = i0 + (tid >> 4);
+        const bool src = i < m && S.unit[i] == -2 && fail == 0;
+        if (__ballot(src) == 0) continue;
+        const int32_t v = src ? S.ids[i] : 0;
+        const uint32_t* const row = B + (src ? i : 0) * W;
+        uint32_t nu = 0, nr = 0, nd = 0;
+        uint32_t win[4] = {0, 0, 0, 0};
+        int64_t off = 0, end = 0;  // the row's place in the structure
+        if (list_ptr != nullptr && src) {
+          off = gload(list_ptr + v);
+          end = gload(list_ptr + v + 1);
+        }
+        for (int w = sl; src && w < W; w += kEll) {
+          const uint32_t x = row[w];
+          uint32_t up = x;
+          if (w < Wi) {
+            const int b = i - w * 32;  // the diagonal's bit: below 0 R's part is empty, above 31 U's
+            const uint32_t below = b <= 0 ? 0u : b >= 32 ? ~0u : (1u << b) - 1u;
+            const uint32_t diag = b >= 0 && b < 32 ? 1u << b : 0u;
+            const uint32_t r = x & below;
+            up = x & ~below & ~diag;
+            if (d == 0) {
+#pragma unroll
+              for (int q = 0; q < kPd; ++q) nd += (uint32_t)__popc(r & pd[q]) << q;
+#pragma unroll
+              for (int q = 0; q < kPc; ++q) nr += (uint32_t)__popc(r & pc[q]) << q;
+              for (int q = kPd; q < nbd; ++q) nd += (uint32_t)__popc(r & S.pdeg[q * wi_max + w]) << q;
+              for (int q = kPc; q < nbc; ++q) nr += (uint32_t)__popc(r & S.pcnt[q * wi_max + w]) << q;
+            }
+          }
+          nu += __popc(up);
+          if (win_dir && up != 0 && w < Wn) {
+            // rows v + 1 .. v + 128
+            const int32_t chunk_end = min(n, (v / chunk + 1) * chunk);
+            if (w == sl ? run : true) {
+              // consecutive vertices: the word's bits, shifted to their place in the window
+              const int t0 = (w == sl ? first_id : c + 1 + 32 * (w - Wi)) - v - 1;  // bit 0's place
+              const int room = chunk_end - v - 1;  // places of the window inside the chunk
+              if (t0 < 128) {
+                const uint64_t z = t0 >= 0 ? (uint64_t)up << (t0 & 31) : (uint64_t)(up >> -t0);
+                const int q0 = t0 >= 0 ? t0 >> 5 : 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                  uint32_t part = q == q0 ? (uint32_t)z : q == q0 + 1 ? (uint32_t)(z >> 32) : 0u;
+                  const int valid = room - 32 * q;
+                  if (valid < 32) part &= valid <= 0 ? 0u : (1u << valid) - 1u;
+                  win[q] |= part;
+                }
+              }
+            } else {
+              for (uint32_t y = up; y; y &= y - 1) {
+                const int32_t id = S.ids[w * 32 + __ffs(y) - 1];
+                if (id - v > 128) break;  // nodes ascend
+                window_bit(win, v, id, chunk_end);
+              }
+            }
+          }
+        }
+        const uint32_t U = sum16(nu);
+        if (d == 0) {
+          nr = sum16(nr);
+          nd = sum16(nd);
+        }
+        if (win_dir) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            uint32_t x = win[q];
+            x |= dpp_u32<0x111>(x);
+            x |= dpp_u32<0x112>(x);
+            x |= dpp_u32<0x114>(x);
+            x |= dpp_u32<0x118>(x);
+            win[q] = x;
+          }
+        }
+        if (src && sl == kEll - 1) {
+          gstore(cnt + v, (int32_t)U);
+          t_fill += U - (uint32_t)S.seed[i];
+          if (d == 0) {
+            t_w += (uint64_t)(uint32_t)S.wdeg[i] + nd;
+            t_r += nr;
+            t_u += U;
+            t_v += 1;
+          } else {
+            t_l += U;
+          }
+          if (win_dir) gstore_v4(wins + 4 * (int64_t)v, win[0], win[1], win[2], win[3]);
+        }
+        if (list_ptr != nullptr) {
+          const uint32_t all = __shfl(U, kEll - 1, kEll);
+          const bool ok = src && end - off == (int64_t)all;
+          if (src && !ok && sl == 0) atomicOr(&M.acc[kAccOverflow], 1ull);
+          int32_t* dst = pool + off;
+          for (int wb = 0; wb < W; wb += kEll) {
+            const int w = wb + sl;
+            uint32_t y = ok && w < W ? row[w] : 0u;
+            if (w < Wi) {
+              const int b = i - w * 32;
+              y &= b < 0 ? ~0u : b >= 31 ? 0u : ~1u << b;
+            }
+            const uint32_t cu = __popc(y);
+            const uint32_t incl = sum16(cu);
+            const uint32_t total = __shfl(incl, kEll - 1, kEll);
+            int32_t* p = dst + (incl - cu);
+            while (y) {
+              const int b = __ffs(y) - 1;
+              y &= y - 1;
+              gstore(p++, w < Wi ? S.ids[w * 32 + b] : w < Wn ? c + 1 + (w - Wi) * 32 + b : S.ext[(w - Wn) * 32 + b]);
+            }
+            dst += total;
+          }
+        }
+      }
+      if (fail && tid == 0) atomicOr(&M.acc[kAccScheduleError], 1ull);
+    }
+    // ---- contract the root, in the workgroup of the direction that ends last ----
+    // a wave's entries of a list, one reservation per wave
+    auto append = [&](int dd, bool some, int32_t v) {
+      const uint64_t mk = __ballot(some);
+      if (mk == 0) return;
+      int at = 0;
+      if (lane == 0) at = atomicAdd(&s_len[dd], (int)__popcll(mk));
+      at = __builtin_amdgcn_readfirstlane(at) + (int)rank_below(mk);
+      if (some) gstore(M.ulist + F.off + (int64_t)dd * F.cap + at, v);
+    };
+    const uint32_t* const last = B + (m - 1) * W;  // the root's row
+    if (fits)
+      for (int x0 = wave * 64; x0 < (W - Wi) * 32; x0 += T) {  // the root's entries above c
+        const int x = x0 + lane, w = Wi + (x >> 5);
+        const bool some = w < W && ((last[w] >> (x & 31)) & 1u) != 0;
+        append(d, some, !some ? 0 : w < Wn ? c + 1 + x : S.ext[x - 32 * nw]);
+      }
+    uint32_t r_own = fits && tid < m ? (last[tid >> 5] >> (tid & 31)) & 1u : 0u;
+    if (tid == m - 1) r_own = 0;
+    uint32_t r_other = sym ? r_own : 0u;
+    bool both = fits, other = false;
+    if (!sym) {
+      // published with the root's reached nodes and the length of its list so far
+      uint32_t* const msg = M.umsg + (int64_t)(2 * u + d) * kFrontMsg;
+      if (wave * 64 < m) {
+        const uint64_t b = __ballot(r_own != 0);
+        if (lane < 2) __hip_atomic_store(msg + wave * 2 + lane, (uint32_t)(b >> (32 * lane)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      if (tid == 0) {
+        __hip_atomic_store(msg + kFrontMsg - 1, (uint32_t)s_len[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      // The exchange goes through agent-scope accesses only, which no cache of an XCD keeps; they are
+      // acknowledged before the counter moves. (A release fence would write back the XCD's whole L2:
+      // 177 -> 432 us for the 2,048 workgroups of a level at 659,033 rows.)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) s_other = (int32_t)atomicAdd(M.uctr + u, fits ? 1u : 16u);
+      __syncthreads();
+      const int32_t before = s_other;
+      if (before == 0) continue;  // uniform: the other direction's workgroup contracts
+      other = before == 1;  // it fitted
+      both = fits && other;
+      const uint32_t* const om = M.umsg + (int64_t)(2 * u + 1 - d) * kFrontMsg;
+      if (tid < m)
+        r_other = (__hip_atomic_load(om + (tid >> 5), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> (tid & 31)) & 1u;
+      if (tid == 0)
+        s_len[1 - d] = (int32_t)__hip_atomic_load(om + kFrontMsg - 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+    }
+    if (!both) {
+      // one direction's rows are finished, or none's: nothing is contracted
+      const int32_t bits = fits ? done : other ? kStDone0 ^ kStDone1 ^ done : 0;
+      if (tid < m && S.unit[tid] < 0 && bits) gstore(M.st + S.ids[tid], gload(M.st + S.ids[tid]) | bits);
+      continue;  // uniform
+    }
+    if (wave * 64 < m) {
+      const bool on = tid < m, root = tid == m - 1, in = on && (root || (r_own && r_other));
+      const int32_t v = on ? S.ids[tid] : 0;
+      if (in) gstore(M.st + v, kStDone0 | kStDone1 | (root ? kStRoot : 0) | (u + 1));
+      else if (on && S.unit[tid] < 0) gstore(M.st + v, kStDone0 | kStDone1);
+      const uint32_t sd = wave_sum_u32(in ? (uint32_t)wd : 0u), sc = wave_sum_u32(in ? (uint32_t)wc : 0u);
+      if (lane == 0) {
+        atomicAdd(&s_sdeg, (int32_t)sd);
+        atomicAdd(&s_scnt, (int32_t)sc);
+      }
+      append(d, on && r_own && !in, v);
+      if (!sym) append(1 - d, on && r_other && !in, v);
+    }
+    __syncthreads();
+    if (tid < 2) gstore(M.ulen + 2 * (int64_t)u + tid, s_len[tid]);
+    if (tid == 0) {
+      gstore(M.uwt + 2 * (int64_t)u, s_sdeg);
+      gstore(M.uwt + 2 * (int64_t)u + 1, s_scnt);
+    }
+  }
+  flush();
+}
+
+// ------------------------------------------------------------------------------------------
+// The condensed graph: a node for every vertex that no unit's root stands for, in the vertices'
+// order, so that every rule of k_heavy (chaining, imports, cuts) holds on it as on the matrix. A
+// root's edges (its unit's list) do not fit one 16-entry row: they are held by list nodes right below
+// the root (leaves of up to 16 edges, then nodes over up to 16 leaves when there are more than 16),
+// which have no vertices and no degree of their own.
+// ------------------------------------------------------------------------------------------
+__device__ __forceinline__ int32_t cond_leaves(int32_t len) { return len <= kEll ? 0 : (len + kEll - 1) / kEll; }
+__device__ __forceinline__ int32_t cond_list_len(const MatDev& M, int d, int32_t k) {
+  return M.sym && d == 1 ? 0 : gload(M.ulen + 2 * (int64_t)k + d);
+}
+// list nodes of one direction: leaves, and nodes over them (a list has at most 4,096 entries)
+__device__ __forceinline__ int32_t cond_tree(int32_t len) {
+  const int32_t leaves = cond_leaves(len);
+  return leaves + cond_leaves(leaves);
+}
+__device__ __forceinline__ int32_t cond_list_nodes(const MatDev& M, int32_t k) {
+  return max(cond_tree(cond_list_len(M, 0, k)), cond_tree(cond_list_len(M, 1, k)));
+}
+// The nodes vertex v brings: itself, a root's list nodes and itself, or none (contracted).
+__device__ __forceinline__ int32_t cond_nodes(const MatDev& M, int32_t v) {
+  if (M.st == nullptr) return 0;
+  const int32_t st = gload(M.st + v);
+  if ((st & kStUnit) == 0) return 1;
+  return (st & kStRoot) ? 1 + cond_list_nodes(M, (st & kStUnit) - 1) : 0;
+}
+
+// Nodes per matrix, and after them unfinished rows of direction 0 (when a set is created: they size the condensed
+// graph and choose its launch).
 __global__ __launch_bounds__(256) void k_cond_sizes(const MatDev* __restrict__ mats, int nmats,
                                                     const int64_t* __restrict__ row_base, int64_t nrows,
                                                     unsigned long long* __restrict__ sizes) {
   for (int64_t g0 = (int64_t)blockIdx.x * blockDim.x; g0 < nrows; g0 += (int64_t)gridDim.x * blockDim.x) {
     const int64_t g = g0 + threadIdx.x;
     const int mb = nmats == 1 ? 0 : find_segment(row_base, nmats, min(g, nrows - 1));
-    const int32_t c = g < nrows ? cond_nodes(mats[mb], (int32_t)(g - row_base[mb])) : 0;
+    const MatDev& M = mats[mb];
+    const int32_t v = (int32_t)(g - row_base[mb]);
+    uint32_t c = 0, open = 0;
+    if (g < nrows && M.st != nullptr) {
+      const int32_t st = gload(M.st + v);
+      c = (uint32_t)cond_nodes(M, v);
+      open = (st & kStDone0) == 0 ? 1u : 0u;
+    }
     const int mb0 = __builtin_amdgcn_readfirstlane(mb);
     if (__ballot(mb != mb0) == 0) {
-      const uint32_t sum = wave_sum_u32((uint32_t)c);
+      const uint32_t sum = wave_sum_u32(c), sumo = wave_sum_u32(open);
       if (lane_id() == 0 && sum) atomicAdd(&sizes[mb0], (unsigned long long)sum);
-    } else if (c) {
-      atomicAdd(&sizes[mb], (unsigned long long)c);
+      if (lane_id() == 0 && sumo) atomicAdd(&sizes[nmats + mb0], (unsigned long long)sumo);
+    } else {
+      if (c) atomicAdd(&sizes[mb], (unsigned long long)c);
+      if (open) atomicAdd(&sizes[nmats + mb], (unsigned long long)open);
     }
   }
 }
@@ -1217,7 +2083,7 @@ __global__ __launch_bounds__(kScanBlock) void k_cond_apply(const MatDev* __restr
     carry += all;
     if (i >= nrows) continue;
     const MatDev& M = mats[mbs[k]];
-    if (M.vroot == nullptr) continue;
+    if (M.st == nullptr) continue;
     const int32_t v = (int32_t)(i - row_base[mbs[k]]);
     // the nodes were counted when the set was created; a run that counts others reports an error
     // (and stays inside the graph's buffers)
@@ -1231,10 +2097,11 @@ __global__ __launch_bounds__(kScanBlock) void k_cond_apply(const MatDev* __restr
     const int32_t id = (int32_t)(first - lo);
     gstore(M.nid + v, c[k] ? id + c[k] - 1 : -1);
     if (c[k]) gstore(orig + id + c[k] - 1, v);
-    if (gload(M.subtree + v) < 0) {
-      const int32_t r = gload(M.vroot + v);
-      gstore(M.root_id + r, id + c[k] - 1);
-      for (int32_t j = 0; j < c[k] - 1; ++j) gstore(orig + id + j, -(r + 1));
+    const int32_t st = gload(M.st + v);
+    if (st & kStRoot) {
+      const int32_t u = (st & kStUnit) - 1;
+      gstore(M.uid + u, id + c[k] - 1);
+      for (int32_t j = 0; j < c[k] - 1; ++j) gstore(orig + id + j, -(u + 1));
     }
   }
 }
@@ -1242,8 +2109,8 @@ __global__ __launch_bounds__(kScanBlock) void k_cond_apply(const MatDev* __restr
 // The condensed graph's rows, 16 lanes per node and direction (blocks [0, 2 ell_blocks), direction
 // 1 after direction 0), and its workgroup-path items, one wave per block of chain_block nodes (the
 // blocks after them). Items go by descending block (cblk_base / cblk_mat: the condensed matrices,
-// largest first), both directions of a block together; a block without an escalated row keeps
-// kNoItem. A block is cut at the node whose subtree is at least 1.5 times its predecessor's and at
+// largest first), both directions of a block together; a block without an unfinished row
+// keeps kNoItem. A block is cut at the node whose subtree is at least 1.5 times its predecessor's and at
 // least rows / cut_divisor vertices (the largest such): its rows before the cut are items of their
 // own, after the others.
 __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mats, const MatDev* __restrict__ cmats,
@@ -1264,18 +2131,19 @@ __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mat
     const int32_t K = C.chain_block;
     const int32_t b = (int32_t)(cblk_base[o + 1] - 1 - k);
     const int32_t r0 = b * K, r1 = (int32_t)min((int64_t)C.n, (int64_t)r0 + K);
-    uint64_t any0 = 0, any1 = 0;
+    uint64_t any0 = 0, any1 = 0;  // an unfinished row, per direction
     int32_t best = 0, cut = -1;
     for (int32_t j0 = r0; j0 < r1; j0 += 64) {
       const int32_t j = j0 + lane;
       const int32_t v = j < r1 ? gload(C.orig + j) : -1;
-      any0 |= __ballot(v >= 0 && gload(M.esc[0] + v) != 0);
-      any1 |= __ballot(v >= 0 && !M.sym && gload(M.esc[1] + v) != 0);
+      const int32_t st = v >= 0 ? gload(M.st + v) : -1;
+      any0 |= __ballot((st & kStDone0) == 0);
+      any1 |= __ballot((st & kStDone1) == 0);
       if (cut_divisor > 0) {
         const int32_t u = j > r0 && j < r1 ? gload(C.orig + j - 1) : -1;
         int32_t size = 0;
         if (v >= 0 && u >= 0) {
-          const int32_t sv = gload(M.subtree + v) & INT32_MAX, su = gload(M.subtree + u) & INT32_MAX;
+          const int32_t sv = gload(M.subtree + v), su = gload(M.subtree + u);
           if (2 * (int64_t)sv >= 3 * (int64_t)su && sv >= M.rows / cut_divisor) size = sv;
         }
         int32_t most = size;
@@ -1287,9 +2155,9 @@ __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mat
       }
     }
     if (lane < 2) {
-      const bool any = lane == 0 ? any0 != 0 : any1 != 0;
-      items[2 * k + lane] = any ? encode_item((uint32_t)mb, (uint32_t)lane, (uint32_t)(cut >= 0 ? cut : r0), 0u) : kNoItem;
-      if (any && cut >= 0) {
+      const bool some = lane == 0 ? any0 != 0 : any1 != 0 && !M.sym;
+      items[2 * k + lane] = some ? encode_item((uint32_t)mb, (uint32_t)lane, (uint32_t)(cut >= 0 ? cut : r0), 0u) : kNoItem;
+      if (some && cut >= 0) {
         const unsigned long long pos = atomicAdd(&ws->cut_count, 1ull);
         items[2 * nblk + (int64_t)pos] = encode_item((uint32_t)mb, (uint32_t)lane, (uint32_t)cut, 1u);
       }
@@ -1305,17 +2173,21 @@ __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mat
   const MatDev& C = cmats[mb];
   if (d == 1 && M.sym) return;
   const int32_t j = (int32_t)(g - cbase[mb]);
+  // the node of a vertex: its own, or that of the root it was contracted into (level by level)
   auto node_of = [&](int32_t m) -> int32_t {
-    const int32_t id = gload(M.nid + m);
-    return id >= 0 ? id : gload(M.root_id + gload(M.vroot + m));
+    int32_t id = gload(M.nid + m);
+    while (id < 0) {
+      m = gload(&M.units[(gload(M.st + m) & kStUnit) - 1].c);
+      id = gload(M.nid + m);
+    }
+    return id;
   };
   const int32_t v = gload(C.orig + j);
+  const int32_t st = v >= 0 ? gload(M.st + v) : 0;
   int32_t e = kPad;
   int32_t wt_deg = 0, wt_r = 0;
   uint8_t esc = 0;
-  const int32_t r = v >= 0 ? gload(M.vroot + v) : -(v + 1);
-  const bool root = v >= 0 && r >= 0 && gload(M.subtree + v) < 0 && cond_valid(M, r);
-  if (v >= 0 && !root) {
+  if (v >= 0 && (st & kStRoot) == 0) {
     e = gload(M.ell[d] + (int64_t)v * kEll + l);
     const bool tail = l == kEll - 1 && e <= -2;
     if (e >= 0) e = node_of(e);
@@ -1326,12 +2198,14 @@ __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mat
       gstore(const_cast<int32_t*>(C.rowptr[d]) + j + 1, pe);
     }
     if (d == 0 && M.dup_all) wt_deg = gload(M.dup_all + v);
-    esc = gload(M.esc[d] + v);
+    esc = (st & (d == 0 ? kStDone0 : kStDone1)) == 0 ? 1 : 0;
   } else {
-    // a contracted root, or one of its list nodes
-    const int32_t len = cond_list_len(M, d, r);
-    const int32_t leaves = cond_leaves(len), mids = cond_mids(leaves);
-    const int32_t first = gload(M.root_id + r) - cond_list_nodes(M, r);  // the root's first list node
+    // a unit's root, or one of its list nodes
+    const bool root = v >= 0;
+    const int32_t u = root ? (st & kStUnit) - 1 : -(v + 1);
+    const int32_t len = cond_list_len(M, d, u);
+    const int32_t leaves = cond_leaves(len), mids = cond_leaves(leaves);
+    const int32_t first = gload(M.uid + u) - cond_list_nodes(M, u);  // the root's first list node
     const int32_t i = j - first;
     int32_t at = -1, node = kPad;  // a list entry, or a list node
     if (root) {
@@ -1344,11 +2218,12 @@ __global__ __launch_bounds__(256) void k_cond_ell(const MatDev* __restrict__ mat
       const int32_t q = (i - leaves) * kEll + l;
       node = q < leaves ? first + q : kPad;
     }
-    e = at >= 0 ? node_of(gload(M.root_list[d] + (int64_t)r * M.list_cap + at)) : node;
+    e = node;
+    if (at >= 0) e = node_of(gload(M.ulist + M.units[u].off + (int64_t)d * M.units[u].cap + at));
     // its entries are not input entries, and a list node is no vertex
     const int32_t entries = __popcll((__ballot(e >= 0) >> (lane & 48)) & 0xFFFFull);
-    wt_deg = (root ? gload(M.root_w + r) : 0) - entries;
-    wt_r = root ? gload(M.root_r + r) - 1 : -1;
+    wt_deg = (root ? gload(M.uwt + 2 * (int64_t)u) : 0) - entries;
+    wt_r = root ? gload(M.uwt + 2 * (int64_t)u + 1) - 1 : -1;
   }
   gstore(const_cast<int32_t*>(C.ell[d]) + (int64_t)j * kEll + l, e);
   if (l == 0) {
@@ -2764,12 +3639,13 @@ hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, c
 }
 
 hipError_t launch_light(const MatDev* mats, int nmats, const int64_t* item_base, int64_t nitems, WorkState* ws, int grid,
-                        int bits, bool roots, hipStream_t s) {
-  const void* f = bits == kLightBitsBig
-                      ? (roots ? (const void*)k_light<kLightBitsBig, true> : (const void*)k_light<kLightBitsBig, false>)
-                      : (roots ? (const void*)k_light<kLightBits, true> : (const void*)k_light<kLightBits, false>);
-  void* args[] = {&mats, &nmats, &item_base, &nitems, &ws};
-  return hipLaunchKernel(f, dim3(grid), dim3(kLightWaves * 64), args, 0, s);
+                        int bits, hipStream_t s) {
+  if (bits == kLightBitsBig)
+    hipLaunchKernelGGL(k_light<kLightBitsBig>, dim3(grid), dim3(kLightWaves * 64), 0, s, mats, nmats, item_base, nitems,
+                       ws);
+  else
+    hipLaunchKernelGGL(k_light<kLightBits>, dim3(grid), dim3(kLightWaves * 64), 0, s, mats, nmats, item_base, nitems, ws);
+  return hipGetLastError();
 }
 
 hipError_t launch_heavy_order(const MatDev* mats, int64_t nblk_total, int nmats, const int64_t* blkq_base,
@@ -2874,10 +3750,42 @@ int heavy_cond_occupancy(int threads, size_t bytes) {
   return nb;
 }
 
+template <int kLevel>
+static int front_ready(const FrontSize& z) {
+  const void* f = (const void*)k_front<kLevel>;
+  const size_t bytes = FrontLds(nullptr, z, front_slots(kLevel)).bytes;
+  int occ = 0;
+  if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, f, kFrontThreads[kLevel], bytes) != hipSuccess)
+    return 0;
+  return occ;
+}
+int front_occupancy(int level, const FrontSize& z) {
+  if (level == 1) return front_ready<1>(z);
+  if (level == 2) return front_ready<2>(z);
+  int occ = 0;
+  return hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_front_leaf, kLeafWaves * 64, 0) == hipSuccess ? occ : 0;
+}
+
+hipError_t launch_front(int level, const FrontLaunch& L, const MatDev* mats, const FrontUnit* units, FrontSize* most,
+                        hipStream_t s) {
+  if (L.u1 <= L.u0) return hipSuccess;
+  // a wave per unit, or a workgroup per unit and direction
+  const int64_t work = level == 0 ? (L.u1 - L.u0 + kLeafWaves - 1) / kLeafWaves : 2 * (int64_t)(L.u1 - L.u0);
+  const dim3 g((unsigned)std::min<int64_t>(L.grid, work));
+  if (level == 0) {
+    hipLaunchKernelGGL(k_front_leaf, g, dim3(kLeafWaves * 64), 0, s, mats, units, L.u0, L.u1);
+    return hipGetLastError();
+  }
+  const size_t bytes = FrontLds(nullptr, L.size, front_slots(level)).bytes;
+  if (level == 1) hipLaunchKernelGGL(k_front<1>, g, dim3(kFrontThreads[1]), bytes, s, mats, units, L.u0, L.u1, L.size, most);
+  else hipLaunchKernelGGL(k_front<2>, g, dim3(kFrontThreads[2]), bytes, s, mats, units, L.u0, L.u1, L.size, most);
+  return hipGetLastError();
+}
+
 hipError_t launch_cond_sizes(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows,
                              unsigned long long* sizes, hipStream_t s) {
   const int g = grid_for(nrows, 256, 16384);
-  hipLaunchKernelGGL(k_cond_append, dim3(g), dim3(256), 0, s, mats, nmats, row_base, nrows);
   hipLaunchKernelGGL(k_cond_sizes, dim3(g), dim3(256), 0, s, mats, nmats, row_base, nrows, sizes);
   return hipGetLastError();
 }
@@ -2888,7 +3796,6 @@ hipError_t launch_condense(const MatDev* mats, const MatDev* cmats, int nmats, c
                            WorkState* ws, uint64_t* items, hipStream_t s) {
   const int64_t per = (int64_t)kScanBlock * kScanItems;
   const int64_t nb = (nrows + per - 1) / per;
-  hipLaunchKernelGGL(k_cond_append, dim3(grid_for(nrows, 256, 16384)), dim3(256), 0, s, mats, nmats, row_base, nrows);
   hipLaunchKernelGGL(k_cond_reduce, dim3((unsigned)nb), dim3(kScanBlock), 0, s, mats, nmats, row_base, nrows, block_sums);
   hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScanBlock), 0, s, block_sums, nb, total);
   hipLaunchKernelGGL(k_cond_apply, dim3((unsigned)nb), dim3(kScanBlock), 0, s, mats, cmats, nmats, row_base, nrows,
@@ -2936,8 +3843,8 @@ int heavy_occupancy(int threads, size_t lds_bytes, bool hbm_bitmap) {
 int light_occupancy(int bits) {
   int nb = 0;
   const hipError_t e = bits == kLightBitsBig
-                           ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBitsBig, true>, kLightWaves * 64, 0)
-                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBits, true>, kLightWaves * 64, 0);
+                           ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBitsBig>, kLightWaves * 64, 0)
+                           : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_light<kLightBits>, kLightWaves * 64, 0);
   return e == hipSuccess ? nb : 0;
 }
 }  // namespace gsofa
