@@ -395,21 +395,14 @@ int gsofa_structure_get(gsofa_plan* p, int64_t* u_rowptr, int32_t* u_col, int64_
     int rc = gsofa_sync(p);
     if (rc != GSOFA_OK) return rc;
   }
-  std::vector<int64_t> up, lp;
-  std::vector<int32_t> ui, li;
-  int rc = p->set.read_structure(0, up, ui, lp, li);
+  const std::vector<int64_t>*up, *lp;
+  int rc = p->set.structure_offsets(0, up, lp);
   if (rc != GSOFA_OK) return rc;
-  std::memcpy(u_rowptr, up.data(), up.size() * 8);
-  std::memcpy(l_colptr, lp.data(), lp.size() * 8);
-  if (!ui.empty()) {
-    if (!u_col) return fail(GSOFA_ERR_INVALID_ARG, "u_col is null");
-    std::memcpy(u_col, ui.data(), ui.size() * 4);
-  }
-  if (!li.empty()) {
-    if (!l_row) return fail(GSOFA_ERR_INVALID_ARG, "l_row is null");
-    std::memcpy(l_row, li.data(), li.size() * 4);
-  }
-  return GSOFA_OK;
+  std::memcpy(u_rowptr, up->data(), up->size() * 8);
+  std::memcpy(l_colptr, lp->data(), lp->size() * 8);
+  if (up->back() && !u_col) return fail(GSOFA_ERR_INVALID_ARG, "u_col is null");
+  if (lp->back() && !l_row) return fail(GSOFA_ERR_INVALID_ARG, "l_row is null");
+  return p->set.read_structure(0, u_col, l_row);
 }
 
 int gsofa_plan_stage_timing(gsofa_plan* p, int32_t on) {
@@ -508,7 +501,14 @@ static int plan_structure_cache(gsofa_plan* p) {
   if (!p->set.structure_ready()) return fail(GSOFA_ERR_STATE, "structure not produced: enable it and run first");
   int rc = plan_flags(p, p->sn_flags);
   if (rc != GSOFA_OK) return rc;
-  rc = p->set.read_structure(0, p->sn_up, p->sn_ui, p->sn_lp, p->sn_li);
+  const std::vector<int64_t>*up, *lp;
+  rc = p->set.structure_offsets(0, up, lp);
+  if (rc != GSOFA_OK) return rc;
+  p->sn_up = *up;
+  p->sn_lp = *lp;
+  p->sn_ui.resize((size_t)up->back());
+  p->sn_li.resize((size_t)lp->back());
+  rc = p->set.read_structure(0, p->sn_ui.data(), p->sn_li.data());
   if (rc != GSOFA_OK) return rc;
   p->sn_cached = true;
   return GSOFA_OK;

@@ -493,6 +493,8 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
   if (q.n_top > 0) GSOFA_SEQ(hipStreamWaitEvent(s, q.join, 0), "hipStreamWaitEvent(join)");
   if (q.mirror_any) GSOFA_SEQ(launch_mirror(q.mats, q.nmats, q.blk_base, q.nblocks_sup, s), "k_mirror");
   GSOFA_SEQ(launch_supernodes(q.mats, q.nmats, q.blk_base, q.nblocks_sup, s), "k_supernodes");
+  if (q.sort_lists)
+    GSOFA_SEQ(launch_sort_lists(q.mats, q.nmats, q.row_base, q.nrows, q.n_max, q.cus, q.sort_region, s), "sort the structure");
   if (q.sum_totals) GSOFA_SEQ(launch_totals(q.mats, q.nmats, s), "k_totals");
   if (ev) GSOFA_SEQ(hipEventRecord(ev[4], s), "hipEventRecord");
 #undef GSOFA_SEQ
@@ -510,6 +512,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   DeviceInfo info;
   GSOFA_TRY(device_info(opt.device, info));
   GSOFA_HIP(hipSetDevice(opt.device), "hipSetDevice");
+  cus_ = info.cus;
 
   ns_.resize(nmats_);
   row_base_h_.assign(nmats_ + 1, 0);
@@ -1106,6 +1109,9 @@ Sequence DeviceSet::sequence() const {
   q.cn_max = cn_max_;
   q.cut_divisor = cut_divisor_;
   q.cond_zero = cond_zero_;
+  q.sort_lists = pools_sized_ ? 1 : 0;
+  q.cus = cus_;
+  q.sort_region = sort_region_;
   q.units = units_;
   for (int l = 0; l < kFrontLevels; ++l) q.fronts[l] = fronts_[l];
   q.citems = citems_;
@@ -1206,6 +1212,8 @@ int DeviceSet::size_pools_from_counts() {
     GSOFA_TRY(alloc(list_ptr_l_, (size_t)nptr, "L offsets"));
     GSOFA_TRY(alloc(pool_u_, (size_t)pool_base_u_[nmats_], "U structure"));
     GSOFA_TRY(alloc(pool_l_, (size_t)pool_base_l_[nmats_], "L structure"));
+    const int64_t words = sort_region_words(n_max_, cus_);
+    if (words > 0) GSOFA_TRY(alloc(sort_region_, (size_t)words, "structure sort bitmaps"));
   }
   GSOFA_TRY(upload(list_ptr_u_, up.data(), up.size() * 8, "upload U offsets"));
   GSOFA_TRY(upload(list_ptr_l_, lp.data(), lp.size() * 8, "upload L offsets"));
@@ -1228,27 +1236,24 @@ int DeviceSet::size_pools_from_counts() {
   return GSOFA_OK;
 }
 
-int DeviceSet::read_structure(int mat, std::vector<int64_t>& u_ptr, std::vector<int32_t>& u_idx,
-                              std::vector<int64_t>& l_ptr, std::vector<int32_t>& l_idx) {
+int DeviceSet::structure_offsets(int mat, const std::vector<int64_t>*& u_ptr, const std::vector<int64_t>*& l_ptr) const {
   if (!pools_sized_) return fail(GSOFA_ERR_STATE, "structure was not produced (structure option off)");
   if (mat < 0 || mat >= nmats_) return fail(GSOFA_ERR_INVALID_ARG, "matrix index");
-  u_ptr = u_ptr_h_[mat];
-  l_ptr = l_ptr_h_[mat];
-  const int64_t nu = u_ptr.back(), nl = l_ptr.back();
-  u_idx.resize((size_t)nu);
-  l_idx.resize((size_t)nl);
-  if (nu) GSOFA_TRY(download(u_idx.data(), pool_u_ + pool_base_u_[mat], (size_t)nu * 4, "read U"));
-  if (mirror_[mat]) {
-    l_idx = u_idx;  // L's column v is U's row v
-  } else if (nl) {
-    GSOFA_TRY(download(l_idx.data(), pool_l_ + pool_base_l_[mat], (size_t)nl * 4, "read L"));
-  }
-  const int32_t n = ns_[mat];
-  for (int32_t v = 0; v < n; ++v) {
-    std::sort(u_idx.begin() + u_ptr[v], u_idx.begin() + u_ptr[v + 1]);
-    std::sort(l_idx.begin() + l_ptr[v], l_idx.begin() + l_ptr[v + 1]);
-  }
+  u_ptr = &u_ptr_h_[mat];
+  l_ptr = &l_ptr_h_[mat];
   return GSOFA_OK;
+}
+
+int DeviceSet::read_structure(int mat, int32_t* u_idx, int32_t* l_idx) {
+  const std::vector<int64_t>*up, *lp;
+  GSOFA_TRY(structure_offsets(mat, up, lp));
+  const size_t nu = (size_t)up->back(), nl = (size_t)lp->back();
+  GSOFA_TRY(download(u_idx, pool_u_ + pool_base_u_[mat], nu * 4, "read U"));
+  if (mirror_[mat]) {
+    if (nl) std::memcpy(l_idx, u_idx, nl * 4);  // L's column v is U's row v
+    return GSOFA_OK;
+  }
+  return download(l_idx, pool_l_ + pool_base_l_[mat], nl * 4, "read L");
 }
 
 }  // namespace gsofa

@@ -168,6 +168,9 @@ struct Sequence {
   // (launch_condense) and the workgroup path on them. nplain: the others, which the wave path and the
   // plain workgroup path run (none: no such launches).
   int ncond = 0, nplain = 0;
+  // The explicit structure's lists are to be sorted (sort_region_words at sort_region).
+  int sort_lists = 0, cus = 0;
+  uint32_t* sort_region = nullptr;
   MatDev* cmats = nullptr;
   int64_t *cbase = nullptr, *cblk_base = nullptr;
   int32_t* cblk_mat = nullptr;
@@ -225,9 +228,10 @@ class DeviceSet {
   // After the stream completed: read per-matrix totals.
   int read_results(std::vector<MatResult>& out);
   int read_counts(int mat, int32_t* cnt_u, int32_t* cnt_l, uint8_t* sup_flag, int32_t* nzu);
-  // Structure of matrix `mat`: strict U rows (CSR) and strict L columns (CSC), sorted.
-  int read_structure(int mat, std::vector<int64_t>& u_ptr, std::vector<int32_t>& u_idx, std::vector<int64_t>& l_ptr,
-                     std::vector<int32_t>& l_idx);
+  // Structure of matrix `mat`: strict U rows (CSR) and strict L columns (CSC), sorted. The offsets, and
+  // the entries into arrays of their size (straight from the device: they are sorted there).
+  int structure_offsets(int mat, const std::vector<int64_t>*& u_ptr, const std::vector<int64_t>*& l_ptr) const;
+  int read_structure(int mat, int32_t* u_idx, int32_t* l_idx);
   bool structure_ready() const { return pools_sized_; }
   int size_pools_from_counts();
   int nmats() const { return nmats_; }
@@ -300,6 +304,8 @@ class DeviceSet {
   // fronts and condensed graphs (Sequence)
   int create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree, const DeviceInfo& info);
   int ncond_ = 0, nplain_ = 0;
+  int cus_ = 0;
+  uint32_t* sort_region_ = nullptr;  // bitmaps of the structure's sort (patterns beyond its LDS)
   std::vector<uint8_t> cond_;         // per matrix: it runs by fronts and a condensed graph
   std::vector<MatDev> cmats_h_;
   MatDev* cmats_d_ = nullptr;

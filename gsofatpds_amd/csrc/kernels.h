@@ -245,6 +245,11 @@ hipError_t launch_top_setup(const MatDev* mats, int nmats, WorkState* ws, int64_
 // a mirrored matrix's fill and workgroup-path entries doubled, nnz_L = nnz_U.
 hipError_t launch_totals(const MatDev* mats, int nmats, hipStream_t s);
 // Mirrored matrices: L counts = U counts (one thread per row, blocks as for launch_supernodes).
+// The explicit structure's lists into ascending order (after the traversals, and by the offsets: every
+// matrix has lists). region: sort_region_words words (0: none needed).
+int64_t sort_region_words(int64_t n_max, int cus);
+hipError_t launch_sort_lists(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows, int64_t n_max, int cus,
+                             uint32_t* region, hipStream_t s);
 hipError_t launch_mirror(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 hipError_t launch_supernodes(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 constexpr int kLightThreads = 256;
