@@ -216,8 +216,10 @@ class DeviceSet {
   DeviceSet& operator=(const DeviceSet&) = delete;
   ~DeviceSet();
   // alloc_stream != null: stream-ordered allocations and uploads on that stream (no device-wide
-  // synchronisation; used by the server), freed on the same stream by the destructor.
-  int create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream = nullptr);
+  // synchronisation; used by the server), freed on the same stream by the destructor; from `pool`, or
+  // the device's default pool.
+  int create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream = nullptr,
+             hipMemPool_t pool = nullptr);
   // Device bytes create() will allocate for these matrices (admission by footprint).
   static int64_t footprint(const std::vector<const Prepared*>& mats, const Options& opt, int64_t* out_bytes);
   // Enqueue the whole symbolic factorisation on `s` (no host synchronisation, no allocation,
@@ -321,6 +323,7 @@ class DeviceSet {
   LaunchConfig ccfg_;
   std::vector<void*> owned_;
   hipStream_t alloc_stream_ = nullptr;
+  hipMemPool_t alloc_pool_ = nullptr;
   // the early launch of top-separator items (top_separator_rows)
   int64_t n_top_ = 0;
   int top_grid_ = 0;
