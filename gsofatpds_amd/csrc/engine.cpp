@@ -352,7 +352,8 @@ int configure_launch(int32_t n_max, int64_t nrows, bool paired_any, const Option
   // lds holds the window's rows already; the static part is the rest
   if (lds + kHeavyLdsReserve > info.lds_per_block)
     return fail(GSOFA_ERR_CAPACITY, "heavy LDS request exceeds the device limit");
-  const hipError_t e = heavy_set_lds_limit(threads, lds, out.hbm_bitmap);
+  hipError_t e = heavy_set_lds_limit(threads, lds, out.hbm_bitmap);
+  if (e == hipSuccess && paired_any) e = heavy_set_lds_limit(kCheckpointThreads, lds, out.hbm_bitmap);
   if (e != hipSuccess) return fail(GSOFA_ERR_HIP, std::string("hipFuncSetAttribute(k_heavy): ") + hipGetErrorString(e));
   const int occ = heavy_occupancy(threads, lds, out.hbm_bitmap);
   if (occ <= 0) return fail(GSOFA_ERR_CAPACITY, "k_heavy cannot be resident with this LDS size");
@@ -469,7 +470,7 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
   } while (0)
   if (ev) GSOFA_SEQ(hipEventRecord(ev[0], s), "hipEventRecord");
   GSOFA_SEQ(launch_clear_run(q.acc, (int64_t)q.nmats * kAccSlots * acc_copies(q.nmats), reinterpret_cast<unsigned long long*>(q.ws),
-                             q.ncond > 0 ? 8 : 4, reinterpret_cast<int32_t*>(q.esc), q.esc_words,
+                             q.ck_total > 0 ? 12 : q.ncond > 0 ? 8 : 4, reinterpret_cast<int32_t*>(q.esc), q.esc_words,
                              reinterpret_cast<int32_t*>(q.blk_flag), 2 * q.nblk_total, q.bucket, q.nb_max,
                              q.cond_zero, q.cond_words, s),
             "clear the run's state");
@@ -482,7 +483,7 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
     GSOFA_SEQ(launch_top_setup(q.mats, q.nmats, q.ws_top, q.n_top, q.side), "early launch set-up");
     if (q.top_ev) GSOFA_SEQ(hipEventRecord(q.top_ev[0], q.side), "hipEventRecord");
     GSOFA_SEQ(launch_heavy(q.cfg.heavy_threads, q.top_grid, q.mats, q.ws_top, q.top_items, q.cfg.bw_max, q.cfg.qcap,
-                           q.n_max, q.paired_any, q.spill_top, nullptr, q.cfg.ucap, kAccTopExecEdges, q.side),
+                           q.n_max, q.paired_any, q.spill_top, nullptr, q.cfg.ucap, kAccTopExecEdges, 0, q.side),
               "k_heavy (early launch)");
     if (q.top_ev) GSOFA_SEQ(hipEventRecord(q.top_ev[1], q.side), "hipEventRecord");
     GSOFA_SEQ(hipEventRecord(q.join, q.side), "hipEventRecord(join)");
@@ -500,9 +501,14 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
                                q.block_sums, q.total, q.ws, q.heavy_items, s),
             "workgroup-path queue");
   if (ev) GSOFA_SEQ(hipEventRecord(ev[2], s), "hipEventRecord");
+  if (q.ck_total > 0)
+    GSOFA_SEQ(launch_heavy(kCheckpointThreads, (int)std::min<int64_t>(q.cfg.heavy_grid, q.ck_total), q.mats, q.ws_ck,
+                           nullptr, q.cfg.bw_max, q.cfg.qcap, q.n_max, q.paired_any, q.spill, q.hbm_bm, q.cfg.ucap,
+                           kAccHeavyExecEdges, q.ck_total, s),
+              "k_heavy (checkpoints)");
   if (q.nplain > 0)
     GSOFA_SEQ(launch_heavy(q.cfg.heavy_threads, q.cfg.heavy_grid, q.mats, q.ws, q.heavy_items, q.cfg.bw_max, q.cfg.qcap,
-                           q.n_max, q.paired_any, q.spill, q.hbm_bm, q.cfg.ucap, kAccHeavyExecEdges, s),
+                           q.n_max, q.paired_any, q.spill, q.hbm_bm, q.cfg.ucap, kAccHeavyExecEdges, 0, s),
               "k_heavy");
   if (q.ncond > 0)
     GSOFA_SEQ(launch_heavy_cond(q.ccfg.heavy_threads, q.ccfg.heavy_grid, q.cmats, q.ws_cond, q.citems, q.ccfg.bw_max,
@@ -552,7 +558,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     blk_base_h_[b + 1] = blk_base_h_[b] + ((int64_t)P.n + 255) / 256;
     any_dup |= !P.dup_u.empty();
     mirror_[b] = mirrored(P, opt) ? 1 : 0;
-    paired_any_ |= (!mirror_[b] && pair_directions(P, opt.pair_directions)) ? 1 : 0;
+    paired_any_ |= pair_directions(P, opt.pair_directions) ? 1 : 0;
   }
   mirror_any_ = 0;
   mirror_all_ = 1;
@@ -667,7 +673,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   row_base_d_ = item_base_d_ + (nmats_ + 1);
   blk_base_d_ = row_base_d_ + (nmats_ + 1);
   blkq_base_d_ = blk_base_d_ + (nmats_ + 1);
-  GSOFA_TRY(alloc(ws_, 2, "work state"));  // the second: the early launch's, or the condensed graphs'
+  GSOFA_TRY(alloc(ws_, 3, "work state"));  // the second: the early launch's, or the condensed graphs'; the third: the checkpoints'
   GSOFA_TRY(alloc(heavy_items_, 2 * (nblk_total_ + ncut), "escalation list"));
   if (ncut > 0) {
     GSOFA_TRY(alloc(cut_, (size_t)nblk_total_, "block cuts"));
@@ -822,6 +828,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     GSOFA_TRY(alloc(spill_, (size_t)(heavy_grid_ + top_grid_) * (size_t)heavy_region_ints(n_max_, paired_any_ != 0),
                     "heavy spill regions"));
     if (hbm_bitmap_) GSOFA_TRY(alloc(hbm_bm_, (size_t)heavy_grid_ * (size_t)bw_max_, "heavy bitmaps"));
+    GSOFA_TRY(create_checkpoints(mats));
   } else {
     heavy_threads_ = ccfg_.heavy_threads;
     heavy_grid_ = ccfg_.heavy_grid;
@@ -829,6 +836,37 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     qcap_ = ccfg_.qcap;
     opt_.chain_block = ccfg_.chain_block;
   }
+  return GSOFA_OK;
+}
+
+// Checkpoints of the unstructured matrices. Not with the early launch, whose items are fixed.
+int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats) {
+  if (n_top_ > 0) return GSOFA_OK;
+  auto none = [&](int b) {
+    return ns_[b] < kCheckpointRows || (!cond_.empty() && cond_[b]) || !pair_directions(*mats[b], opt_.pair_directions);
+  };
+  int64_t words = 0, count = 0;
+  for (int b = 0; b < nmats_; ++b) {
+    if (none(b)) continue;
+    words += checkpoint_words(ns_[b]);
+    ++count;
+  }
+  if (count == 0) return GSOFA_OK;
+  GSOFA_TRY(alloc(ck_bits_, (size_t)words, "checkpoint bitmaps"));
+  GSOFA_TRY(alloc(ck_facts_, (size_t)(8 * kCheckpoints * count), "checkpoint facts"));
+  int64_t at = 0, k = 0;
+  for (int b = 0; b < nmats_; ++b) {
+    if (none(b)) continue;
+    MatDev& M = mats_h_[b];
+    M.ck_step = checkpoint_step(ns_[b]);
+    M.ck_n = checkpoint_count(ns_[b]);
+    M.ck_bits = ck_bits_ + at;
+    M.ck_facts = ck_facts_ + 8 * kCheckpoints * k++;
+    at += checkpoint_words(ns_[b]);
+  }
+  ck_total_ = 2 * kCheckpoints * nmats_;
+  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(checkpoints)");
   return GSOFA_OK;
 }
 
@@ -1057,6 +1095,7 @@ int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Opt
   b += 4 * (heavy_grid + kTopMaxItems) * heavy_region_ints(nmax, paired);  // spill (and the early launch's)
   if (place_bitmaps_in_hbm(nmax, opt, info)) b += 4 * (int64_t)cus * (((int64_t)nmax + 31) / 32);  // one per CU
   if (dup) b += 8 * nrows;
+  b += (int64_t)kCheckpoints * (nrows / 4 + 8 * (int64_t)mats.size() + 64 * (int64_t)mats.size());  // checkpoints
   // subtree sizes; fronts (states, nodes, units of at least kFrontMean rows on average with their lists)
   // and the condensed graphs (at most kCondMaxShare + 0.1 of the rows)
   if (opt.pre_escalate != -1)
@@ -1135,6 +1174,8 @@ Sequence DeviceSet::sequence() const {
   q.cn_max = cn_max_;
   q.cut_divisor = cut_divisor_;
   q.cond_zero = cond_zero_;
+  q.ck_total = ck_total_;
+  q.ws_ck = ws_ + 2;
   q.sort_lists = pools_sized_ ? 1 : 0;
   q.cus = cus_;
   q.sort_region = sort_region_;

@@ -168,6 +168,9 @@ struct Sequence {
   // (launch_condense) and the workgroup path on them. nplain: the others, which the wave path and the
   // plain workgroup path run (none: no such launches).
   int ncond = 0, nplain = 0;
+  // Workgroup-path launch of the checkpoints before the main one (0: none), with its work counter.
+  int32_t ck_total = 0;
+  WorkState* ws_ck = nullptr;
   // The explicit structure's lists are to be sorted (sort_region_words at sort_region).
   int sort_lists = 0, cus = 0;
   uint32_t* sort_region = nullptr;
@@ -304,9 +307,13 @@ class DeviceSet {
   std::vector<std::vector<int64_t>> u_ptr_h_, l_ptr_h_;    // host copies of the offsets
   std::vector<MatDev> mats_h_;
   // fronts and condensed graphs (Sequence)
+  int create_checkpoints(const std::vector<const Prepared*>& mats);
   int create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree, const DeviceInfo& info);
   int ncond_ = 0, nplain_ = 0;
   int cus_ = 0;
+  int32_t ck_total_ = 0;
+  uint32_t* ck_bits_ = nullptr;           // checkpoints' bitmaps and facts of the whole set
+  unsigned long long* ck_facts_ = nullptr;
   uint32_t* sort_region_ = nullptr;  // bitmaps of the structure's sort (patterns beyond its LDS)
   std::vector<uint8_t> cond_;         // per matrix: it runs by fronts and a condensed graph
   std::vector<MatDev> cmats_h_;

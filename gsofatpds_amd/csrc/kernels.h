@@ -85,7 +85,7 @@ struct MatDev {
   unsigned long long* acc;        // kAccSlots: copy 0
   int64_t acc_stride;             // slots from one copy to the next
   int32_t acc_mask;               // copies - 1
-  uint8_t* esc[2];                // n: 1 where the wave path escalated the source
+  uint8_t* esc[2];                // n: 1 where the wave path escalated the source, kEscDone a finished checkpoint
   uint32_t* blk_flag[2];          // ceil(n / chain_block): 1 where the block has an escalated row
   const int32_t* split;           // ceil(n / chain_block): a row where the block is cut into two
                                   // workgroup-path items, or -1 (null: no block is cut)
@@ -101,6 +101,11 @@ struct MatDev {
   const int32_t* subtree;         // n: elimination-subtree sizes of A + A^T (null: none)
   int32_t pre_size;               // a row whose subtree exceeds this escalates without a
                                   // wave-path attempt (its reached set would exceed the limit)
+  // Checkpoints of the workgroup path (kernels.hip): rows (j + 1) ck_step - 1, j < ck_n (0: none), and
+  // per direction and checkpoint its bitmap (n bits, in whole words) and 4 words of facts
+  int32_t ck_n, ck_step;
+  uint32_t* ck_bits;
+  unsigned long long* ck_facts;
   // Fronts and the condensed graph (kernels.hip, k_front); st is null for a matrix without them.
   int32_t* st;                    // n: state of the vertex (kSt*)
   int32_t* nid;                   // n: the vertex's node in the condensed graph, -1 if contracted
@@ -134,7 +139,8 @@ struct WorkState {
 // chain_block rows (v is the block's first row, or a cut; e > 0 only for the early launch's
 // items), or, with bit 63, the rows of v's block before v.
 constexpr int kItemExtraMax = 1023;
-constexpr uint64_t kNoItem = ~0ull;  // condensed graphs: a block without an escalated row
+constexpr uint64_t kNoItem = ~0ull;  // a condensed graph's block without an escalated row, no checkpoint
+constexpr uint8_t kEscDone = 2;
 __host__ __device__ inline uint64_t encode_item(uint32_t mat, uint32_t dir, uint32_t row, uint32_t before_cut,
                                                 uint32_t extra = 0) {
   return ((uint64_t)before_cut << 63) | ((uint64_t)extra << 53) | ((uint64_t)mat << 33) | ((uint64_t)dir << 32) |
@@ -193,13 +199,24 @@ constexpr int64_t heavy_region_ints(int64_t n_max, bool paired_any) {
   const int64_t nbw = (n_max + 31) / 32;
   return paired_any ? 4 * n_max + 2 * kSavedRing * nbw : 3 * n_max + nbw;
 }
+// Checkpoints (kernels.hip, checkpoint_item): at most kCheckpoints per matrix, kCheckpointStep rows or
+// more apart, in matrices of kCheckpointRows rows or more (smaller ones hardly escalate a row: the wave
+// path's limit is 256 vertices). Edges that a 20,011-row matrix executes with 16 / 32 / 64 / 128 of them,
+// theirs included: 33 / 25 / 25 / 24 million.
+constexpr int32_t kCheckpoints = 32, kCheckpointStep = 16, kCheckpointRows = 512;
+constexpr int kCheckpointThreads = 1024;
+inline int32_t checkpoint_step(int32_t n) { return n / (kCheckpoints + 1) > kCheckpointStep ? n / (kCheckpoints + 1) : kCheckpointStep; }
+inline int32_t checkpoint_count(int32_t n) { return (n - 1) / checkpoint_step(n) < kCheckpoints ? (n - 1) / checkpoint_step(n) : kCheckpoints; }
+// Words of a matrix's checkpoint bitmaps.
+inline int64_t checkpoint_words(int32_t n) { return (int64_t)2 * checkpoint_count(n) * ((n + 31) / 32); }
 // hbm_bitmaps: null (bitmaps in LDS), or grid * bw_max words, one bitmap per workgroup
 // (1024-thread workgroups only).
 // exec_slot: the accumulator slot of the launch's first executed-work counter (kAccHeavyExecEdges,
 // or kAccTopExecEdges for the early launch).
+// ck_total > 0: the launch of the checkpoints (kCheckpoints * 2 * matrices; heavy_items is not read).
 hipError_t launch_heavy(int threads, int grid, const MatDev* mats, WorkState* ws, const uint64_t* heavy_items,
                         int32_t bw_max, int32_t qcap, int64_t n_max, int32_t paired_any, int32_t* spill,
-                        uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, hipStream_t s);
+                        uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, int32_t ck_total, hipStream_t s);
 // What a front level holds per unit: alive nodes (its rows not yet contracted), surface vertices (rows
 // above the unit that its rows hold), words of one direction's bit matrix and of one of its rows. A
 // unit with more is left to the next level or to k_heavy.

@@ -2291,6 +2291,26 @@ __device__ __forceinline__ void flush_totals(const MatDev* mats, int mb, Totals&
   t = Totals{};
 }
 
+// Checkpoints (unstructured matrices): every ck_step-th row, run by a launch of its own (ck_total > 0)
+// before the others, which keeps X_c of both directions. The first row of an item, which has no
+// predecessor here, then imports the X_c of a checkpoint c below the item as soon as it is known to
+// reach c: when it reaches some v <= c in the other direction's X_c (v reaches c through vertices below
+// c). Vertices of X_c between c and the row are reached too, and join the next level, for their own
+// neighbours may be new. Bound by the latency of the levels: without checkpoints the first rows were
+// 231 of the 248 million edges that a 20,011-row matrix took (27,622 escalated rows, items of 9). With
+// them its workgroup path takes 28 million edges and 820 us (117 of them the checkpoints', by
+// 1,024-thread workgroups: 240 with 256), before 1,270; a batch of 24 with 12 such members 3,730 us,
+// before 6,030. Structured patterns keep to their own rows: in a 4,096-row band in natural order the
+// rows between a checkpoint and an item are a filament of as many levels, while s - 1 is three away
+// (720 us with checkpoints, 540 without).
+__device__ __forceinline__ uint64_t checkpoint_item(const MatDev* mats, int32_t idx, int32_t total) {
+  const int32_t per = total / kCheckpoints;  // both directions of every matrix, the last checkpoints first
+  const int32_t j = kCheckpoints - 1 - idx / per, b = (idx % per) >> 1, d = idx & 1;
+  const MatDev& M = mats[b];
+  if (j >= M.ck_n || (d == 1 && M.sym)) return kNoItem;
+  return encode_item((uint32_t)b, (uint32_t)d, (uint32_t)((j + 1) * M.ck_step - 1), 0u);
+}
+
 // One workgroup per item = a block of chain_block consecutive rows; it traverses the block's
 // escalated rows in increasing order and reuses the previous row's reached set
 // X_{s-1} = {s-1} + R_{s-1} + U_{s-1} whenever s-1 is in R_s, because then R_{s-1}, s-1 and
@@ -2331,13 +2351,15 @@ constexpr int kSoloNarrow = 4;  // levels of at most this many vertices: 16 lane
 constexpr int kSoloMax = 64;    // levels of at most this many vertices: the leader alone
 
 enum : int32_t { kCmdDone = 0, kCmdClear = 1, kCmdCopyIn = 2, kCmdImport = 3, kCmdSave = 4, kCmdWide = 5 };
+constexpr int kCkSlot = -2;  // in place of a saved bitmap's slot: the item's checkpoint
+constexpr int kCkFacts = kSavedRing + 1, kCkTried = 4;
 
 // The leader's request: written by its lane 0 before a barrier, read by every thread after it.
 struct HeavyCtl {
   int32_t cmd, d, src, level;
   int32_t imported, slot;  // slot: the saved bitmap to copy in, OR in or write
   uint32_t ubase;          // carried U-list entries (the row's new entries follow them)
-  int32_t has_prev;
+  int32_t has_prev, t;     // an import is pending, of X_t
 };
 
 // The leader's state between its turns, in LDS: a turn starts from it and writes it back before
@@ -2353,7 +2375,8 @@ struct LeaderState {
   uint32_t ubase, gap;
 };
 
-// kPairedAny: some matrix of the set runs paired items (otherwise that code is compiled out).
+// kPairedAny: some matrix of the set is unstructured: it runs paired items (unless it is mirrored) and
+// has checkpoints (otherwise that code is compiled out).
 // kCond: the matrices are condensed graphs (below k_cond_ell): rows are nodes, results go to the
 // nodes' vertices, and the items before a cut come first.
 template <int kThreads, bool kPairedAny, bool kHbmBitmap, bool kCond = false>
@@ -2363,7 +2386,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                                                     int32_t bw_max, int32_t qcap, int64_t n_max,
                                                     int32_t* __restrict__ spill_all,
                                                     uint32_t* __restrict__ hbm_bitmaps, int32_t ucap,
-                                                    int32_t exec_slot) {
+                                                    int32_t exec_slot, int32_t ck_total) {
   static_assert(kEll == 16, "the window scan maps one row to 16 lanes");
   static_assert(!kCond || (!kPairedAny && !kHbmBitmap), "condensed graphs run plain items with LDS bitmaps");
   extern __shared__ uint32_t dyn[];
@@ -2447,22 +2470,26 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   };
   // Per direction: the rows of the saved bitmaps (index k < kSavedRing) and the last row
   // traversed (index kSavedRing). Written by the leader when it finishes a row.
-  __shared__ RowFacts s_facts[2][kSavedRing + 1];
+  // Then the item's checkpoint (index kCkFacts).
+  __shared__ RowFacts s_facts[2][kSavedRing + 2];
+  __shared__ int32_t s_ck;  // its row, or -1
 
   int last_mat = -1;
   __shared__ Totals tot;  // thread 0 only (in LDS: keeps the registers for the traversal)
   if (tid == 0) tot = Totals{};
 
   const unsigned long long ncut = kCond ? ws->cut_count : 0ull;
-  const unsigned long long total = ws->heavy_count + ncut;
+  const bool ck_run = kPairedAny && ck_total > 0;  // the items are the checkpoints, single rows
+  const unsigned long long total = ck_run ? (unsigned long long)ck_total : ws->heavy_count + ncut;
   while (true) {
     if (tid == 0) s_idx = atomicAdd(&ws->heavy_next, 1ull);
     bsync();
     const unsigned long long idx = s_idx;
     if (idx >= total) break;
     // condensed: the items before a cut (after the others in the array) go first
-    const uint64_t item = heavy_items[kCond ? (idx < ncut ? total - ncut + idx : idx - ncut) : idx];
-    if (kCond && item == kNoItem) {
+    const uint64_t item = ck_run ? checkpoint_item(mats, (int32_t)idx, ck_total)
+                                 : heavy_items[kCond ? (idx < ncut ? total - ncut + idx : idx - ncut) : idx];
+    if (item == kNoItem) {
       bsync();
       continue;
     }
@@ -2471,7 +2498,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     const int32_t v = (int32_t)(item & 0xffffffffu);
     const int before_cut = (int)(item >> 63);
     const MatDev& M = mats[mb];
-    const bool paired = kPairedAny && M.paired != 0;
+    const bool paired = kPairedAny && M.paired != 0 && !ck_run;
     const int ndir = paired ? 2 : 1;
     const int32_t n = M.n;
     const int32_t rows = kCond ? M.rows : n;  // rows of the matrix (chunks, window bits)
@@ -2480,7 +2507,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
     // v (decoded from the item alone: a table read here costs the traversal registers)
     const int32_t vb = v - v % M.chain_block;
     const int32_t r0 = before_cut ? vb : v;
-    const int32_t r1 = before_cut ? v : (int32_t)min((int64_t)n, vb + (int64_t)M.chain_block * (1 + (int32_t)((item >> 53) & 0x3ffu)));
+    const int32_t r1 = ck_run ? v + 1 : before_cut ? v : (int32_t)min((int64_t)n, vb + (int64_t)M.chain_block * (1 + (int32_t)((item >> 53) & 0x3ffu)));
     const bool want_list = M.list_ptr[0] != nullptr;  // both directions or neither
 
     // The leader's state of this item, per direction (index = direction; a plain item uses its
@@ -2494,7 +2521,40 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         for (int k = 0; k < kSavedRing; ++k) s_ls.sv[dd][k] = -1;
       }
       s_ls.lds_row = s_ls.lds_dir = -1;
+      s_ck = -1;
+      if (kPairedAny && M.ck_n > 0 && !ck_run) {
+        // One of the last checkpoints below the item, of those that the checkpoints' launch ran in both
+        // directions: the last whose reach in the direction that reaches less is over half of the best's
+        // (a row outside the large strongly connected part is of no use).
+        const int32_t last = min(r0 / M.ck_step, M.ck_n) - 1;
+        unsigned long long r[kCkTried];
+        unsigned long long most = 0;
+#pragma unroll
+        for (int k = 0; k < kCkTried; ++k) {
+          const int32_t j = last - k, c = (j + 1) * M.ck_step - 1;
+          r[k] = 0;
+          const int32_t o = M.sym ? 0 : 1;  // mirrored: the other direction is the same
+          if (j >= 0 && gload(M.esc[0] + c) == kEscDone && gload(M.esc[o] + c) == kEscDone)
+            r[k] = min(gload(M.ck_facts + 4 * j + 2), gload(M.ck_facts + 4 * (o * M.ck_n + j) + 2));
+          most = max(most, r[k]);
+        }
+        int32_t j = -1;
+#pragma unroll
+        for (int k = kCkTried - 1; k >= 0; --k)
+          if (r[k] > 0 && 2 * r[k] >= most) j = last - k;
+        if (j >= 0) {
+          s_ck = (j + 1) * M.ck_step - 1;
+          for (int dd = 0; dd < (M.sym ? 1 : 2); ++dd) {
+            const unsigned long long* const f = M.ck_facts + 4 * (dd * M.ck_n + j);
+            s_facts[dd][kCkFacts] = RowFacts{gload(f), gload(f + 1), gload(f + 2), 0u, 0u};
+          }
+        }
+      }
     }
+    // the checkpoint's bitmap of a direction
+    auto ck_bits = [&](int dd, int32_t c) -> uint32_t* {
+      return M.ck_bits + ((int64_t)dd * M.ck_n + (c + 1) / M.ck_step - 1) * bw;
+    };
 #define GSOFA_SV(dd, k) (s_ls.sv[dd][k])
 #define GSOFA_SLOT(dd, r)                                                             \
   ((r) < 0 ? -1                                                                       \
@@ -2513,7 +2573,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         int32_t* const stash = (kPairedAny && dd) ? stash1 : stash0;
         int32_t esc_v = 0;
         int64_t lp_v = 0;
-        if (tid < np) esc_v = gload(M.esc[dd] + w0 + tid);
+        if (tid < np) {  // (a checkpoint is finished already)
+          esc_v = gload(M.esc[dd] + w0 + tid);
+          if (kPairedAny && esc_v == kEscDone) esc_v = 0;
+        }
         if constexpr (kCond) {
           if (tid < np) {
             const int32_t o = gload(M.orig + w0 + tid);
@@ -2706,7 +2769,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               // the saved bitmap of the chain base, or of t1 for a late import
               tslot = chained ? GSOFA_SLOT(d, t) : slot1;
               // late import (of X_{s-1} only, when s-1 is reached)
+              // (or of the checkpoint's)
               has_prev = !chained && t1 == src - 1 && slot1 >= 0;
+              if (kPairedAny && !chained && !has_prev && s_ck >= 0) {
+                has_prev = true;
+                t = s_ck;
+                fi = kCkFacts;
+                slot1 = kCkSlot;
+              }
               if (lane == 0) {
                 s_cnt[0] = 1;
                 s_cnt[1] = 0;
@@ -2782,7 +2852,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             }
             if (phase == 2) {
               // ---- BFS levels: the leader alone while a level has at most kSoloMax vertices ----
-              const uint32_t* const gprev = gslot(d, slot1 < 0 ? 0 : slot1);  // saved X_{s-1}
+              const bool ck = kPairedAny && slot1 == kCkSlot;
+              const uint32_t* const gprev = ck ? ck_bits(d, t) : gslot(d, slot1 < 0 ? 0 : slot1);  // saved X_t
+              const uint32_t* const gother = ck ? ck_bits(M.sym ? d : 1 - d, t) : gprev;
+              const int32_t imp_at = has_prev && !ck ? src - 1 : -2;  // reaching it imports X_{s-1}
               const int32_t* const stash = (kPairedAny && d) ? stash1 : stash0;
               while (true) {
                 const int32_t ncur = s_cnt[level % 3];
@@ -2813,7 +2886,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     const uint32_t bit = 1u << (m & 31);
                     if (!fresh_check || (bm_get(m >> 5) & bit) == 0) isnew = (atomicOr(&bm[m >> 5], bit) & bit) == 0;
                   }
-                  if (isnew && has_prev && m == src - 1) {  // import X_{src-1} instead of expanding it
+                  if (isnew && m == imp_at) {  // import X_{src-1} instead of expanding it
                     imp = true;
                     isnew = false;
                   }
@@ -2836,8 +2909,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   if (vi < ncur) v = seed ? src : qget(cur_l, cur_g, qcap, vi);
                   int32_t m = kPad;
                   if (v >= 0) m = seed ? stash[li * kEll + sl] : gload(M.ell[d] + (int64_t)v * kEll + sl);
-                  const bool chk = v >= 0 && !seed && has_prev;
+                  const bool chk = v >= 0 && !seed && has_prev && v <= t;
                   const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
+                  // v <= t in the other direction's X_t: v, and so src, reaches the checkpoint
+                  if (ck && chk && !imported) imp = ((gload(gother + (v >> 5)) >> (v & 31)) & 1u) != 0;
                   uint32_t dupv = 0, rv = 1;
                   node_weight(M, d, sl == 0 ? v : -1, dupv, rv);
                   const bool in_prev = chk && ((pword >> (v & 31)) & 1u) != 0;
@@ -2893,8 +2968,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 } else {
                   // wide pass of the leader: one vertex per lane, its ELL slots 8 at a time
                   int32_t v = lane < ncur ? qget(cur_l, cur_g, qcap, lane) : -1;
-                  const bool chk = v >= 0 && has_prev;
+                  const bool chk = v >= 0 && has_prev && v <= t;
                   const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
+                  if (ck && chk && !imported) imp = ((gload(gother + (v >> 5)) >> (v & 31)) & 1u) != 0;
                   RowCursor rc;
                   load_row(M, d, v, rc);
                   uint32_t dupv = 0, rv = 1;
@@ -2924,7 +3000,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                       if (m >= 0) {
                         ++deg;
                         if (((old[j] >> (m & 31)) & 1u) == 0) {
-                          if (has_prev && m == src - 1) imp = true;
+                          if (m == imp_at) imp = true;
                           else if (m < src) mask_r |= 1u << (h + j);
                           else if (m > src) mask_u |= 1u << (h + j);
                         }
@@ -3067,8 +3143,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               // this one (only an import can use it).
               // Mirrored: never (s+1 chains from the LDS copy when it can, and otherwise s is not in
               // R_{s+1}, so no import takes X_s).
-              const bool save = paired ? next_in
-                                       : !M.sym && next_in && s_esc[d][li + 1] != 0 && s_hold[d][li + 1] == 0;
+              const bool save = ck_run   ? true
+                                : paired ? next_in
+                                         : !M.sym && next_in && s_esc[d][li + 1] != 0 && s_hold[d][li + 1] == 0;
               const int wslot = s_ls.wp[d];  // the ring slot this row's save takes
               const int32_t vsrc = kCond ? s_orig[li] : src;
               if (kCond && (d == 1 || M.sym)) {
@@ -3088,6 +3165,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 const RowFacts f{wr, dg0, rr, U, want_list ? kept : 0u};
                 s_facts[d][kSavedRing] = f;
                 if (save) s_facts[d][wslot] = f;
+                if (ck_run) {
+                  unsigned long long* const out = M.ck_facts + 4 * (d * M.ck_n + (src + 1) / M.ck_step - 1);
+                  gstore(out, (unsigned long long)f.wr);
+                  gstore(out + 1, (unsigned long long)f.deg);
+                  gstore(out + 2, (unsigned long long)f.r);
+                  gstore(M.esc[d] + src, kEscDone);
+                }
                 if (mb != last_mat) {
                   flush_totals(mats, last_mat, tot, exec_slot);
                   last_mat = mb;
@@ -3194,6 +3278,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             s_ctl.slot = cslot;
             s_ctl.ubase = ubase;
             s_ctl.has_prev = has_prev ? 1 : 0;
+            s_ctl.t = t;
           }
         }
         bsync();
@@ -3232,7 +3317,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           }
           bsync();
         } else if (ctl.cmd == kCmdSave) {
-          uint32_t* const gout = gslot(cd, ctl.slot);
+          uint32_t* const gout = ck_run ? ck_bits(cd, csrc) : gslot(cd, ctl.slot);
           for (int32_t w = tid; w < bw; w += kThreads) gstore(gout + w, bm_get(w));
           bsync();
         } else {
@@ -3243,13 +3328,18 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             if ((int32_t)i < ucap) ul[i] = v;
             else gstore(ustage + ((int32_t)i - ucap), v);
           };
-          const uint32_t* const gprev = gslot(cd, ctl.slot < 0 ? 0 : ctl.slot);  // saved X_{s-1}
+          const bool cck = kPairedAny && ctl.slot == kCkSlot;
+          const int32_t ct = ctl.t;
+          const uint32_t* const gprev = cck ? ck_bits(cd, ct) : gslot(cd, ctl.slot < 0 ? 0 : ctl.slot);  // saved X_t
+          const uint32_t* const gother = cck ? ck_bits(M.sym ? cd : 1 - cd, ct) : gprev;
           const bool chas_prev = ctl.has_prev != 0;
+          const int32_t cimp_at = chas_prev && !cck ? csrc - 1 : -2;
           const uint32_t cubase = ctl.ubase;
           bool cimported = ctl.imported != 0;
           uint32_t p_w = 0, p_wo = 0, p_x = 0, p_r = 0, p_ro = 0, p_un = 0;
-          // OR in X_{src-1}; its new bits above src are U entries of src, the rest is R_{src-1}
-          auto import_prev = [&]() {
+          // OR in X_t; its new bits above src are U entries of src, those between t and src join the
+          // level to come (they are reached, but their own neighbours are not covered), the rest is R_t
+          auto import_prev = [&](int lev) {
             for (int32_t wb = 0; wb < bw; wb += kThreads * kImportBatch) {
               uint32_t pw[kImportBatch];
 #pragma unroll
@@ -3271,6 +3361,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   }
                   nb = pw[q] & ~cw;
                   const int32_t b0 = w * 32;
+                  if (cck) {
+                    uint32_t g = b0 < csrc && b0 + 31 > ct ? nb : 0u;
+                    if (b0 <= ct) g &= ~0u << (ct - b0 < 31 ? ct - b0 + 1 : 0);
+                    if (b0 + 31 >= csrc) g &= (1u << ((csrc - b0) & 31)) - 1u;
+                    if (g) {
+                      int32_t at = atomicAdd(&s_cnt[lev % 3], (int32_t)__popc(g));
+                      for (; g; g &= g - 1) qput((lev & 1) ? ql1 : ql0, (lev & 1) ? qg1 : qg0, qcap, at++, w * 32 + __ffs(g) - 1);
+                    }
+                  }
                   if (b0 + 31 <= csrc) nb = 0;
                   else if (b0 <= csrc) nb &= ~0u << ((csrc - b0) & 31) << 1;  // keep bits above src
                 }
@@ -3295,7 +3394,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           };
           int clevel = ctl.level;
           if (ctl.cmd == kCmdImport) {
-            import_prev();
+            import_prev(clevel);
             cimported = true;
             bsync();
           } else {
@@ -3315,8 +3414,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 const int32_t e = base + tid;
                 int32_t v = e < ncur ? qget(cur_l, cur_g, qcap, e) : -1;
                 // issued together: membership in the saved X_{s-1}, the row, its duplicate surplus
-                const bool chk = v >= 0 && chas_prev;
+                const bool chk = v >= 0 && chas_prev && v <= ct;
                 const uint32_t pword = chk ? gload(gprev + (v >> 5)) : 0u;
+                if (cck && chk && !cimported && ((gload(gother + (v >> 5)) >> (v & 31)) & 1u) != 0) s_import = 1;
                 RowCursor rc;
                 load_row(CM, cd, v, rc);
                 uint32_t dupv = 0, rv = 1;
@@ -3349,7 +3449,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     if (m >= 0) {
                       ++deg;
                       if (((old[j] >> (m & 31)) & 1u) == 0) {
-                        if (chas_prev && m == csrc - 1) s_import = 1;  // import X_{src-1} instead of expanding it
+                        if (m == cimp_at) s_import = 1;  // import X_{src-1} instead of expanding it
                         else if (m < csrc) mask_r |= 1u << (h + j);
                         else if (m > csrc) mask_u |= 1u << (h + j);
                       }
@@ -3396,7 +3496,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     uint32_t* wp = &bm[m >> 5];
                     if ((bm_get(m >> 5) & bit) == 0) isnew = (atomicOr(wp, bit) & bit) == 0;
                   }
-                  if (isnew && chas_prev && m == csrc - 1) {
+                  if (isnew && m == cimp_at) {
                     s_import = 1;
                     isnew = false;
                   }
@@ -3441,7 +3541,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               bsync();
               // s_import only ever goes 0 -> 1 during a row, and only in claims before this barrier
               if (!cimported && s_import != 0) {
-                import_prev();
+                import_prev(clevel + 1);
                 cimported = true;
                 bsync();
               }
@@ -3912,11 +4012,11 @@ hipError_t heavy_set_lds_limit(int threads, size_t bytes, bool hbm_bitmap) {
 
 hipError_t launch_heavy(int threads, int grid, const MatDev* mats, WorkState* ws, const uint64_t* heavy_items,
                         int32_t bw_max, int32_t qcap, int64_t n_max, int32_t paired_any, int32_t* spill,
-                        uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, hipStream_t s) {
+                        uint32_t* hbm_bitmaps, int32_t ucap, int32_t exec_slot, int32_t ck_total, hipStream_t s) {
   const bool hbm = hbm_bitmaps != nullptr;
   const void* f = heavy_fn(threads, paired_any != 0, hbm);
   if (!f) return hipErrorInvalidValue;
-  void* args[] = {&mats, &ws, &heavy_items, &bw_max, &qcap, &n_max, &spill, &hbm_bitmaps, &ucap, &exec_slot};
+  void* args[] = {&mats, &ws, &heavy_items, &bw_max, &qcap, &n_max, &spill, &hbm_bitmaps, &ucap, &exec_slot, &ck_total};
   return hipLaunchKernel(f, dim3(grid), dim3(threads), args,
                          heavy_lds_bytes(bw_max, qcap, hbm, ucap, paired_any != 0), s);
 }
@@ -3926,8 +4026,8 @@ hipError_t launch_heavy_cond(int threads, int grid, const MatDev* cmats, WorkSta
   const void* f = heavy_cond_fn(threads);
   if (!f) return hipErrorInvalidValue;
   uint32_t* none = nullptr;
-  int32_t exec_slot = kAccHeavyExecEdges;
-  void* args[] = {&cmats, &ws, &items, &bw_max, &qcap, &n_max, &spill, &none, &ucap, &exec_slot};
+  int32_t exec_slot = kAccHeavyExecEdges, ck_total = 0;
+  void* args[] = {&cmats, &ws, &items, &bw_max, &qcap, &n_max, &spill, &none, &ucap, &exec_slot, &ck_total};
   return hipLaunchKernel(f, dim3(grid), dim3(threads), args, heavy_lds_bytes(bw_max, qcap, false, ucap, false), s);
 }
 

@@ -80,7 +80,9 @@ struct Layout {
   uint8_t* esc;
   int32_t* bucket;
   int32_t* spill;
-  size_t fixed_bytes, spill_bytes;
+  uint32_t* ck_bits;  // checkpoints, where the scratch holds them too
+  unsigned long long* ck_facts;
+  size_t fixed_bytes, spill_bytes, ck_bytes;
 };
 
 void carve_layout(unsigned char* base, int32_t n, int64_t nnz, int64_t nblk, int32_t nb_max, int64_t esc_words,
@@ -102,7 +104,7 @@ void carve_layout(unsigned char* base, int32_t n, int64_t nnz, int64_t nblk, int
   L.acc = c.take<unsigned long long>(kAccSlots * acc_copies(1));
   L.mats = c.take<MatDev>(1);
   L.bases = c.take<int64_t>(8);
-  L.ws = c.take<WorkState>(1);
+  L.ws = c.take<WorkState>(3);  // the wave path's and k_heavy's; none; the checkpoints'
   L.heavy_items = c.take<uint64_t>(2 * nblk);
   L.esc = c.take<uint8_t>(esc_words * 4);
   L.blk_flag = c.take<uint32_t>(2 * nblk);
@@ -110,6 +112,9 @@ void carve_layout(unsigned char* base, int32_t n, int64_t nnz, int64_t nblk, int
   L.fixed_bytes = c.off;
   L.spill = c.take<int32_t>(heavy_grid * region_ints);
   L.spill_bytes = c.off - L.fixed_bytes;
+  L.ck_bits = c.take<uint32_t>(checkpoint_words(n));
+  L.ck_facts = c.take<unsigned long long>(8 * kCheckpoints);
+  L.ck_bytes = c.off - L.fixed_bytes - L.spill_bytes;
 }
 
 // Sets *bad unless rowptr/adj is a CSR pattern of n rows whose rows are strictly increasing
@@ -302,6 +307,13 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   M.subtree = nullptr;  // no pre-escalation: the subtree sizes need the host's elimination tree
   M.pre_size = INT32_MAX;
   M.rows = n;
+  const bool ck = paired && n >= kCheckpointRows && L.fixed_bytes + L.spill_bytes + L.ck_bytes <= kScratchBytes;
+  if (ck) {
+    M.ck_n = checkpoint_count(n);
+    M.ck_step = checkpoint_step(n);
+    M.ck_bits = L.ck_bits;
+    M.ck_facts = L.ck_facts;
+  }
   M.light_limit = n <= kLightSmallRows ? kLightLimitSmall
                   : cfg.light_bits == kLightBitsBig ? kLightLimitBig : kLightLimitMax;
   const int64_t bases[8] = {0, nitems, 0, n, 0, nblocks_sup, 0, nblk};
@@ -350,6 +362,8 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   q.blk_flag = L.blk_flag;
   q.hbm_bm = nullptr;
   q.nplain = 1;
+  q.ck_total = ck ? 2 * kCheckpoints : 0;
+  q.ws_ck = L.ws + 2;
   q.sum_totals = 0;  // k_noalloc_totals does
   q.mats = L.mats;
   q.item_base = item_base;
