@@ -2349,6 +2349,7 @@ __device__ __forceinline__ uint64_t checkpoint_item(const MatDev* mats, int32_t 
 constexpr int kImportBatch = 8;
 constexpr int kSoloNarrow = 4;  // levels of at most this many vertices: 16 lanes per vertex
 constexpr int kSoloMax = 64;    // levels of at most this many vertices: the leader alone
+constexpr int kSoloChain = 16;  // levels of at most this many vertices follow one another without the general passes
 
 enum : int32_t { kCmdDone = 0, kCmdClear = 1, kCmdCopyIn = 2, kCmdImport = 3, kCmdSave = 4, kCmdWide = 5 };
 constexpr int kCkSlot = -2;  // in place of a saved bitmap's slot: the item's checkpoint
@@ -2857,8 +2858,111 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               const uint32_t* const gother = ck ? ck_bits(M.sym ? d : 1 - d, t) : gprev;
               const int32_t imp_at = has_prev && !ck ? src - 1 : -2;  // reaching it imports X_{s-1}
               const int32_t* const stash = (kPairedAny && d) ? stash1 : stash0;
+              const int32_t* const ell = M.ell[d];
+              bool chain = !want_list && qcap >= kSoloChain * kEll;
+              const bool weigh = d == 0 && (kCond || M.dup_all != nullptr);
               while (true) {
-                const int32_t ncur = s_cnt[level % 3];
+                int32_t ncur = s_cnt[level % 3];
+                if (chain && level > 0 && ncur > 0 && ncur <= kSoloChain) {
+                  // A chain of levels of at most kSoloChain vertices: lane = (vertex, ELL slot), four
+                  // vertices to a round, the rounds' reads and claims in flight together. Left for the
+                  // passes below (queue and counts as they need them) when a level is wider, holds a
+                  // row with a CSR tail, or reaches an import. Bound by one row read, one claim and one
+                  // queue write and read, each waiting for the one before: 2,400 cycles a level, where
+                  // the passes below, whose reads wait for one another too, take 4,600. 16 vertices:
+                  // with 32 a level's instructions outweigh what it saves (band of 4,096 rows 585 us;
+                  // 500 with 16, 540 without; 20,011 unstructured rows 715, 820 without).
+                  const int vi = lane >> 4, sl = lane & (kEll - 1);
+                  bool imp = false;
+                  while (true) {
+                    constexpr int R = kSoloChain / 4;
+                    const int32_t* const cur = (level & 1) ? ql1 : ql0;
+                    int32_t* const nxt = (level & 1) ? ql0 : ql1;
+                    int32_t v[R], m[R];
+                    uint32_t pword[R], oword[R], old[R];
+#pragma unroll
+                    for (int k = 0; k < R; ++k)
+                      if (4 * k < ncur) v[k] = cur[4 * k + vi];  // (beyond ncur: any entry of the queue)
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                      v[k] = 4 * k + vi < ncur ? v[k] : -1;
+                      m[k] = kPad;
+                      if (4 * k >= ncur) continue;
+                      const int32_t at = max(v[k], 0);
+                      m[k] = gload(ell + (int64_t)at * kEll + sl);
+                      if (has_prev) {
+                        pword[k] = gload(gprev + (at >> 5));
+                        if (ck) oword[k] = gload(gother + (at >> 5));
+                      }
+                    }
+                    bool tail = false;
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                      if (4 * k >= ncur) continue;
+                      m[k] = v[k] < 0 ? kPad : m[k];
+                      tail = tail || m[k] <= -2;
+                    }
+                    if (__ballot(tail && sl == kEll - 1) != 0) {
+                      chain = false;
+                      break;
+                    }
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                      if (4 * k >= ncur) continue;
+                      uint32_t in_prev = 0;
+                      if (has_prev) {
+                        const bool below = v[k] >= 0 && v[k] <= t;  // may be in X_t
+                        in_prev = below ? (pword[k] >> (v[k] & 31)) & 1u : 0u;
+                        if (ck && !imported && below && ((oword[k] >> (v[k] & 31)) & 1u) != 0) imp = true;
+                        if (in_prev != 0 && imported) {  // covered by the imported X_t
+                          v[k] = -1;
+                          m[k] = kPad;
+                        }
+                      }
+                      uint32_t dupv = 0, rv = 1;
+                      if (weigh) node_weight(M, d, sl == 0 ? v[k] : -1, dupv, rv);
+                      const uint32_t valid = m[k] != kPad ? 1u : 0u;  // an entry, or the diagonal's mark
+                      const uint32_t one = v[k] >= 0 && sl == 0 ? rv : 0u;
+                      w_all += valid + dupv;
+                      x_e += valid;
+                      r_all += one;
+                      if (has_prev) {
+                        w_ovl += in_prev != 0 ? valid + dupv : 0u;
+                        r_ovl += in_prev != 0 ? one : 0u;
+                      }
+                      old[k] = ~0u;
+                      if (m[k] >= 0) old[k] = atomicOr(&bm[m[k] >> 5], 1u << (m[k] & 31));
+                    }
+                    int32_t nn = 0;
+#pragma unroll
+                    for (int k = 0; k < R; ++k) {
+                      if (4 * k >= ncur) continue;
+                      bool isnew = m[k] >= 0 && ((old[k] >> (m[k] & 31)) & 1u) == 0;
+                      if (isnew && m[k] == imp_at) {
+                        imp = true;
+                        isnew = false;
+                      }
+                      u_new += isnew && m[k] > src;
+                      const uint64_t mr = __ballot(isnew && m[k] < src);
+                      if (isnew && m[k] < src) nxt[nn + (int32_t)rank_below(mr)] = m[k];
+                      nn += __popcll(mr);
+                    }
+                    ++level;
+                    ncur = nn;
+                    wave_sync();  // the next level's queue
+                    if (!imported && __ballot(imp) != 0) {
+                      cmd = kCmdImport;
+                      cslot = slot1;
+                    }
+                    if (cmd >= 0 || ncur == 0 || ncur > kSoloChain) break;
+                  }
+                  if (lane == 0) {
+                    s_cnt[level % 3] = ncur;
+                    s_cnt[(level + 1) % 3] = 0;
+                  }
+                  wave_sync();  // the counts
+                  if (cmd >= 0) break;
+                }
                 if (ncur == 0) {
                   phase = 3;
                   break;
