@@ -275,9 +275,16 @@ template <typename T>
 int DeviceSet::alloc(T*& p, size_t count, const char* what) {
   void* q = nullptr;
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-  hipError_t e = !alloc_stream_ ? hipMalloc(&q, bytes)
-                 : alloc_pool_  ? hipMallocFromPoolAsync(&q, bytes, alloc_pool_, alloc_stream_)
-                                : hipMallocAsync(&q, bytes, alloc_stream_);
+  if (arena_) {
+    const size_t step = (bytes + 255) & ~size_t(255);
+    arena_->asked += step;
+    if (arena_->used + step <= arena_->bytes) {
+      p = reinterpret_cast<T*>(arena_->base + arena_->used);
+      arena_->used += step;
+      return GSOFA_OK;
+    }
+  }
+  hipError_t e = alloc_stream_ ? hipMallocAsync(&q, bytes, alloc_stream_) : hipMalloc(&q, bytes);
   if (e != hipSuccess) return hip_fail(e, what);
   owned_.push_back(q);
   p = static_cast<T*>(q);
@@ -527,10 +534,10 @@ int enqueue_sequence(const Sequence& q, hipStream_t s, hipEvent_t* ev) {
 }
 
 int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream,
-                      hipMemPool_t pool) {
+                      DeviceArena* arena) {
   opt_ = opt_in_ = opt;
   alloc_stream_ = alloc_stream;
-  alloc_pool_ = pool;
+  arena_ = arena;
   nmats_ = (int)mats.size();
   if (nmats_ <= 0) return fail(GSOFA_ERR_INVALID_ARG, "empty matrix set");
   if (nmats_ > (1 << 20)) return fail(GSOFA_ERR_CAPACITY, "too many matrices in one set");

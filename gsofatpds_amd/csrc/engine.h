@@ -210,6 +210,13 @@ int enqueue_fronts(const Sequence& q, hipStream_t s, FrontSize* most = nullptr);
 // mirrored. Part of enqueue_sequence when q.prepare is set.
 int enqueue_preparation(const Sequence& q, hipStream_t s);
 
+// A block of device memory that one set at a time takes its arrays from; asked: bytes that the present
+// set has asked for in all, whether or not they fitted.
+struct DeviceArena {
+  char* base = nullptr;
+  size_t bytes = 0, used = 0, asked = 0;
+};
+
 // Device state for one matrix (plain plan) or many (batch); all matrices share one launch of
 // each kernel.
 class DeviceSet {
@@ -219,10 +226,10 @@ class DeviceSet {
   DeviceSet& operator=(const DeviceSet&) = delete;
   ~DeviceSet();
   // alloc_stream != null: stream-ordered allocations and uploads on that stream (no device-wide
-  // synchronisation; used by the server), freed on the same stream by the destructor; from `pool`, or
-  // the device's default pool.
+  // synchronisation; used by the server), freed on the same stream by the destructor. What fits comes
+  // from `arena` first, whose owner runs its sets one after another on that stream.
   int create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream = nullptr,
-             hipMemPool_t pool = nullptr);
+             DeviceArena* arena = nullptr);
   // Device bytes create() will allocate for these matrices (admission by footprint).
   static int64_t footprint(const std::vector<const Prepared*>& mats, const Options& opt, int64_t* out_bytes);
   // Enqueue the whole symbolic factorisation on `s` (no host synchronisation, no allocation,
@@ -330,7 +337,7 @@ class DeviceSet {
   LaunchConfig ccfg_;
   std::vector<void*> owned_;
   hipStream_t alloc_stream_ = nullptr;
-  hipMemPool_t alloc_pool_ = nullptr;
+  DeviceArena* arena_ = nullptr;
   // the early launch of top-separator items (top_separator_rows)
   int64_t n_top_ = 0;
   int top_grid_ = 0;

@@ -4,7 +4,8 @@
 // onto one of `slots` HIP streams as soon as a slot is free and their device footprint fits the
 // HBM budget. A slot takes the front request together with the requests queued behind it
 // (same options, FIFO order, up to max_group of them, within the budget) as one group: one
-// device set for all of them, i.e. one launch sequence, as a batch. Device state is allocated
+// device set for all of them, i.e. one launch sequence, as a batch. Device state comes
+// from memory that the slot keeps (bounded, and given back when the server stops), or is allocated
 // and freed stream-ordered on the slot (hipMallocAsync / hipFreeAsync: no device-wide
 // synchronisation). Groups on different slots run concurrently: their workgroups fill the CUs
 // others leave free, or, with cu_share set, each group's persistent grids are sized for that
@@ -55,6 +56,10 @@ struct Slot {
   hipEvent_t start = nullptr, done = nullptr;
   std::vector<Request*> group;  // empty: the slot is free
   std::unique_ptr<DeviceSet> set;
+  // Kept from group to group. Without it every group asks hipMallocAsync for some 45 arrays and gives
+  // them back: 24 requests, one set of four groups after another, took 16 to 24 ms, and after some
+  // thousands of such calls 60 ms and more, most of it waits in steps of 10 ms; from the arena 9 to 10.
+  DeviceArena arena;
   int64_t footprint = 0;        // charged against the budget while the group runs
   int error = GSOFA_OK;
   std::string error_text;
@@ -95,7 +100,7 @@ struct gsofa_server {
   int max_group = 16;
   int64_t budget = 0;
   std::atomic<int64_t> in_use{0};
-  hipMemPool_t pool = nullptr;  // the groups' device memory; null: the device's default pool
+  size_t arena_max = 0;  // bytes of a slot's arena at most
   std::vector<std::unique_ptr<Slot>> slots;
   std::mutex mu;
   std::condition_variable cv_admit, cv_done;
@@ -187,7 +192,18 @@ void gsofa_server::admit_loop() {
     int rc = GSOFA_OK;
     s.set.reset(new (std::nothrow) DeviceSet);
     if (!s.set) rc = fail(GSOFA_ERR_OUT_OF_MEMORY, "device set");
-    if (rc == GSOFA_OK) rc = s.set->create(mats, r->opt, s.stream, pool);
+    // the arena grows to what the slot's last group asked for (its memory is idle: the slot was free)
+    const size_t want = std::min(arena_max, s.arena.asked + s.arena.asked / 8);
+    if (want > s.arena.bytes) {
+      if (s.arena.base) (void)hipFreeAsync(s.arena.base, s.stream);
+      void* q = nullptr;
+      const bool ok = hipMallocAsync(&q, want, s.stream) == hipSuccess;
+      if (!ok) (void)hipGetLastError();
+      s.arena.base = static_cast<char*>(q);
+      s.arena.bytes = ok ? want : 0;
+    }
+    s.arena.used = s.arena.asked = 0;
+    if (rc == GSOFA_OK) rc = s.set->create(mats, r->opt, s.stream, &s.arena);
     if (rc == GSOFA_OK && hipEventRecord(s.start, s.stream) != hipSuccess) rc = fail(GSOFA_ERR_HIP, "hipEventRecord");
     if (rc == GSOFA_OK) rc = s.set->enqueue(s.stream);
     if (rc != GSOFA_OK) {
@@ -315,21 +331,9 @@ int gsofa_server_start(const gsofa_server_options* opt, gsofa_server** out) {
         hipEventCreate(&s->start) != hipSuccess || hipEventCreate(&s->done) != hipSuccess)
       return fail(GSOFA_ERR_HIP, "slot stream/event creation");
   }
-  // A pool of the server's own that keeps what its groups free, up to a 32nd of the device's memory
-  // (and the budget): the default pool gives all of it back at the next synchronisation of any
-  // stream, and a group of 16 maps some hundreds of MB anew (24 requests, one every so often: 65 ms
-  // each time, 16 with the pool). It goes back with the server.
-  hipMemPoolProps props{};
-  props.allocType = hipMemAllocationTypePinned;
-  props.location.type = hipMemLocationTypeDevice;
-  props.location.id = opt->device;
-  if (hipMemPoolCreate(&srv->pool, &props) == hipSuccess) {
-    uint64_t keep = (uint64_t)std::min<int64_t>(srv->budget, (int64_t)(total_b / 32));
-    (void)hipMemPoolSetAttribute(srv->pool, hipMemPoolAttrReleaseThreshold, &keep);
-  } else {
-    (void)hipGetLastError();
-    srv->pool = nullptr;
-  }
+  // Device memory that the slots keep between groups: a 32nd of the device's at most, and of the
+  // budget an eighth.
+  srv->arena_max = (size_t)std::min<int64_t>(srv->budget / 8, (int64_t)(total_b / 32)) / (size_t)opt->slots;
   srv->admit_thread = std::thread([p = srv.get()] { p->admit_loop(); });
   srv->done_thread = std::thread([p = srv.get()] { p->done_loop(); });
   *out = srv.release();
@@ -531,12 +535,12 @@ int gsofa_server_stop(gsofa_server* srv) {
   if (srv->done_thread.joinable()) srv->done_thread.join();  // drains running requests
   for (auto& sp : srv->slots) {
     Slot& s = *sp;
+    if (s.arena.base) (void)hipFreeAsync(s.arena.base, s.stream);
     if (s.stream) (void)hipStreamSynchronize(s.stream);
     if (s.start) (void)hipEventDestroy(s.start);
     if (s.done) (void)hipEventDestroy(s.done);
     if (s.stream) (void)hipStreamDestroy(s.stream);
   }
-  if (srv->pool) (void)hipMemPoolDestroy(srv->pool);  // the last groups' frees are done: the streams were waited for
   delete srv;
   return GSOFA_OK;
 }
