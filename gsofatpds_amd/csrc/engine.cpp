@@ -445,7 +445,12 @@ int enqueue_preparation(const Sequence& q, hipStream_t s) {
     return fail(e == hipErrorOutOfMemory ? GSOFA_ERR_OUT_OF_MEMORY : GSOFA_ERR_HIP,
                 std::string(what) + ": " + hipGetErrorString(e));
   };
-  hipError_t e = launch_ell_build(q.nrows, q.nmats, q.row_base, q.rowptr_a, q.adj_a, q.ell_a, s);
+  hipError_t e;
+  if (q.nmats == 1 && !q.mirror_all && q.nrows <= kSmallRows && q.nnz <= kSmallRowEntries * q.nrows) {
+    e = launch_prepare_small((int32_t)q.nrows, q.rowptr_a, q.adj_a, q.ell_a, q.rowptr_t, q.adj_t, q.ell_t, s);
+    return e == hipSuccess ? GSOFA_OK : hf(e, "small pattern's layout");
+  }
+  e = launch_ell_build(q.nrows, q.nmats, q.row_base, q.rowptr_a, q.adj_a, q.ell_a, s);
   if (e != hipSuccess) return hf(e, "ell A");
   if (!q.mirror_all) {  // A^T: traversed from every matrix that is not mirrored
     e = launch_transpose(q.nrows, q.nmats, q.row_base, q.rowptr_a, q.adj_a, q.col_cnt, q.rowptr_t, q.cursor, q.adj_t,
@@ -1135,6 +1140,7 @@ int DeviceSet::top_ms(double* ms) {
 Sequence DeviceSet::sequence() const {
   Sequence q;
   q.nrows = nrows_;
+  q.nnz = nnz_;
   q.nitems = nitems_;
   q.nblk_total = nblk_total_;
   q.nblocks_sup = nblocks_sup_;

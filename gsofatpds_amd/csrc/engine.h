@@ -146,6 +146,7 @@ int configure_launch(int32_t n_max, int64_t nrows, bool paired_any, const Option
 // entry's (which carves the same buffers from a static array).
 struct Sequence {
   int64_t nrows = 0, nitems = 0, nblk_total = 0, nblocks_sup = 0, esc_words = 0;
+  int64_t nnz = 0;
   int nmats = 0;
   int32_t nb_max = 0, n_max = 0;
   int32_t paired_any = 0;

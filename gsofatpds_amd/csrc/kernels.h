@@ -165,6 +165,10 @@ hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, c
                             const int32_t* adj, int32_t* ell, hipStream_t s);
 // Builds A^T of every matrix: col_cnt/cursor/rowptr_t have nrows (+1) entries, block_sums
 // ceil(nrows / 4096), total one int.
+// The layout of one matrix of at most kSmallRows rows in one launch: ell of A, A^T and its ell.
+constexpr int kSmallRows = 4096, kSmallRowEntries = 16;  // (entries per row on average, at most)
+hipError_t launch_prepare_small(int32_t n, const int32_t* rowptr, const int32_t* adj, int32_t* ell, int32_t* rowptr_t,
+                                int32_t* adj_t, int32_t* ell_t, hipStream_t s);
 hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* col_cnt, int32_t* rowptr_t, int32_t* cursor,
                             int32_t* adj_t, int32_t* block_sums, int32_t* total, hipStream_t s);

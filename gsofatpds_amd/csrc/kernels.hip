@@ -18,10 +18,12 @@
 //   k_fill_u64 / k_fill_i32     clear accumulators and counters (graph-safe, no memset nodes)
 //   k_ell_build                 pack rows into 64-byte ELL-16 slots
 //   k_col_hist, scan, k_transpose_scatter, k_ell_build   build A^T in the same layout
+//   k_prepare_small             all of these for one small matrix
 //   k_light                     one wave per block of rows, LDS hash set; escalates big sources
 //   k_front_leaf, k_front       (matrices with fronts, instead) elimination subtrees as bit matrices
 //   k_cond_*                    (these) the graph of what the fronts left, and its items
 //   k_heavy_hist, scan, k_heavy_scatter   the workgroup path's queue, costliest blocks first
+//   k_heavy_order_small         the same for few blocks
 //   k_heavy                     one workgroup per block of escalated (or left) rows, n-bit bitmap
 //   k_supernodes                the reference's supernode rule, one thread per row
 //   k_totals                    sums the accumulators' copies
@@ -178,37 +180,101 @@ __global__ void k_clear_run(unsigned long long* __restrict__ acc, int64_t nacc, 
 // ------------------------------------------------------------------------------------------
 // layout: ELL-16 packing and the transpose
 // ------------------------------------------------------------------------------------------
-// Row g of the concatenated pattern: entries adj[rowptr[g] .. rowptr[g+1]) (local column ids).
+// Row g of the concatenated pattern, vertex v of its matrix: entries adj[rowptr[g] .. rowptr[g+1])
+// (local column ids).
+__device__ __forceinline__ void ell_row(int64_t g, int32_t v, const int32_t* rowptr, const int32_t* adj, int32_t* ell) {
+  const int32_t b = rowptr[g], e = rowptr[g + 1];
+  const int32_t deg = e - b;
+  int32_t slot[kEll];
+#pragma unroll
+  for (int k = 0; k < kEll; ++k) slot[k] = kPad;
+  if (deg < kEll) {
+    // off-diagonal entries first, then the diagonal's mark (at most slot 14)
+    int k = 0;
+    bool diag = false;
+    for (int p = 0; p < deg; ++p) {
+      const int32_t c = adj[b + p];
+      if (c == v) diag = true;
+      else slot[k++] = c;
+    }
+    if (diag) slot[k] = kDiag;
+  } else if (deg == kEll) {
+    for (int k = 0; k < kEll; ++k) slot[k] = adj[b + k];
+  } else {
+    for (int k = 0; k < kEll - 1; ++k) slot[k] = adj[b + k];
+    slot[kEll - 1] = -(b + (kEll - 1) + 2);
+  }
+  int4* dst = reinterpret_cast<int4*>(ell + g * kEll);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) dst[q] = make_int4(slot[4 * q], slot[4 * q + 1], slot[4 * q + 2], slot[4 * q + 3]);
+}
+
 __global__ void k_ell_build(int64_t nrows, int nmats, const int64_t* __restrict__ row_base,
                             const int32_t* __restrict__ rowptr, const int32_t* __restrict__ adj,
                             int32_t* __restrict__ ell) {
-  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < nrows; g += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t b = rowptr[g], e = rowptr[g + 1];
-    const int32_t deg = e - b;
-    int32_t slot[kEll];
+  for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < nrows; g += (int64_t)gridDim.x * blockDim.x)
+    ell_row(g, (int32_t)(g - row_base[nmats == 1 ? 0 : find_segment(row_base, nmats, g)]), rowptr, adj, ell);
+}
+
+// Exclusive scan of kSmallRows counts in LDS, in place, by one workgroup of kSmallThreads; returns
+// their sum.
+constexpr int kSmallThreads = 1024;
+__device__ __forceinline__ int32_t scan_small(int32_t* cnt, int32_t* s_wave) {
+  constexpr int kPer = kSmallRows / kSmallThreads;
+  static_assert(kPer * kSmallThreads == kSmallRows, "every count by one thread");
+  const int tid = threadIdx.x;
+  int32_t c[kPer], sum = 0;
 #pragma unroll
-    for (int k = 0; k < kEll; ++k) slot[k] = kPad;
-    if (deg < kEll) {
-      // off-diagonal entries first, then the diagonal's mark (at most slot 14)
-      const int32_t v = (int32_t)(g - row_base[nmats == 1 ? 0 : find_segment(row_base, nmats, g)]);
-      int k = 0;
-      bool diag = false;
-      for (int p = 0; p < deg; ++p) {
-        const int32_t c = adj[b + p];
-        if (c == v) diag = true;
-        else slot[k++] = c;
-      }
-      if (diag) slot[k] = kDiag;
-    } else if (deg == kEll) {
-      for (int k = 0; k < kEll; ++k) slot[k] = adj[b + k];
-    } else {
-      for (int k = 0; k < kEll - 1; ++k) slot[k] = adj[b + k];
-      slot[kEll - 1] = -(b + (kEll - 1) + 2);
-    }
-    int4* dst = reinterpret_cast<int4*>(ell + g * kEll);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) dst[q] = make_int4(slot[4 * q], slot[4 * q + 1], slot[4 * q + 2], slot[4 * q + 3]);
+  for (int k = 0; k < kPer; ++k) {
+    c[k] = cnt[tid * kPer + k];
+    sum += c[k];
   }
+  int32_t incl = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int32_t y = __shfl_up(incl, o, 64);
+    if (lane_id() >= o) incl += y;
+  }
+  if (lane_id() == 63) s_wave[tid >> 6] = incl;
+  __syncthreads();
+  int32_t off = incl - sum, all = 0;
+  for (int w = 0; w < kSmallThreads / 64; ++w) {
+    off += w < (tid >> 6) ? s_wave[w] : 0;
+    all += s_wave[w];
+  }
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    cnt[tid * kPer + k] = off;
+    off += c[k];
+  }
+  __syncthreads();
+  return all;
+}
+
+// One matrix of at most kSmallRows rows: its ELL rows, A^T and the ELL rows of that in one launch by one
+// workgroup, the column counts and cursors in LDS. Bound by the latency of a few rounds of reads: 13 us
+// for a band of 1,024 rows and 53 for 4,096, where eight launches end after 107 and 110, most of it the
+// gaps between them. Twice the rows would take as long as the launches: the line.
+__global__ __launch_bounds__(kSmallThreads) void k_prepare_small(int32_t n, const int32_t* __restrict__ rowptr,
+                                                                 const int32_t* __restrict__ adj, int32_t* __restrict__ ell,
+                                                                 int32_t* rowptr_t, int32_t* adj_t, int32_t* ell_t) {
+  __shared__ int32_t s_cnt[kSmallRows], s_wave[kSmallThreads / 64];
+  const int tid = threadIdx.x;
+  for (int i = tid; i < kSmallRows; i += kSmallThreads) s_cnt[i] = 0;
+  __syncthreads();
+  for (int32_t v = tid; v < n; v += kSmallThreads) {
+    ell_row(v, v, rowptr, adj, ell);
+    for (int32_t p = rowptr[v]; p < rowptr[v + 1]; ++p) atomicAdd(&s_cnt[adj[p]], 1);
+  }
+  __syncthreads();
+  const int32_t all = scan_small(s_cnt, s_wave);
+  for (int32_t v = tid; v < n; v += kSmallThreads) rowptr_t[v] = s_cnt[v];
+  if (tid == 0) rowptr_t[n] = all;
+  __syncthreads();
+  for (int32_t v = tid; v < n; v += kSmallThreads)
+    for (int32_t p = rowptr[v]; p < rowptr[v + 1]; ++p) adj_t[atomicAdd(&s_cnt[adj[p]], 1)] = v;
+  __syncthreads();
+  for (int32_t v = tid; v < n; v += kSmallThreads) ell_row(v, v, rowptr_t, adj_t, ell_t);
 }
 
 // Column counts of every matrix of the set: one thread per global row.
@@ -1053,6 +1119,53 @@ __global__ void k_heavy_scatter(const MatDev* __restrict__ mats, int64_t nblk_to
       heavy_items[pos] = encode_item((uint32_t)m, dir, (uint32_t)(b * mats[m].chain_block), 0u);
     }
   }
+}
+
+// The same sort in one launch by one workgroup, for at most kSmallRows block indices and slots: 5 us,
+// where the three launches above take 15 and two gaps.
+__global__ __launch_bounds__(kSmallThreads) void k_heavy_order_small(const MatDev* __restrict__ mats, int32_t nslots, int nmats,
+                                                                     const int64_t* __restrict__ blkq_base,
+                                                                     const uint32_t* __restrict__ blk_flag, int32_t nb_max,
+                                                                     WorkState* __restrict__ ws,
+                                                                     uint64_t* __restrict__ heavy_items) {
+  __shared__ int32_t s_cnt[kSmallRows], s_wave[kSmallThreads / 64];
+  constexpr int kPer = kSmallRows / kSmallThreads;
+  const int tid = threadIdx.x;
+  for (int i = tid; i < kSmallRows; i += kSmallThreads) s_cnt[i] = 0;
+  __syncthreads();
+  // per slot of this thread: its block, matrix, direction and cut, found once
+  int32_t at[kPer], cut[kPer];
+  uint64_t whole[kPer];
+  bool early[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int32_t g = k * kSmallThreads + tid;
+    int m;
+    uint32_t dir;
+    int32_t b;
+    at[k] = -1;
+    if (g >= nslots || !heavy_slot(mats, nslots / 2, nmats, blkq_base, blk_flag, g, m, dir, b)) continue;
+    at[k] = nb_max - 1 - b;
+    cut[k] = block_cut(mats[m], b);
+    early[k] = cut[k] >= mats[m].light_end;
+    whole[k] = encode_item((uint32_t)m, dir, (uint32_t)(cut[k] >= 0 ? cut[k] : b * mats[m].chain_block), 0u);
+    atomicAdd(&s_cnt[at[k]], cut[k] >= 0 && !early[k] ? 2 : 1);
+  }
+  __syncthreads();
+  const int32_t all = scan_small(s_cnt, s_wave);
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    if (at[k] < 0) continue;
+    const uint64_t before = whole[k] | (1ull << 63);
+    if (cut[k] >= 0 && !early[k]) {
+      const int32_t pos = atomicAdd(&s_cnt[at[k]], 2);
+      heavy_items[pos] = whole[k];
+      heavy_items[pos + 1] = before;
+    } else {
+      heavy_items[atomicAdd(&s_cnt[at[k]], 1)] = cut[k] >= 0 ? before : whole[k];
+    }
+  }
+  if (tid == 0) ws->heavy_count = (unsigned long long)all;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -4016,6 +4129,13 @@ hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, c
   return hipGetLastError();
 }
 
+hipError_t launch_prepare_small(int32_t n, const int32_t* rowptr, const int32_t* adj, int32_t* ell, int32_t* rowptr_t,
+                                int32_t* adj_t, int32_t* ell_t, hipStream_t s) {
+  if (n > kSmallRows) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_prepare_small, dim3(1), dim3(kSmallThreads), 0, s, n, rowptr, adj, ell, rowptr_t, adj_t, ell_t);
+  return hipGetLastError();
+}
+
 hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* col_cnt, int32_t* rowptr_t, int32_t* cursor,
                             int32_t* adj_t, int32_t* block_sums, int32_t* total, hipStream_t s) {
@@ -4046,6 +4166,11 @@ hipError_t launch_heavy_order(const MatDev* mats, int64_t nblk_total, int nmats,
                               const uint32_t* blk_flag, int32_t nb_max, int32_t* bucket, int32_t* cursor,
                               int32_t* block_sums, int32_t* total, WorkState* ws, uint64_t* heavy_items, hipStream_t s) {
   const int64_t nslots = 2 * nblk_total;
+  if (nslots <= kSmallRows) {  // (no more block indices than slots)
+    hipLaunchKernelGGL(k_heavy_order_small, dim3(1), dim3(kSmallThreads), 0, s, mats, (int32_t)nslots, nmats, blkq_base,
+                       blk_flag, nb_max, ws, heavy_items);
+    return hipGetLastError();
+  }
   const int g = grid_for(nslots, 256, 8192);
   // bucket is zero already (the run's clears)
   hipLaunchKernelGGL(k_heavy_hist, dim3(g), dim3(256), 0, s, mats, nblk_total, nmats, blkq_base, blk_flag, nb_max, bucket,

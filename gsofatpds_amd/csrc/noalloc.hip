@@ -117,26 +117,29 @@ void carve_layout(unsigned char* base, int32_t n, int64_t nnz, int64_t nblk, int
   L.ck_bytes = c.off - L.fixed_bytes - L.spill_bytes;
 }
 
-// Sets *bad unless rowptr/adj is a CSR pattern of n rows whose rows are strictly increasing
-// column ids in [0, n), with rowptr[0] == 0 and rowptr[n] == nnz. Reads adj only inside checked
-// extents.
+// Whether row v is one of a CSR pattern of n rows whose rows are strictly increasing column ids in
+// [0, n), with rowptr[0] == 0 and rowptr[n] == nnz. Reads adj only inside checked extents.
+__device__ __forceinline__ bool row_ok(int64_t v, int32_t n, int64_t nnz, const int32_t* rowptr, const int32_t* adj) {
+  const int64_t b = rowptr[v], e = rowptr[v + 1];
+  bool ok = b >= 0 && b <= e && e <= nnz;
+  if (v == 0) ok = ok && b == 0;
+  if (v == n - 1) ok = ok && e == nnz;
+  if (ok) {
+    int32_t last = -1;
+    for (int64_t p = b; p < e && ok; ++p) {
+      const int32_t c = adj[p];
+      ok = c > last && c < n;
+      last = c;
+    }
+  }
+  return ok;
+}
+
+// Sets *bad unless every row is one.
 __global__ void k_noalloc_check(int32_t n, int64_t nnz, const int32_t* __restrict__ rowptr,
                                 const int32_t* __restrict__ adj, uint32_t* __restrict__ bad) {
-  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t b = rowptr[v], e = rowptr[v + 1];
-    bool ok = b >= 0 && b <= e && e <= nnz;
-    if (v == 0) ok = ok && b == 0;
-    if (v == n - 1) ok = ok && e == nnz;
-    if (ok) {
-      int32_t last = -1;
-      for (int64_t p = b; p < e && ok; ++p) {
-        const int32_t c = adj[p];
-        ok = c > last && c < n;
-        last = c;
-      }
-    }
-    if (!ok) atomicOr(bad, 1u);
-  }
+  for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += (int64_t)gridDim.x * blockDim.x)
+    if (!row_ok(v, n, nnz, rowptr, adj)) atomicOr(bad, 1u);
 }
 
 // The pattern into the scratch, or, when the check failed, an empty pattern of n rows (every
@@ -162,6 +165,28 @@ __global__ void k_noalloc_tables(Tables t, MatDev* __restrict__ mats, int64_t* _
     *mats = t.m;
     for (int k = 0; k < 8; ++k) bases[k] = t.bases[k];
   }
+}
+
+// All of the above for a small pattern, by one workgroup: the check, then the copy, and the tables.
+__global__ __launch_bounds__(1024) void k_noalloc_input_small(int32_t n, int64_t nnz, const int32_t* __restrict__ rowptr,
+                                                              const int32_t* __restrict__ adj, uint32_t* __restrict__ bad,
+                                                              int32_t* __restrict__ rowptr_a, int32_t* __restrict__ adj_a,
+                                                              Tables t, MatDev* __restrict__ mats, int64_t* __restrict__ bases) {
+  __shared__ uint32_t s_bad;
+  if (threadIdx.x == 0) {
+    s_bad = 0;
+    *mats = t.m;
+    for (int k = 0; k < 8; ++k) bases[k] = t.bases[k];
+  }
+  __syncthreads();
+  for (int32_t v = threadIdx.x; v < n; v += 1024)
+    if (!row_ok(v, n, nnz, rowptr, adj)) s_bad = 1;
+  __syncthreads();
+  const bool empty = s_bad != 0;
+  if (threadIdx.x == 0) *bad = empty ? 1u : 0u;
+  for (int32_t i = threadIdx.x; i <= n; i += 1024) rowptr_a[i] = empty ? 0 : rowptr[i];
+  if (!empty)
+    for (int64_t i = threadIdx.x; i < nnz; i += 1024) adj_a[i] = adj[i];
 }
 
 // Totals in the order gsofa_run_noalloc documents: fill, nnz_F, nnz_L, nnz_U, W, |R|, reported
@@ -324,16 +349,22 @@ int gsofa_run_noalloc(int32_t n, int64_t nnz, const int32_t* rowptr, const int32
   int64_t* blkq_base = L.bases + 6;
 
   hipStream_t s = static_cast<hipStream_t>(hip_stream);
-  const int g = (int)std::min<int64_t>(4096, ((int64_t)std::max<int64_t>(n + 1, nnz) + 255) / 256);
-  NA_HIP(launch_fill_i32(reinterpret_cast<int32_t*>(L.bad), 1, 0, s), "clear input flag");
-  hipLaunchKernelGGL(k_noalloc_check, dim3(std::min(4096, (n + 255) / 256)), dim3(256), 0, s, n, nnz, rowptr, adj,
-                     L.bad);
-  hipLaunchKernelGGL(k_noalloc_copy, dim3(g), dim3(256), 0, s, n, nnz, rowptr, adj, L.bad, L.rowptr_a, L.adj_a);
-  hipLaunchKernelGGL(k_noalloc_tables, dim3(1), dim3(64), 0, s, t, L.mats, L.bases);
+  if (n <= kSmallRows && nnz <= (int64_t)kSmallRowEntries * n) {
+    hipLaunchKernelGGL(k_noalloc_input_small, dim3(1), dim3(1024), 0, s, n, nnz, rowptr, adj, L.bad, L.rowptr_a, L.adj_a, t,
+                       L.mats, L.bases);
+  } else {
+    const int g = (int)std::min<int64_t>(4096, ((int64_t)std::max<int64_t>(n + 1, nnz) + 255) / 256);
+    NA_HIP(launch_fill_i32(reinterpret_cast<int32_t*>(L.bad), 1, 0, s), "clear input flag");
+    hipLaunchKernelGGL(k_noalloc_check, dim3(std::min(4096, (n + 255) / 256)), dim3(256), 0, s, n, nnz, rowptr, adj,
+                       L.bad);
+    hipLaunchKernelGGL(k_noalloc_copy, dim3(g), dim3(256), 0, s, n, nnz, rowptr, adj, L.bad, L.rowptr_a, L.adj_a);
+    hipLaunchKernelGGL(k_noalloc_tables, dim3(1), dim3(64), 0, s, t, L.mats, L.bases);
+  }
   NA_HIP(hipGetLastError(), "input kernels");
   // the launch sequence of a plan, without its allocation
   Sequence q;
   q.nrows = n;
+  q.nnz = nnz;
   q.nitems = nitems;
   q.nblk_total = nblk;
   q.nblocks_sup = nblocks_sup;
