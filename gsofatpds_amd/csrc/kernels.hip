@@ -3283,6 +3283,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               if (cmd >= 0) break;
             }
             if (phase == 3) {
+              // condensed: the nodes of the 128 vertices behind the row's, read while the sums below run
+              int32_t win_id[2] = {-1, -1};
+              if (kCond && (d == 1 || M.sym)) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                  const int32_t x = s_orig[li] + 1 + 64 * q + lane;
+                  if (x < chunk_end) win_id[q] = gload(M.nid + x);
+                }
+              }
               // ---- this row's totals: the leader's own sums plus the cooperative phases' ----
               // (a sum no lane contributed to costs no reduction: a row that reaches nothing new
               // below itself has only its seed sums)
@@ -3370,17 +3379,16 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               const int wslot = s_ls.wp[d];  // the ring slot this row's save takes
               const int32_t vsrc = kCond ? s_orig[li] : src;
               if (kCond && (d == 1 || M.sym)) {
-                // window bits of a node: its next 128 nodes hold every vertex vsrc + 1 .. vsrc + 128
-                // of the graph; a set bit stands for its node's vertex
-                uint32_t win[4] = {0, 0, 0, 0};
+                // window bits by vertex: bit t is the node of vsrc + 1 + t. (Not by node: list nodes stand
+                // between the vertices.) A contracted vertex has no bit of its own, and none is missed: a
+                // row's U entries are ancestors of it, and a row below a contracted vertex is finished.
+                uint64_t win[2];
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                  const int32_t j = src + 1 + 64 * q + lane;
-                  if (j < n && ((bm_get(j >> 5) >> (j & 31)) & 1u) != 0) window_bit(win, vsrc, gload(M.orig + j), chunk_end);
-                }
-                const uint32_t w0 = wave_or_u32(win[0]), w1 = wave_or_u32(win[1]);
-                const uint32_t w2 = wave_or_u32(win[2]), w3 = wave_or_u32(win[3]);
-                if (lane == 0) reinterpret_cast<uint4*>(M.win)[vsrc] = make_uint4(w0, w1, w2, w3);
+                for (int q = 0; q < 2; ++q)
+                  win[q] = __ballot(win_id[q] >= 0 && ((bm_get(max(win_id[q], 0) >> 5) >> (win_id[q] & 31)) & 1u) != 0);
+                if (lane == 0)
+                  reinterpret_cast<uint4*>(M.win)[vsrc] = make_uint4((uint32_t)win[0], (uint32_t)(win[0] >> 32),
+                                                                    (uint32_t)win[1], (uint32_t)(win[1] >> 32));
               }
               if (lane == 0) {
                 const RowFacts f{wr, dg0, rr, U, want_list ? kept : 0u};
