@@ -115,6 +115,7 @@ _SIGNATURES = {
     "gsofa_work_split": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64),
                                    C.POINTER(C.c_uint64)]),
     "gsofa_executed_work": (C.c_int, [C.c_void_p, C.POINTER(C.c_uint64)]),
+    "gsofa_plan_fronts": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_int64)]),
     "gsofa_early_top": (C.c_int, [C.c_void_p, C.POINTER(C.c_int64), C.POINTER(C.c_double), C.POINTER(C.c_uint64)]),
     "gsofa_plan_stage_timing": (C.c_int, [C.c_void_p, C.c_int32]),
     "gsofa_plan_destroy": (None, [C.c_void_p]),
@@ -451,6 +452,13 @@ class Plan:
         _check(lib().gsofa_executed_work(self._h, w))
         return {"heavy_edges": w[0], "heavy_rows": w[1], "heavy_out": w[2],
                 "light_edges": w[3], "light_rows": w[4], "light_out": w[5]}
+
+    def fronts(self) -> dict:
+        """Subtrees that the plan's runs finish as bit matrices, and nodes of the condensed graph (both
+        0: it runs without)."""
+        u, n = C.c_int64(), C.c_int64()
+        _check(lib().gsofa_plan_fronts(self._h, C.byref(u), C.byref(n)))
+        return {"units": u.value, "nodes": n.value}
 
     def early_top(self) -> dict:
         """The last run's early launch of the top separator's items: item count (0: none), device

@@ -553,6 +553,13 @@ int gsofa_plan_config(gsofa_plan* p, int32_t* out4) {
   return GSOFA_OK;
 }
 
+int gsofa_plan_fronts(gsofa_plan* p, int64_t* units, int64_t* nodes) {
+  if (!p) return fail(GSOFA_ERR_INVALID_ARG, "plan is null");
+  if (units) *units = p->set.unit_count();
+  if (nodes) *nodes = p->set.condensed_nodes();
+  return GSOFA_OK;
+}
+
 int gsofa_batch_config(gsofa_batch* b, int32_t* out4) {
   if (!b || !out4) return fail(GSOFA_ERR_INVALID_ARG, "null argument");
   config_of(b->set, out4);

@@ -256,6 +256,10 @@ class DeviceSet {
   int qcap() const { return qcap_; }
   int heavy_wgs_per_cu() const { return heavy_wgs_per_cu_; }
   bool bitmap_in_hbm() const { return hbm_bitmap_; }
+  // Elimination subtrees that the fronts take, and nodes of the condensed graphs (0: every matrix runs
+  // without).
+  int64_t unit_count() const { return ncond_ > 0 ? fronts_[kFrontLevels - 1].u1 : 0; }
+  int64_t condensed_nodes() const { return ncond_ > 0 ? cnodes_ : 0; }
   // Items of the early launch (0: none) and, after a run enqueued with stage events, its time.
   int64_t top_items() const { return n_top_; }
   int top_ms(double* ms);

@@ -1372,12 +1372,12 @@ __global__ __launch_bounds__(kLeafWaves * 64) void k_front_leaf(const MatDev* __
           t_w += deg + nd;
           t_r += (uint32_t)__popcll(r);
           t_u += U;
-          ++t_v;
         }
       } else if (on) {
         t_l += U;
       }
       if (on) {
+        ++t_v;
         t_fill += U - seed;
         gstore(M.cnt[d] + v, (int32_t)U);
       }
@@ -1797,6 +1797,7 @@ __global__ __launch_bounds__(kFrontThreads[kLevel]) __attribute__((amdgpu_waves_
           if (key[k] >= 0) put_bit((k0 + k) * kRows + (tid >> 4), column(key[k], x[k]));
       }
       long_rows([&](int i, int32_t x) {
+        ++t_e;
         if (S.unit[i] == -2 && x > S.ids[i]) atomicAdd(&S.seed[i], 1);
         int32_t h = find(x, home(x));
         while (h < 0) {  // contracted: its root's node
@@ -1975,10 +1976,10 @@ __global__ __launch_bounds__(kFrontThreads[kLevel]) __attribute__((amdgpu_waves_
             t_w += (uint64_t)(uint32_t)S.wdeg[i] + nd;
             t_r += nr;
             t_u += U;
-            t_v += 1;
           } else {
             t_l += U;
           }
+          ++t_v;
           if (win_dir) gstore_v4(wins + 4 * (int64_t)v, win[0], win[1], win[2], win[3]);
         }
         if (list_ptr != nullptr) {
@@ -2516,6 +2517,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   __shared__ uint32_t s_unew;      // new U entries found by cooperative phases
   __shared__ unsigned long long s_wall, s_wovl, s_xe;  // row sums of earlier turns and cooperative phases
   __shared__ uint32_t s_rall, s_rovl, s_useed, s_deg0;
+  __shared__ uint32_t s_xv;        // condensed: nodes expanded (s_rall counts the vertices that they stand for)
   __shared__ int32_t s_import, s_src_was_set;
   __shared__ int32_t s_esc[2][kHeavyWin + 1];   // row w0 + i was escalated (per direction)
   __shared__ int32_t s_hold[2][kHeavyWin + 1];  // row w0 + i holds w0 + i - 1
@@ -2778,6 +2780,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           uint32_t ubase = s_ls.ubase, gap = s_ls.gap;
           // per-lane row sums of this turn's passes (earlier turns' are in the LDS sums)
           uint32_t w_all = 0, w_ovl = 0, x_e = 0, r_all = 0, r_ovl = 0, u_seed = 0, u_new = 0, deg0 = 0;
+          uint32_t x_v = 0;  // condensed
           int32_t cmd = -1;
           int32_t cslot = 0;
           while (cmd < 0) {
@@ -2903,9 +2906,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 s_unew = 0;
                 s_wall = s_wovl = s_xe = 0;
                 s_rall = s_rovl = s_useed = s_deg0 = 0;
+                if (kCond) s_xv = 0;
                 s_import = 0;
               }
-              w_all = w_ovl = x_e = r_all = r_ovl = u_seed = u_new = deg0 = 0;
+              w_all = w_ovl = x_e = r_all = r_ovl = u_seed = u_new = deg0 = x_v = 0;
               gap = 0;
               phase = 1;
               if (!chained) {
@@ -3043,6 +3047,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                       w_all += valid + dupv;
                       x_e += valid;
                       r_all += one;
+                      if (kCond) x_v += v[k] >= 0 && sl == 0 ? 1u : 0u;
                       if (has_prev) {
                         w_ovl += in_prev != 0 ? valid + dupv : 0u;
                         r_ovl += in_prev != 0 ? one : 0u;
@@ -3158,6 +3163,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                     w_all += valid + dupv;
                     if (in_prev) w_ovl += valid + dupv;
                     if (v >= 0 && sl == 0) {
+                      if (kCond) ++x_v;
                       r_all += rv;
                       if (in_prev) r_ovl += rv;
                     }
@@ -3260,6 +3266,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                   if (v >= 0) {
                     deg += dupv;
                     w_all += deg;
+                    if (kCond) ++x_v;
                     r_all += rv;
                     if (in_prev) {
                       w_ovl += deg;
@@ -3301,6 +3308,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
               const uint64_t a_x = (uint64_t)wsum(x_e) + s_xe;
               const uint64_t a_r = (uint64_t)wsum(r_all) + s_rall;
               const uint64_t a_ro = (uint64_t)wsum(r_ovl) + s_rovl;
+              const uint64_t a_xv = kCond ? (uint64_t)wsum(x_v) + s_xv : a_r;
               const uint32_t a_us = wsum(u_seed) + s_useed;
               const uint32_t a_un = wsum(u_new) + s_unew;
               const uint64_t dg0 = (uint64_t)wsum(deg0) + s_deg0;
@@ -3409,7 +3417,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 tot.fill += U - a_us;
                 tot.heavy += 1;
                 tot.x_edges += a_x;
-                tot.x_verts += a_r + 1;
+                tot.x_verts += a_xv + 1;
                 tot.x_out += U;
                 if (d == 0) {
                   tot.w += dg0 + wr;
@@ -3470,7 +3478,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
             const uint32_t a_w = wave_sum_u32(w_all), a_wo = wave_sum_u32(w_ovl), a_x = wave_sum_u32(x_e);
             const uint32_t a_r = wave_sum_u32(r_all), a_ro = wave_sum_u32(r_ovl), a_us = wave_sum_u32(u_seed);
             const uint32_t a_un = wave_sum_u32(u_new), a_d0 = wave_sum_u32(deg0);
+            const uint32_t a_xv = kCond ? wave_sum_u32(x_v) : 0u;
             if (lane == 0) {
+              if (kCond) s_xv += a_xv;
               s_wall += a_w;
               s_wovl += a_wo;
               s_xe += a_x;
@@ -3565,7 +3575,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           const int32_t cimp_at = chas_prev && !cck ? csrc - 1 : -2;
           const uint32_t cubase = ctl.ubase;
           bool cimported = ctl.imported != 0;
-          uint32_t p_w = 0, p_wo = 0, p_x = 0, p_r = 0, p_ro = 0, p_un = 0;
+          uint32_t p_w = 0, p_wo = 0, p_x = 0, p_r = 0, p_ro = 0, p_un = 0, p_xv = 0;
           // OR in X_t; its new bits above src are U entries of src, those between t and src join the
           // level to come (they are reached, but their own neighbours are not covered), the rest is R_t
           auto import_prev = [&](int lev) {
@@ -3760,6 +3770,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
                 if (v >= 0) {
                   deg += dupv;
                   p_w += deg;
+                  if (kCond) ++p_xv;
                   p_r += rv;
                   if (in_prev) {
                     p_wo += deg;
@@ -3780,7 +3791,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
           {
             const uint32_t a_w = wave_sum_u32(p_w), a_wo = wave_sum_u32(p_wo), a_x = wave_sum_u32(p_x);
             const uint32_t a_r = wave_sum_u32(p_r), a_ro = wave_sum_u32(p_ro), a_un = wave_sum_u32(p_un);
+            const uint32_t a_xv = kCond ? wave_sum_u32(p_xv) : 0u;
             if (lane == 0) {
+              if (kCond && a_xv) atomicAdd(&s_xv, a_xv);
               if (a_w) atomicAdd(&s_wall, (unsigned long long)a_w);
               if (a_wo) atomicAdd(&s_wovl, (unsigned long long)a_wo);
               if (a_x) atomicAdd(&s_xe, (unsigned long long)a_x);

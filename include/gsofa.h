@@ -268,8 +268,14 @@ int gsofa_work_split(gsofa_plan* plan, uint64_t* heavy_edge_checks, uint64_t* he
 /* Work the last run actually executed, both directions: work6 = {workgroup path: neighbour
  * inspections, rows expanded, F entries written; wave path: the same three}. Chaining and the
  * two directions make these differ from W and |R|; the roofline of each kernel is priced on
- * them. No counterpart in the reference. */
+ * them. On a plan that runs by fronts (gsofa_plan_fronts) the workgroup path's rows are nodes of the
+ * condensed graph, and the second three are the fronts': entries read into the bit matrices, rows
+ * finished, F entries written. No counterpart in the reference. */
 int gsofa_executed_work(gsofa_plan* plan, uint64_t* work6);
+/* Elimination subtrees that the plan's runs finish as bit matrices in place of the wave path, and
+ * nodes of the condensed graph that the workgroup path then runs on; both 0 for a plan that runs
+ * without. Either may be null. No counterpart in the reference. */
+int gsofa_plan_fronts(gsofa_plan* plan, int64_t* units, int64_t* nodes);
 void gsofa_plan_destroy(gsofa_plan* plan);
 
 /* ---- batched form: many matrices in one captured graph of persistent launches ----------- */
