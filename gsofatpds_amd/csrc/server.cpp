@@ -7,7 +7,8 @@
 // device set for all of them, i.e. one launch sequence, as a batch. Device state comes
 // from memory that the slot keeps (bounded, and given back when the server stops), or is allocated
 // and freed stream-ordered on the slot (hipMallocAsync / hipFreeAsync: no device-wide
-// synchronisation). Groups on different slots run concurrently: their workgroups fill the CUs
+// synchronisation). What the slots keep counts against the budget like the running groups' footprints,
+// and is given back where a group needs the room. Groups on different slots run concurrently: their workgroups fill the CUs
 // others leave free, or, with cu_share set, each group's persistent grids are sized for that
 // many CUs. A completion thread polls the slots' events, reads the results of a finished group
 // on its stream and releases the slot. Latency is submit-to-result on the host clock.
@@ -99,6 +100,9 @@ struct gsofa_server {
   int cu_share = 0;
   int max_group = 16;
   int64_t budget = 0;
+  // Running groups' footprints and all slots' arenas. Only the admission thread adds to it, and only
+  // it touches the arenas; a group is charged in full beside its slot's arena, since an array that
+  // the arena has no room for leaves a part of it unused.
   std::atomic<int64_t> in_use{0};
   size_t arena_max = 0;  // bytes of a slot's arena at most
   std::vector<std::unique_ptr<Slot>> slots;
@@ -120,6 +124,25 @@ struct gsofa_server {
       if (s->group.empty()) return s.get();
     return nullptr;
   }
+  // Whether `bytes` more fit the budget once the arenas of free slots are given back.
+  bool fits(int64_t bytes) {
+    int64_t idle = 0;
+    for (auto& s : slots)
+      if (s->group.empty()) idle += (int64_t)s->arena.bytes;
+    return in_use.load() - idle + bytes <= budget;
+  }
+  // Gives back free slots' arenas, the last slots' first, until `bytes` more fit.
+  void make_room(int64_t bytes) {
+    for (auto it = slots.rbegin(); it != slots.rend() && in_use.load() + bytes > budget; ++it) {
+      Slot& s = **it;
+      if (!s.group.empty() || !s.arena.base) continue;
+      (void)hipFreeAsync(s.arena.base, s.stream);
+      (void)hipStreamSynchronize(s.stream);  // idle but for the free
+      in_use -= (int64_t)s.arena.bytes;
+      s.arena.base = nullptr;
+      s.arena.bytes = 0;
+    }
+  }
 };
 
 void gsofa_server::admit_loop() {
@@ -131,7 +154,7 @@ void gsofa_server::admit_loop() {
       if (pending.empty()) return false;
       Request* r = pending.front();
       if (r->cancel_requested) return true;
-      return free_slot() != nullptr && in_use.load() + r->footprint <= budget;
+      return free_slot() != nullptr && fits(r->footprint);
     });
     if (stopping) return;
     Request* r = pending.front();
@@ -162,7 +185,7 @@ void gsofa_server::admit_loop() {
       if (!same_options(q->opt, r->opt)) break;
       gmats.push_back(&q->prep);
       int64_t fq = 0;
-      if (DeviceSet::footprint(gmats, r->opt, &fq) != GSOFA_OK || in_use.load() + fq > budget) {
+      if (DeviceSet::footprint(gmats, r->opt, &fq) != GSOFA_OK || !fits(fq)) {
         gmats.pop_back();
         break;
       }
@@ -170,6 +193,7 @@ void gsofa_server::admit_loop() {
       fp = fq;
       pending.pop_front();
     }
+    make_room(fp);
     Slot& s = *free_slot();
     s.group = grp;
     s.footprint = fp;
@@ -192,14 +216,16 @@ void gsofa_server::admit_loop() {
     int rc = GSOFA_OK;
     s.set.reset(new (std::nothrow) DeviceSet);
     if (!s.set) rc = fail(GSOFA_ERR_OUT_OF_MEMORY, "device set");
-    // the arena grows to what the slot's last group asked for (its memory is idle: the slot was free)
+    // the arena grows to what the slot's last group asked for (its memory is idle: the slot was free),
+    // within the budget
     const size_t want = std::min(arena_max, s.arena.asked + s.arena.asked / 8);
-    if (want > s.arena.bytes) {
+    if (want > s.arena.bytes && in_use.load() + (int64_t)(want - s.arena.bytes) <= budget) {
       if (s.arena.base) (void)hipFreeAsync(s.arena.base, s.stream);
       void* q = nullptr;
       const bool ok = hipMallocAsync(&q, want, s.stream) == hipSuccess;
       if (!ok) (void)hipGetLastError();
-      s.arena.base = static_cast<char*>(q);
+      in_use += (int64_t)(ok ? want : 0) - (int64_t)s.arena.bytes;
+      s.arena.base = ok ? static_cast<char*>(q) : nullptr;
       s.arena.bytes = ok ? want : 0;
     }
     s.arena.used = s.arena.asked = 0;

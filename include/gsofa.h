@@ -305,7 +305,8 @@ typedef struct gsofa_server gsofa_server;
 typedef struct gsofa_server_options {
   int32_t device;
   int32_t slots;            /* concurrent requests on the device, default 4                      */
-  int64_t hbm_budget_bytes; /* admission budget; 0 = 80% of the free device memory at start      */
+  int64_t hbm_budget_bytes; /* device memory that the server may hold; 0 = 80% of the free
+                               device memory at start                                          */
   int32_t cu_share;         /* CUs each group's persistent grids are sized for; 0 = all          */
   int32_t max_group;        /* requests a free slot takes from the queue at once (same options,
                                FIFO order) and runs as one batch; default 16, 1 = one at a time */
@@ -337,6 +338,8 @@ int gsofa_server_request_info(gsofa_server* srv, int64_t request_id, double* lat
                               uint64_t* nzu_digest, uint64_t* supernode_digest);
 /* The FNV-1a digest (64-bit) gsofa_server_request_info reports, of any byte range. */
 int gsofa_digest_fnv1a(const void* data, int64_t bytes, uint64_t* out);
+/* hbm_in_use: the footprints of the running groups and the memory that the slots keep from group to
+ * group (at most an eighth of the budget; given back where a group needs the room). */
 int gsofa_server_stats(gsofa_server* srv, int64_t* completed, int32_t* running, int32_t* peak_running,
                        int64_t* pending, int64_t* hbm_in_use, int64_t* hbm_budget);
 /* Drops pending requests, waits for running ones, releases everything. */
