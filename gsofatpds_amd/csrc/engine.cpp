@@ -1080,19 +1080,24 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
 
 int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Options& opt, int64_t* out_bytes) {
   // mirrors the allocations of create() (spill sized for the resident heavy grid)
+  if (opt.structure || opt.split_blocks != -1 || opt.early_top > 0 || opt.pre_escalate != -1)
+    return fail(GSOFA_ERR_INVALID_ARG, "footprint: counts without cuts, early launch and elimination tree only");
   DeviceInfo info;
   int rc = device_info(opt.device, info);
   if (rc != GSOFA_OK) return rc;
-  int64_t nrows = 0, nnz = 0, nblk = 0;
+  int64_t nrows = 0, nnz = 0, nblk = 0, ck = 0;
   int32_t nmax = 0;
   bool dup = false, paired = false;
   for (const Prepared* P : mats) {
     nrows += P->n;
     nnz += (int64_t)P->adj.size();
     nmax = std::max(nmax, P->n);
-    nblk += ((int64_t)P->n + 3) / 4;  // smallest automatic chain block
+    const int64_t chain = opt.chain_block > 0 ? opt.chain_block : 4;  // the smallest automatic one
+    nblk += ((int64_t)P->n + chain - 1) / chain;
     dup |= !P->dup_u.empty();
-    paired |= pair_directions(*P, opt.pair_directions);
+    if (!pair_directions(*P, opt.pair_directions)) continue;
+    paired = true;
+    if (P->n >= kCheckpointRows) ck += 4 * checkpoint_words(P->n) + 64 * (int64_t)kCheckpoints;
   }
   const int cus = opt.cu_share > 0 ? std::min(opt.cu_share, info.cus) : info.cus;
   const int64_t heavy_grid = (int64_t)cus * 4;  // upper bound on resident workgroups per CU
@@ -1102,19 +1107,13 @@ int64_t DeviceSet::footprint(const std::vector<const Prepared*>& mats, const Opt
   b += 4 * nrows * kEll * 2;          // ELL A, A^T
   b += 4 * nrows * 3 + 16 * nrows;    // column counts, U/L counts, window bits
   b += nrows + 2 * nrows + 4 * 2 * nblk + 8 * 2 * nrows;  // flags, escalations, block flags, items
-  b += 4 * nblk + 8 * 2 * nblk;                           // block cuts and their extra items
   b += 4 * (int64_t)nmax + 8 * ((int64_t)mats.size() + 1);  // block index histogram, chain block bases
-  b += 4 * (heavy_grid + kTopMaxItems) * heavy_region_ints(nmax, paired);  // spill (and the early launch's)
+  b += 4 * heavy_grid * heavy_region_ints(nmax, paired);     // spill
   if (place_bitmaps_in_hbm(nmax, opt, info)) b += 4 * (int64_t)cus * (((int64_t)nmax + 31) / 32);  // one per CU
   if (dup) b += 8 * nrows;
-  b += (int64_t)kCheckpoints * (nrows / 4 + 8 * (int64_t)mats.size() + 64 * (int64_t)mats.size());  // checkpoints
-  // subtree sizes; fronts (states, nodes, units of at least kFrontMean rows on average with their lists)
-  // and the condensed graphs (at most kCondMaxShare + 0.1 of the rows)
-  if (opt.pre_escalate != -1)
-    b += 12 * nrows + (nrows / kFrontMean + 1) * (int64_t)(sizeof(FrontUnit) + 24 + 8 * kFrontMsg + 8 * (kFrontMax[0].nodes + kFrontMax[0].ext) * 2) +
-         8 * nnz + (int64_t)(0.7 * 150.0 * (double)nrows) + 4 * heavy_grid * heavy_region_ints(nmax, false);
-  if (opt.structure) b += 16 * (nrows + (int64_t)mats.size());  // offsets; pools are sized later
-  b += (1 << 20) + (int64_t)mats.size() * kAccSlots * 8 * acc_copies((int)mats.size());  // tables, accumulators, scan scratch
+  b += ck;  // checkpoints
+  // tables, scan scratch, accumulators
+  b += std::max<int64_t>(1 << 20, (1 << 19) + (int64_t)mats.size() * kAccSlots * 8 * acc_copies((int)mats.size()));
   *out_bytes = b;
   return GSOFA_OK;
 }

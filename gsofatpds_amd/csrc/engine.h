@@ -231,7 +231,8 @@ class DeviceSet {
   // from `arena` first, whose owner runs its sets one after another on that stream.
   int create(const std::vector<const Prepared*>& mats, const Options& opt, hipStream_t alloc_stream = nullptr,
              DeviceArena* arena = nullptr);
-  // Device bytes create() will allocate for these matrices (admission by footprint).
+  // Device bytes create() will allocate for these matrices at most (admission by footprint), for sets as the
+  // server makes them: counts only, without block cuts, the early launch and the elimination tree.
   static int64_t footprint(const std::vector<const Prepared*>& mats, const Options& opt, int64_t* out_bytes);
   // Enqueue the whole symbolic factorisation on `s` (no host synchronisation, no allocation,
   // no memset nodes: safe to capture in a graph).

@@ -61,3 +61,33 @@ def test_memory_kept_between_groups_is_within_the_budget():
             assert max(seen) <= budget
         finally:
             srv.stop()
+
+
+def estimate(p, paired, cus):
+    """What admission charged a request before unstructured matrices had checkpoints."""
+    n, blocks, bw = p.n, (p.n + 3) // 4, (p.n + 31) // 32
+    region = 4 * n + 6 * bw if paired else 3 * n + bw
+    return (12 * (n + 1) + 8 * p.nnz + 128 * n + 28 * n + 3 * n + 8 * blocks + 16 * n + 20 * blocks + 4 * n + 16 +
+            4 * (4 * cus + 32) * region + (1 << 20))
+
+
+def unstructured(n, seed=1):
+    return g.generate(kind=g.GEN_ERDOS_RENYI, n_keep=n, order=g.ORDER_RCM, drop_side=g.DROP_ANY, drop_ppm=100000,
+                      avg_degree_x100=600, seed=seed)
+
+
+@pytest.mark.parametrize("n", [1, 60, 511, 512, 5003, 40000])
+@pytest.mark.parametrize("pair", [0, 1])
+def test_a_request_needs_no_larger_budget_than_it_did(n, pair):
+    p = unstructured(n) if n > 1 else g.Pattern.from_dense(np.ones((1, 1), bool))
+    need = footprint(p, pair_directions=pair)
+    assert need <= estimate(p, pair == 1, g.device_query()["cus"])
+    srv = g.Server(slots=1, hbm_budget_bytes=need)
+    try:
+        got = srv.wait(srv.submit(p, pair_directions=pair), 60.0)
+    finally:
+        srv.stop()
+    with g.Plan(p, pair_directions=pair) as plan:
+        plan.run()
+        want = plan.result()
+    assert (got.fill_count, got.nnz_F, got.edge_checks) == (want.fill_count, want.nnz_F, want.edge_checks)
