@@ -559,7 +559,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
   item_base_h_.assign(nmats_ + 1, 0);
   blk_base_h_.assign(nmats_ + 1, 0);
   n_max_ = 0;
-  bool any_dup = false;
+  bool any_dup = false, pairs = false;
   mirror_.assign((size_t)nmats_, 0);
   for (int b = 0; b < nmats_; ++b) {
     const Prepared& P = *mats[b];
@@ -570,7 +570,9 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     blk_base_h_[b + 1] = blk_base_h_[b] + ((int64_t)P.n + 255) / 256;
     any_dup |= !P.dup_u.empty();
     mirror_[b] = mirrored(P, opt) ? 1 : 0;
-    paired_any_ |= pair_directions(P, opt.pair_directions) ? 1 : 0;
+    if (!pair_directions(P, opt.pair_directions)) continue;
+    paired_any_ = 1;
+    pairs |= !mirror_[b];
   }
   mirror_any_ = 0;
   mirror_all_ = 1;
@@ -585,7 +587,14 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
 
   // ---- launch configuration ----
   LaunchConfig cfg;
-  GSOFA_TRY(configure_launch(n_max_, nrows_, paired_any_ != 0, opt, info, 0, cfg));
+  int rc = configure_launch(n_max_, nrows_, paired_any_ != 0, opt, info, 0, cfg);
+  if (rc == GSOFA_ERR_CAPACITY && paired_any_ && !pairs) {
+    // unstructured and mirrored: no items run both directions, only the checkpoints want that kernel.
+    // A queue that leaves no room for its window's second direction runs without checkpoints.
+    paired_any_ = 0;
+    rc = configure_launch(n_max_, nrows_, false, opt, info, 0, cfg);
+  }
+  GSOFA_TRY(rc);
   cfg_ = cfg;
   bw_max_ = cfg.bw_max;
   hbm_bitmap_ = cfg.hbm_bitmap;
@@ -853,7 +862,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
 
 // Checkpoints of the unstructured matrices. Not with the early launch, whose items are fixed.
 int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats) {
-  if (n_top_ > 0) return GSOFA_OK;
+  if (n_top_ > 0 || !paired_any_) return GSOFA_OK;
   auto none = [&](int b) {
     return ns_[b] < kCheckpointRows || (!cond_.empty() && cond_[b]) || !pair_directions(*mats[b], opt_.pair_directions);
   };
