@@ -828,18 +828,17 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     M.pre_size = pre_size[b];
     M.rows = ns_[b];
   }
-  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
   // The pattern is fixed for the set's lifetime, and so are its device forms (ELL rows, A^T): built
   // here once, like the upload, not on every run.
   GSOFA_TRY(enqueue_preparation(sequence(), alloc_stream_));
   // by fronts: the matrices with subtree sizes, except where the early launch's fixed items or HBM
   // bitmaps were asked for
+  bool uploaded = false;  // the table as it is now
   if (any_pre && opt.early_top <= 0 && opt.bitmap_in_hbm != 1) {
     std::vector<uint8_t> tree((size_t)nmats_, 0);
     for (int b = 0; b < nmats_; ++b) tree[b] = pre_size[b] != INT32_MAX;
-    GSOFA_TRY(create_fronts(mats, tree, info));
+    GSOFA_TRY(create_fronts(mats, tree, info, uploaded));
   }
-  GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(preparation)");
   nplain_ = nmats_ - ncond_;
   if (nplain_ > 0) {
     // per resident workgroup: two frontier spill queues, the U list (beyond its LDS part) and the
@@ -849,7 +848,7 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     GSOFA_TRY(alloc(spill_, (size_t)(heavy_grid_ + top_grid_) * (size_t)heavy_region_ints(n_max_, paired_any_ != 0),
                     "heavy spill regions"));
     if (hbm_bitmap_) GSOFA_TRY(alloc(hbm_bm_, (size_t)heavy_grid_ * (size_t)bw_max_, "heavy bitmaps"));
-    GSOFA_TRY(create_checkpoints(mats));
+    GSOFA_TRY(create_checkpoints(mats, uploaded));
   } else {
     heavy_threads_ = ccfg_.heavy_threads;
     heavy_grid_ = ccfg_.heavy_grid;
@@ -857,11 +856,13 @@ int DeviceSet::create(const std::vector<const Prepared*>& mats, const Options& o
     qcap_ = ccfg_.qcap;
     opt_.chain_block = ccfg_.chain_block;
   }
+  if (!uploaded) GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(preparation)");
   return GSOFA_OK;
 }
 
 // Checkpoints of the unstructured matrices. Not with the early launch, whose items are fixed.
-int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats) {
+int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats, bool& uploaded) {
   if (n_top_ > 0 || !paired_any_) return GSOFA_OK;
   auto none = [&](int b) {
     return ns_[b] < kCheckpointRows || (!cond_.empty() && cond_[b]) || !pair_directions(*mats[b], opt_.pair_directions);
@@ -886,8 +887,7 @@ int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats) {
     at += checkpoint_words(ns_[b]);
   }
   ck_total_ = 2 * kCheckpoints * nmats_;
-  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
-  if (alloc_stream_) GSOFA_HIP(hipStreamSynchronize(alloc_stream_), "hipStreamSynchronize(checkpoints)");
+  uploaded = false;
   return GSOFA_OK;
 }
 
@@ -895,7 +895,7 @@ int DeviceSet::create_checkpoints(const std::vector<const Prepared*>& mats) {
 // fronts (nothing else of it is kept; every run builds its graphs anew, and reports an error should
 // it count other sizes).
 int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree,
-                             const DeviceInfo& info) {
+                             const DeviceInfo& info, bool& uploaded) {
   hipStream_t s = alloc_stream_;
   cond_.assign((size_t)nmats_, 0);
   std::vector<FrontUnit> units[kFrontLevels];
@@ -955,6 +955,7 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
     M.uctr = reinterpret_cast<uint32_t*>(cond_zero_ + nrows_);
   }
   GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
+  uploaded = true;
   // per matrix its nodes and its unfinished rows, then per level the largest units (FrontSize)
   unsigned long long* sizes_d = nullptr;
   GSOFA_TRY(alloc(sizes_d, (size_t)(2 * nmats_ + 2 * kFrontLevels), "condensed sizes"));
@@ -972,6 +973,7 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
   auto drop = [&](int b) {
     cond_[b] = 0;
     mats_h_[b].st = nullptr;
+    uploaded = false;
   };
   for (int b = 0; b < nmats_; ++b)
     if (cond_[b] && (double)sizes[b] > (kCondMaxShare + 0.1) * ns_[b]) drop(b);
@@ -1024,7 +1026,8 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
       item_base_h_[b + 1] = item_base_h_[b] + (mirror_[b] ? nb + (nb & 1) : 2 * nb);
     }
     nitems_ = item_base_h_[nmats_];
-    GSOFA_TRY(upload(item_base_d_, item_base_h_.data(), item_base_h_.size() * 8, "upload"));
+    if (ncond_ > 0 && ncond_ < nmats_)  // (without plain matrices nothing reads them)
+      GSOFA_TRY(upload(item_base_d_, item_base_h_.data(), item_base_h_.size() * 8, "upload"));
     if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(front units)");
   }
   if (ncond_ > 0) {
@@ -1053,14 +1056,17 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
     }
     GSOFA_HIP(launch_fill_i32(orig, cnodes_, 0, s), "clear condensed nodes");
     GSOFA_TRY(alloc(cmats_d_, (size_t)nmats_, "condensed table"));
-    GSOFA_TRY(alloc(cbase_d_, cbase.size(), "condensed node base"));
-    GSOFA_TRY(alloc(cblk_base_d_, cblk_base.size(), "condensed block base"));
-    GSOFA_TRY(alloc(cblk_mat_d_, order.size(), "condensed order"));
+    GSOFA_TRY(alloc(cbase_d_, cbase.size() + cblk_base.size() + (order.size() + 1) / 2, "condensed node and block bases, order"));
+    cblk_base_d_ = cbase_d_ + cbase.size();
+    cblk_mat_d_ = reinterpret_cast<int32_t*>(cblk_base_d_ + cblk_base.size());
     GSOFA_TRY(alloc(citems_, (size_t)(4 * cnblk_), "condensed items"));
     GSOFA_TRY(alloc(cspill_, (size_t)ccfg_.heavy_grid * (size_t)heavy_region_ints(cn_max_, false), "condensed spill regions"));
-    GSOFA_TRY(upload(cbase_d_, cbase.data(), cbase.size() * 8, "upload"));
-    GSOFA_TRY(upload(cblk_base_d_, cblk_base.data(), cblk_base.size() * 8, "upload"));
-    GSOFA_TRY(upload(cblk_mat_d_, order.data(), order.size() * 4, "upload"));
+    std::vector<int64_t> bases(cbase);
+    bases.insert(bases.end(), cblk_base.begin(), cblk_base.end());
+    const size_t at = bases.size();
+    bases.resize(at + (order.size() + 1) / 2);
+    std::memcpy(bases.data() + at, order.data(), order.size() * 4);
+    GSOFA_TRY(upload(cbase_d_, bases.data(), bases.size() * 8, "upload bases"));
     cmats_h_ = mats_h_;
     for (int b = 0; b < nmats_; ++b) {
       MatDev& C = cmats_h_[b];
@@ -1082,8 +1088,6 @@ int DeviceSet::create_fronts(const std::vector<const Prepared*>& mats, const std
   } else {
     cond_words_ = 0;
   }
-  GSOFA_TRY(upload(mats_d_, mats_h_.data(), sizeof(MatDev) * nmats_, "upload table"));
-  if (s) GSOFA_HIP(hipStreamSynchronize(s), "hipStreamSynchronize(condensed graphs)");
   return GSOFA_OK;
 }
 

@@ -320,8 +320,10 @@ class DeviceSet {
   std::vector<std::vector<int64_t>> u_ptr_h_, l_ptr_h_;    // host copies of the offsets
   std::vector<MatDev> mats_h_;
   // fronts and condensed graphs (Sequence)
-  int create_checkpoints(const std::vector<const Prepared*>& mats);
-  int create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree, const DeviceInfo& info);
+  // (uploaded: whether the device has the matrices' table as it is)
+  int create_checkpoints(const std::vector<const Prepared*>& mats, bool& uploaded);
+  int create_fronts(const std::vector<const Prepared*>& mats, const std::vector<uint8_t>& tree, const DeviceInfo& info,
+                    bool& uploaded);
   int ncond_ = 0, nplain_ = 0;
   int cus_ = 0;
   int32_t ck_total_ = 0;
