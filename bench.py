@@ -50,8 +50,8 @@ def parse():
                     help="sources in the CPU baseline's seeded sample (each of 3 timed passes)")
     ap.add_argument("--cpu-full", action="store_true", help="CPU baseline over all sources (minutes)")
     ap.add_argument("--no-cpu", action="store_true")
-    ap.add_argument("--traffic", default=os.path.join(ROOT, "profiles", "traffic_heavy_grid2d_659033.json"),
-                    help="rocprofv3 FETCH_SIZE/WRITE_SIZE summary for the dominant kernel (optional)")
+    ap.add_argument("--traffic", default="",
+                    help="JSON with the dominant stage's kernel names and its measured bytes_per_launch (optional)")
     ap.add_argument("--batch-members", type=int, default=256,
                     help="members of the 256-matrix batch to run batched vs plain (0 = skip)")
     ap.add_argument("--batch-config", default="",
@@ -347,19 +347,34 @@ def main():
     W, R = r.edge_checks, r.reach
     gteps = W / (ms_per_step / 1e3) / 1e9
     fill_rate = r.fill_count / (ms_per_step / 1e3)
-    # Per-unit bytes of the reference's loop: 8 B per neighbour inspection (index + label,
+    # The stages between the run's events, by the kernels that run in them, priced on the work that they
+    # executed (both directions, after reuse of reached sets: the schedule-independent W would count
+    # inspections that no kernel does). Traversals: per-unit bytes of the reference's loop, 8 B per
+    # neighbour inspection (index + label,
     # gSoFa_SOAComparison/symbfact_warp_centric_new_scheduling.cuh:952, 959), 12 B per expanded row
-    # (row extent + label write, same file :923, 948), 4 B per F entry written. Priced on the work
-    # each kernel executed (both directions, after reuse of reached sets): the schedule-independent
-    # W would count inspections the kernels never do.
+    # (row extent + label write, same file :923, 948), 4 B per F entry written. Fronts: 4 B per entry read
+    # (no label), 12 B per finished row, 4 B per F entry. Supernodes: 21 B per row (window, count, flag); the
+    # structure's lists, put in order in the same stage, 8 B per entry.
     # k_heavy: the main launch (its stage); the early launch of the top separator's items runs on
     # its own stream beside the wave path and is priced apart (early_launch below).
-    kern = {"k_heavy": (xw["heavy_edges"] - et["edges"], xw["heavy_rows"] - et["rows"], xw["heavy_out"] - et["out"],
-                        stages["heavy_ms"]),
-            "k_light": (xw["light_edges"], xw["light_rows"], xw["light_out"], stages["light_ms"])}
-    dom = max(kern, key=lambda k: kern[k][3])
-    e_x, v_x, o_x, k_ms = kern[dom]
-    kbytes = 8 * e_x + 12 * v_x + 4 * o_x
+    fronts = plan.fronts()
+    lists = r.nnz_L + r.nnz_U if structure else 0  # (no workload here is symmetric)
+    light = {"edge_inspections": xw["light_edges"], "rows_expanded": xw["light_rows"], "entries_written": xw["light_out"]}
+    heavy = {"edge_inspections": xw["heavy_edges"] - et["edges"], "rows_expanded": xw["heavy_rows"] - et["rows"],
+             "entries_written": xw["heavy_out"] - et["out"]}
+    light_price, light_name = (8, 12, 4), "k_light"
+    if fronts["units"] > 0:
+        light = {"entries_read": xw["light_edges"], "rows_finished": xw["light_rows"], "entries_written": xw["light_out"]}
+        light_price, light_name = (4, 12, 4), "k_front_leaf + k_front + k_cond_*"
+    kern = {  # name: units, bytes of each, ms
+        "k_heavy": (heavy, (8, 12, 4), stages["heavy_ms"]),
+        light_name: (light, light_price, stages["light_ms"]),
+        "k_sort_short + k_sort_long + k_supernodes" if structure else "k_supernodes":
+            ({"list_entries": lists, "rows": p.n}, (8, 21), stages["supernodes_ms"])}
+    kbytes_of = {k: sum(n * b for n, b in zip(u.values(), price)) for k, (u, price, _) in kern.items()}
+    dom = max(kern, key=lambda k: kern[k][2])
+    units, _, k_ms = kern[dom]
+    kbytes = kbytes_of[dom]
     achieved = kbytes / (k_ms / 1e3) / 1e9 if k_ms > 0 else 0.0
     traffic = None
     if os.path.exists(args.traffic):
@@ -369,12 +384,10 @@ def main():
             traffic = tr.get("bytes_per_launch")
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic, "kernel": dom,
-                "kernel_ms": k_ms, "algorithmic_bytes_per_launch": kbytes,
-                "units_per_launch": {"edge_inspections": e_x, "rows_expanded": v_x, "entries_written": o_x}}
+                "kernel_ms": k_ms, "algorithmic_bytes_per_launch": kbytes, "units_per_launch": units}
     x_edges = xw["heavy_edges"] + xw["light_edges"]
     x_rows = xw["heavy_rows"] + xw["light_rows"]
-    x_out = xw["heavy_out"] + xw["light_out"]
-    step_bytes_x = 8 * x_edges + 12 * x_rows + 4 * x_out
+    step_bytes_x = sum(kbytes_of.values()) + 8 * et["edges"] + 12 * et["rows"] + 4 * et["out"]
     step_bytes_w = 8 * W + 12 * R + 4 * r.nnz_F
     out = {
         "metric": METRIC, "value": gteps, "unit": "GTEPS", "n_gpus": 1, "steps": args.steps, "warmup": args.warmup,
@@ -396,13 +409,15 @@ def main():
         "stages_ms": stages,
         "stages_note": "HIP events on the run's stream, averaged over as many runs after the timed ones "
                        "(the timed loop reads nothing but each run's totals)",
+        "stage_kernels": {"light_ms": light_name, "heavy_ms": "k_heavy", "supernodes_ms": list(kern)[2]},
+        "fronts": fronts,
         "executed_work": xw,
         "executed": {"inspections_per_step": x_edges, "rows_expanded_per_step": x_rows,
                      "gteps": x_edges / (ms_per_step / 1e3) / 1e9,
                      "fraction_of_W": x_edges / max(W, 1)},
         "step_roofline": {"achieved": step_bytes_x / (ms_per_step / 1e3) / 1e9, "peak": HBM_PEAK_GBS,
                           "unit": "GB/s", "frac": step_bytes_x / (ms_per_step / 1e3) / 1e9 / HBM_PEAK_GBS,
-                          "bytes_per_step": step_bytes_x, "what": "executed work of both kernels over the step"},
+                          "bytes_per_step": step_bytes_x, "what": "executed work of all stages over the step"},
         "schedule_independent_GBs": step_bytes_w / (ms_per_step / 1e3) / 1e9,
         "roofline": roofline,
     }
