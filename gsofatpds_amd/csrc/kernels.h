@@ -116,7 +116,9 @@ struct MatDev {
   int32_t* uwt;                   // 2 per unit: sum of degrees and number of vertices of its S
   int32_t* uid;                   // per unit: its root's node
   uint32_t* umsg;                 // kFrontMsg per unit and direction: its root's reached nodes as bits,
-                                  // and in the last word the length of its list above the root
+                                  // and in the last word the length of its list above the root. All that
+                                  // one direction's workgroup may read of the other's (agent-scope
+                                  // accesses, no fence: nothing else is visible before the next launch)
   uint32_t* uctr;                 // per unit: directions ended, 1 for each that fitted, 16 for the others
   // A condensed graph as k_heavy sees it (n nodes; ell, rowptr, adj, esc by node).
   const int32_t* orig;            // n: the node's vertex, or -(r + 1): a list node of root r
@@ -163,12 +165,12 @@ hipError_t launch_clear_run(unsigned long long* acc, int64_t nacc, unsigned long
 hipError_t launch_fill_i32(int32_t* p, int64_t count, int32_t v, hipStream_t s);
 hipError_t launch_ell_build(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* ell, hipStream_t s);
-// Builds A^T of every matrix: col_cnt/cursor/rowptr_t have nrows (+1) entries, block_sums
-// ceil(nrows / 4096), total one int.
 // The layout of one matrix of at most kSmallRows rows in one launch: ell of A, A^T and its ell.
 constexpr int kSmallRows = 4096, kSmallRowEntries = 16;  // (entries per row on average, at most)
 hipError_t launch_prepare_small(int32_t n, const int32_t* rowptr, const int32_t* adj, int32_t* ell, int32_t* rowptr_t,
                                 int32_t* adj_t, int32_t* ell_t, hipStream_t s);
+// Builds A^T of every matrix: col_cnt/cursor/rowptr_t have nrows (+1) entries, block_sums
+// ceil(nrows / 4096), total one int.
 hipError_t launch_transpose(int64_t nrows, int nmats, const int64_t* row_base, const int32_t* rowptr,
                             const int32_t* adj, int32_t* col_cnt, int32_t* rowptr_t, int32_t* cursor,
                             int32_t* adj_t, int32_t* block_sums, int32_t* total, hipStream_t s);
@@ -265,12 +267,12 @@ hipError_t launch_top_setup(const MatDev* mats, int nmats, WorkState* ws, int64_
 // After the last kernel that counts: every matrix's copies summed into copy 0 (one block per matrix);
 // a mirrored matrix's fill and workgroup-path entries doubled, nnz_L = nnz_U.
 hipError_t launch_totals(const MatDev* mats, int nmats, hipStream_t s);
-// Mirrored matrices: L counts = U counts (one thread per row, blocks as for launch_supernodes).
 // The explicit structure's lists into ascending order (after the traversals, and by the offsets: every
 // matrix has lists). region: sort_region_words words (0: none needed).
 int64_t sort_region_words(int64_t n_max, int cus);
 hipError_t launch_sort_lists(const MatDev* mats, int nmats, const int64_t* row_base, int64_t nrows, int64_t n_max, int cus,
                              uint32_t* region, hipStream_t s);
+// Mirrored matrices: L counts = U counts (one thread per row, blocks as for launch_supernodes).
 hipError_t launch_mirror(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 hipError_t launch_supernodes(const MatDev* mats, int nmats, const int64_t* blk_base, int64_t nblocks, hipStream_t s);
 constexpr int kLightThreads = 256;

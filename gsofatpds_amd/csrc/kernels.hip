@@ -2043,7 +2043,9 @@ __global__ __launch_bounds__(kFrontThreads[kLevel]) __attribute__((amdgpu_waves_
       }
       // The exchange goes through agent-scope accesses only, which no cache of an XCD keeps; they are
       // acknowledged before the counter moves. (A release fence would write back the XCD's whole L2:
-      // 177 -> 432 us for the 2,048 workgroups of a level at 659,033 rows.)
+      // 177 -> 432 us for the 2,048 workgroups of a level at 659,033 rows.) So nothing that the other
+      // workgroup stored plainly (list entries, counts, windows) may be read before the next launch: what it
+      // has to hand over goes into the message.
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __syncthreads();
       if (tid == 0) s_other = (int32_t)atomicAdd(M.uctr + u, fits ? 1u : 16u);
@@ -2527,8 +2529,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
   __shared__ unsigned long long s_escm[2];      // rows w0 .. w0 + 63 escalated, as bits (per direction)
   __shared__ HeavyCtl s_ctl;
   __shared__ LeaderState s_ls;
-  // The slots some lane of the wave sets (push loops skip the others). Sets with paired items
-  // (unstructured rows, which fill most slots) keep every slot: measured faster there.
   // What a vertex adds to the totals beyond its entries: the duplicate surplus of its input row, or a
   // condensed node's weights (dupv to its entry count, rv vertices). Nothing for v < 0.
   auto node_weight = [](const MatDev& M, int d, int32_t v, uint32_t& dupv, uint32_t& rv) {
@@ -2542,6 +2542,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
       if (v >= 0 && d == 0 && M.dup_all) dupv = (uint32_t)gload(M.dup_all + v);
     }
   };
+  // The slots some lane of the wave sets (push loops skip the others). Sets with paired items
+  // (unstructured rows, which fill most slots) keep every slot: measured faster there.
   auto row_any = [](uint32_t mask) -> uint32_t {
     if constexpr (kPairedAny) return ~0u;
     else return wave_or_u32(mask);

@@ -149,8 +149,9 @@ typedef struct gsofa_options {
                                identical under every candidate); 0 (default): built-in rules */
   int32_t bitmap_in_hbm;    /* 1: the bitmap path keeps its n-bit bitmaps in HBM (L2 atomics);
                                0 (default): only where one does not fit in LDS (n above about
-                               1.2 M rows), so any n runs. The reference's labels live in global
-                               memory at every n (SOA:470-479).                                */
+                               1.2 M rows, or as many nodes of a condensed graph), so any n runs.
+                               The reference's labels live in global memory at every n
+                               (SOA:470-479).                                                  */
   int32_t split_blocks;     /* a workgroup-path block that holds the start of a separator over
                                a large subtree (its elimination subtree at least 1.5x its
                                predecessor's and n / k rows) runs as two items, so two
@@ -174,20 +175,25 @@ typedef struct gsofa_options {
                                run as a few fixed workgroup-path items, three per direction over
                                consecutive blocks, in a launch of their own on an internal
                                stream, which starts with the wave path and joins the run before
-                               supernode detection (counting only, about 3 % faster at 659,033
-                               rows when it is dispatched before the wave path fills the device,
-                               about 10 % slower when not: nothing orders the two). 0 (default)
-                               or -1: not. Results do not depend on it                         */
+                               supernode detection. 0 (default) or -1: not. 1 also switches the
+                               fronts off (see pre_escalate), of which such an order gains far
+                               more: 659,033 rows, counting only, 0.8 ms by default and 5.0 ms
+                               with 1. For matrices that run without fronts anyway it gives or
+                               takes a few percent: nothing orders the two launches. Results do
+                               not depend on it                                                */
   int32_t pre_escalate;     /* 0 (default): in matrices without paired items whose pattern is
                                symmetric or nearly (three quarters of the sampled off-diagonal
                                entries have their transpose), a row whose elimination subtree of
                                A + A^T holds more vertices than the hash path's escalation limit
                                goes to the bitmap path without a hash-path attempt (a symmetric
                                pattern's reached set holds the whole subtree; a nearly symmetric
-                               one's nearly always does). -1:
-                               every row is attempted first. The server does not use it (the
-                               elimination tree costs as much host time as the preparation).
-                               Results do not depend on it                                     */
+                               one's nearly always does), and where the order makes subtrees row
+                               ranges (nested dissection) these are finished as bit matrices and
+                               the rest runs on a condensed graph (gsofa_plan_fronts). -1:
+                               every row is attempted first, without fronts. early_top = 1 and
+                               bitmap_in_hbm = 1 switch the fronts off too. The server does not
+                               use it (the elimination tree costs as much host time as the
+                               preparation). Results do not depend on it                       */
 } gsofa_options;
 
 typedef struct gsofa_result {
@@ -249,9 +255,11 @@ int gsofa_supernodal_from_structure(int32_t n, const uint8_t* flags, const int64
                                     int32_t* usub);
 /* Device time of the last run's stages, from events on the run's stream: ms[0] the run's clears
  * (the pattern's device forms, ELL rows and the transpose, are built once when the plan or batch
- * is created), ms[1] the wave (hash) path and the workgroup-path queue, ms[2] the workgroup
- * (bitmap) path's main launch, ms[3] the wait for the early launch (if it is still running),
- * supernode detection. No counterpart in the reference (its only timers are wtime()). */
+ * is created), ms[1] the wave (hash) path and the workgroup-path queue, or the fronts and the
+ * condensed graph (gsofa_plan_fronts), ms[2] the workgroup (bitmap) path's main launch (and its
+ * checkpoints), ms[3] the wait for the early launch (if it is still running), supernode
+ * detection, the order of the structure's lists, the totals. No counterpart in the reference (its
+ * only timers are wtime()). */
 int gsofa_stage_times(gsofa_plan* plan, double* ms);
 /* Whether gsofa_run records the stage events above (on = 1, the default) or not (0: each event
  * between kernels costs a few microseconds of device time; gsofa_stage_times then reports
